@@ -315,8 +315,9 @@ mcnla_status mcnla_solver_iteration(mcnla_solver s, int64_t* iteration);
 /* Per-stage device times of the last solve (seconds): [sketch, orthogonalize, integrate, form]
  * plus, in sketch_kernel_s, the duration of the sketch GEMM launch alone. */
 mcnla_status mcnla_solver_stage_times(mcnla_solver s, double times[4], double* sketch_kernel_s);
-/* Durations (seconds, HIP events on the solve's stream) of single kernel launches of the last
- * solve: times[0] = sketch GEMM, times[1] = Gram GEMM G = Y'Y (without its split-K reduction).
+/* Durations (seconds, HIP events on the solve's stream) of single products of the last solve:
+ * times[0] = sketch GEMM, times[1] = Gram GEMM G = Y'Y (on the FP64 tiles without its split-K
+ * reduction; by residues with its scaling, packing and reconstruction).
  * No reference counterpart (the reference times whole stages only, stage_wrapper.hpp:120-140);
  * this is for roofline accounting. */
 mcnla_status mcnla_solver_kernel_times(mcnla_solver s, double times[2]);
@@ -354,6 +355,10 @@ mcnla_status mcnla_solve_static(const mcnla_params* params, const mcnla_solver_c
  * measured best at the 100000 x 10000 (Nl = 2048) and 500000 x 2000 (Nl = 8192) shapes.  A split
  * count or tile shape changes only the order of the sums, so a tuned plan gives the same results
  * to rounding, and the same plan always gives the same bits.
+ *
+ * Large FP64 sketches and Gram matrices run by residues on the INT8 cores instead (the `gram`
+ * target then only sizes their workspace; kernels bit 1 keeps the Gram on the FP64 tiles); their
+ * results do not depend on the plan.
  *
  * Tuned plans are kept in a process-wide table keyed by (route, precision, m, n, l, N); a solver
  * created after an entry exists for its key uses it (servers too, per request shape). */

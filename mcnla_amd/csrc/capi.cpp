@@ -235,6 +235,18 @@ GemmShape tall_shape(int64_t ncols) {
 // ------------------------------------------------------------------------------------------------
 // Shared pipeline pieces.
 
+// Workspace lent to an FP64 product that may run by residues (gemm_residue.hip).  Whether it does
+// is decided on `limit` bytes, the part every solver of the shape has, so that it does not depend
+// on where the solver lives; `bytes` (>= limit) is what is there.  flag: the product's device
+// flag, outside ws.  A null flag: no workspace.
+struct ResidueScratch {
+  void* ws = nullptr;
+  size_t bytes = 0, limit = 0;
+  int* flag = nullptr;
+};
+// The most workspace taken for the sake of speed alone: the larger plans measured 2 % faster.
+constexpr size_t kResidueBytes = size_t{2} << 30;
+
 // Y = A * Omega with Omega generated into `omega` (n x Nl FP64).
 struct SketchCore {
   DevBuf omega, ws;
@@ -256,6 +268,22 @@ struct SketchCore {
     s.fmt = sketch_fmt(precision);
     return s;
   }
+  static ResidueArgs residue_args(const mcnla_params& p, const void* A, int64_t lda, int dtype,
+                                  int order, const double* om, void* Y) {
+    ResidueArgs r;
+    r.M = p.nrow;
+    r.N = (p.rank + p.over_rank) * p.num_sketch;
+    r.K = p.ncol;
+    r.A = A;
+    r.lda = lda;
+    r.a_mcontig = (order == MCNLA_COL_MAJOR);
+    r.a_f32 = (dtype == MCNLA_F32);
+    r.B = om;
+    r.ldb = r.N;
+    r.C = static_cast<double*>(Y);
+    r.ldc = r.N;
+    return r;
+  }
   // Allocates Omega and, for a mixed precision, the BF16 panels of A and Omega.
   void prepare(const mcnla_params& p, int precision) {
     omega.ensure(p.ncol * (p.rank + p.over_rank) * p.num_sketch * sizeof(double));
@@ -276,9 +304,10 @@ struct SketchCore {
     }
   }
   // y_f64: a mixed-precision sketch writes its FP32-accumulated Y as FP64 (the fused solver's
-  // Gram and basis products then read FP64); otherwise mixed Y is FP32.
+  // Gram and basis products then read FP64); otherwise mixed Y is FP32.  scratch: where an FP64
+  // sketch may run by residues.
   void project(const mcnla_params& p, int precision, const void* A, int64_t lda, int dtype,
-               int order, void* Y, hipStream_t st, bool y_f64 = false) {
+               int order, void* Y, hipStream_t st, bool y_f64, const ResidueScratch& scratch) {
     const int64_t nl = (p.rank + p.over_rank) * p.num_sketch;
     if (!gemm_beg) {
       MCNLA_HIP(hipEventCreate(&gemm_beg));
@@ -299,6 +328,18 @@ struct SketchCore {
       g.C = static_cast<double*>(Y);
       g.ldc = nl;
       g.shape = GemmShape::kSquare;
+      const ResidueArgs ra = residue_args(p, A, lda, dtype, order, omega.as<double>(), Y);
+      const bool by_residues = scratch.flag != nullptr && residue_pays(ra, scratch.limit);
+      if (by_residues) {
+        MCNLA_HIP(hipEventRecord(gemm_beg, st));
+        gemm_residue(ra, scratch.ws, scratch.bytes, scratch.flag, st);
+        g.gate = scratch.flag;  // rows without a scale: the FP64 product after all
+        g.gate_t = 1;
+        gemm_f64(g, st);
+        MCNLA_HIP(hipEventRecord(gemm_end, st));
+        recorded = true;
+        return;
+      }
       // A column-major FP64 A takes the DMA-tiled GEMM, one workgroup per CU: the rows of whole
       // rounds of the grid go as one product, the rest split K (their last round would otherwise
       // run a few full-length workgroups on a mostly idle device: 6256 tiles at 100000 x 10000,
@@ -407,23 +448,71 @@ struct GramCore {
     g.splits = ceil_div(m, g.kchunk);
     return g;
   }
-  void prepare(bool y_f32, int64_t m, int64_t nl) {
-    const GemmF64Args g = plan(y_f32, m, nl);
-    partial.ensure(gemm_f64_partial_elems(nl, nl, g.splits) * sizeof(double));
+  static ResidueArgs residue_args(const void* Y, bool y_f32, int64_t m, int64_t nl, double* G) {
+    ResidueArgs r;
+    r.M = nl;
+    r.N = nl;
+    r.K = m;
+    r.A = Y;
+    r.lda = nl;
+    r.a_f32 = y_f32;
+    r.sym = true;
+    r.C = G;
+    r.ldc = nl;
+    return r;
   }
-  void run(const void* Y, bool y_f32, int64_t m, int64_t nl, double* G, hipStream_t st) {
+  // Bytes of the FP64 product's split-K partials.
+  size_t partial_bytes(bool y_f32, int64_t m, int64_t nl) const {
+    return gemm_f64_partial_elems(nl, nl, plan(y_f32, m, nl).splits) * sizeof(double);
+  }
+  // Allocates the partials; with more memory than a reserved region holds, at least `more` bytes.
+  void prepare(int64_t m, int64_t nl, size_t more) {
+    const size_t need = partial_bytes(false, m, nl);
+    if (more > need && more > partial.bytes) {
+      try {
+        partial.ensure(more);
+      } catch (const Error& e) {
+        if (e.code != MCNLA_ERR_NOMEM) throw;
+      }
+    }
+    partial.ensure(need);
+  }
+  bool by_residues(int64_t m, int64_t nl) const {
+    return kern == 0 && residue_pays(residue_args(nullptr, false, m, nl, nullptr),
+                                     partial_bytes(false, m, nl));
+  }
+  // Y has leading dimension ld.  A product by residues works in `ws` if that is the larger buffer,
+  // or in that of the partials (flag: its device flag).
+  void run(const void* Y, int64_t ld, bool y_f32, int64_t m, int64_t nl, double* G, int* flag,
+           hipStream_t st, const DevBuf* ws = nullptr) {
     if (!beg) {
       MCNLA_HIP(hipEventCreate(&beg));
       MCNLA_HIP(hipEventCreate(&end));
     }
-    GemmF64Args g = plan(y_f32, m, nl);
-    g.ev_begin = beg;
-    g.ev_end = end;
+    const bool residues = by_residues(m, nl);
+    GemmF64Args g = plan(y_f32 && !residues, m, nl);
+    partial.ensure(gemm_f64_partial_elems(nl, nl, g.splits) * sizeof(double));
+    g.a_f32 = y_f32;
+    g.b_f32 = y_f32;
+    g.lda = ld;
+    g.ldb = ld;
     g.A = Y;
     g.B = Y;
     g.C = G;
-    prepare(y_f32, m, nl);
     g.partial = partial.as<double>();
+    if (residues) {
+      if (ws == nullptr || ws->bytes < partial.bytes) ws = &partial;
+      ResidueArgs r = residue_args(Y, y_f32, m, nl, G);
+      r.lda = ld;
+      MCNLA_HIP(hipEventRecord(beg, st));
+      gemm_residue(r, ws->p, ws->bytes, flag, st);
+      MCNLA_HIP(hipEventRecord(end, st));
+      g.gate = flag;  // columns without a scale: the FP64 product after all
+      g.gate_t = 1;
+    } else {
+      g.ev_begin = beg;
+      g.ev_end = end;
+    }
     gemm_f64(g, st);
     recorded = true;
   }
@@ -612,9 +701,31 @@ struct Sketcher : mcnla_stage_s {
   int threads = 1;
   int64_t exponent = 0;
   SketchCore core;
+  DevBuf residue;                  // flag and workspace of the FP64 sketch by residues
   DevBuf idx, partial;             // column-sampling indices; split-K partials of A'Y
   std::vector<int64_t> host_idx;
   Sketcher() : mcnla_stage_s(kSketcher) {}
+  // The workspace of an FP64 sketch of this A by residues, taken on the first run; none when the
+  // FP64 kernels are faster or the memory is not there.
+  ResidueScratch scratch(const void* A, int64_t lda, int dtype, int order, void* Y) {
+    if (precision != MCNLA_PREC_F64) return {};
+    const ResidueArgs r =
+        SketchCore::residue_args(prm, A, lda, dtype, order, core.omega.as<double>(), Y);
+    if (!residue_pays(r, kResidueBytes)) return {};
+    const size_t need = residue_bytes(r, kResidueBytes);
+    try {
+      residue.ensure(kCarveAlign + need);
+    } catch (const Error& e) {
+      if (e.code != MCNLA_ERR_NOMEM) throw;
+      return {};
+    }
+    ResidueScratch s;
+    s.flag = residue.as<int>();
+    s.ws = residue.as<char>() + kCarveAlign;
+    s.bytes = residue.bytes - kCarveAlign;
+    s.limit = kResidueBytes;
+    return s;
+  }
   bool sampling() const {
     return kind == MCNLA_SKETCHER_COLUMN_SAMPLING || kind == MCNLA_SKETCHER_ROW_BLOCK_COLUMN_SAMPLING;
   }
@@ -635,7 +746,7 @@ struct Integrator : mcnla_stage_s {
   int64_t maxiter = 256;
   double tol = 1e-4;
   int64_t iteration = 0;
-  DevBuf Bs, ws, coef;
+  DevBuf Bs, ws, coef, flag;
   GramCore gram;
   Integrator() : mcnla_stage_s(kIntegrator) {}
 };
@@ -774,8 +885,9 @@ mcnla_status integrate(Integrator& it, const void* Qs, double* Qbar, hipStream_t
   const bool f32 = is_mixed(it.precision);
   it.Bs.ensure(nl * nl * sizeof(double));
   it.coef.ensure(nl * l * sizeof(double));
+  it.flag.ensure(sizeof(int));
   it.timer.start(st);
-  it.gram.run(Qs, f32, m, nl, it.Bs.as<double>(), st);
+  it.gram.run(Qs, nl, f32, m, nl, it.Bs.as<double>(), it.flag.as<int>(), st);
   it.timer.mark(st);
   bool conv = false, ok = true;
   it.iteration = run_integration(it.kind, it.Bs.as<double>(), N, l, it.maxiter, it.tol,
@@ -819,7 +931,11 @@ struct mcnla_solver_s {
   mcnla::SketchCore sketch;
   mcnla::GramCore gram;
   mcnla::FormCore form;
-  mcnla::DevBuf Y, G, W, w, V, T, Bs, tmp, ws, coef, M2, Qbar, bad;
+  mcnla::DevBuf Y, G, W, w, V, T, Bs, tmp, ws, coef, M2, Qbar;
+  // device flags: a Gram block that is not positive definite, and those of the products by
+  // residues (sketch, Gram)
+  static constexpr int kSketchFlag = 1, kGramFlag = 2, kFlags = 3;
+  mcnla::DevBuf bad;
   mcnla::DevBuf L0, T0, W0;  // first block's Cholesky factor, eigen transform, and rotation
   // mcnla_solver_solve_host: the device copy of a host A, the copy stream and one event per chunk
   mcnla::DevBuf Acopy;
@@ -955,7 +1071,20 @@ void apply_tuning(mcnla_solver_s* s, const mcnla_tuning& t) {
                            gemm_f64_partial_elems(n, l, n_by_l_splits(n, nl, t.n_by_l)),
                            gemm_f64_partial_elems(n, l, n_by_l_splits(n, n, t.n_by_l))}) *
                  sizeof(double));
-  s->gram.prepare(false, m, via_a ? n : nl);
+  // the products by residues (Gram, and an FP64 sketch before it) work in the partials' buffer:
+  // give them the workspace of their best plans where memory is not reserved by the byte
+  size_t more = 0;
+  const int64_t gn = via_a ? n : nl;
+  if (current_carve() == nullptr && !s->gram.partial.borrowed) {
+    if (s->gram.by_residues(m, gn))
+      more = residue_bytes(GramCore::residue_args(nullptr, false, m, gn, nullptr), kResidueBytes);
+    const ResidueArgs r = SketchCore::residue_args(s->prm, nullptr, m, MCNLA_F64, MCNLA_COL_MAJOR,
+                                                   nullptr, nullptr);
+    if (!via_a && s->cfg.precision == MCNLA_PREC_F64 &&
+        residue_pays(r, s->gram.partial_bytes(false, m, nl)))
+      more = std::max(more, residue_bytes(r, kResidueBytes));
+  }
+  s->gram.prepare(m, gn, more);
   if (!via_a)  // the Qbar product's split-K partials reuse the Gram's (free by then)
     s->gram.partial.ensure(gemm_f64_partial_elems(m, l, qbar_splits(m, nl, t.qbar)) *
                            sizeof(double));
@@ -1011,7 +1140,7 @@ std::unique_ptr<mcnla_solver_s> new_solver(const mcnla_params* params,
   s->coef.ensure(nl * l * sizeof(double));
   s->M2.ensure(nl * l * sizeof(double));
   s->Qbar.ensure(m * l * sizeof(double));
-  s->bad.ensure(sizeof(int));
+  s->bad.ensure(mcnla_solver_s::kFlags * sizeof(int));
   s->L0.ensure(l * l * sizeof(double));
   s->T0.ensure(l * l * sizeof(double));
   s->W0.ensure(l * l * sizeof(double));
@@ -1087,21 +1216,36 @@ void solve_sketch(mcnla_solver_s* s, const void* A, int64_t lda, int a_dtype, in
   cx.ldar = p.ncol;
   cx.rotate = !is_combining(c.integrator);
   const bool via_a = s->route == MCNLA_ROUTE_GRAM_OF_A;
-  const int64_t n = p.ncol;
+  const int64_t n = p.ncol, nl = (p.rank + p.over_rank) * p.num_sketch;
   // 1. sketch: Y = A * Omega; on the Gram-of-A route, H = A'A (A as row-major FP64) instead
   s->sketch.generate(p, c.seed, c.omega_mode, c.omega_threads,
                      col_block_chain(c.sketcher), st);
   if (!via_a) {
-    s->sketch.project(p, c.precision, A, lda, a_dtype, a_order, s->Y.p, st, true);
-  } else {
-    if (a_dtype == MCNLA_F64 && a_order == MCNLA_ROW_MAJOR && lda == n) {
-      cx.Ar = static_cast<const double*>(A);
-    } else {
-      to_rowmajor_f64(A, lda, a_dtype == MCNLA_F32, a_order == MCNLA_COL_MAJOR, m, n,
-                      s->A64.as<double>(), st);
-      cx.Ar = s->A64.as<double>();
+    // an FP64 sketch by residues works in the buffer of the Gram's partials
+    ResidueScratch scratch;
+    if (c.precision == MCNLA_PREC_F64) {
+      scratch.ws = s->gram.partial.p;
+      scratch.bytes = s->gram.partial.bytes;
+      scratch.limit = s->gram.partial_bytes(false, m, nl);
+      scratch.flag = s->bad.as<int>() + mcnla_solver_s::kSketchFlag;
     }
-    s->gram.run(cx.Ar, false, m, n, s->H.as<double>(), st);
+    s->sketch.project(p, c.precision, A, lda, a_dtype, a_order, s->Y.p, st, true, scratch);
+  } else {
+    int* flag = s->bad.as<int>() + mcnla_solver_s::kGramFlag;
+    const bool rm = a_order == MCNLA_ROW_MAJOR, f32 = a_dtype == MCNLA_F32;
+    if (rm && s->gram.by_residues(m, n)) {
+      // a row-major A is packed as it is, in either type, and Qbar = A X streams it too: the FP64
+      // copy is not made, and its buffer is the workspace
+      s->gram.run(A, lda, f32, m, n, s->H.as<double>(), flag, st, &s->A64);
+    } else {
+      if (!f32 && rm && lda == n) {
+        cx.Ar = static_cast<const double*>(A);
+      } else {
+        to_rowmajor_f64(A, lda, f32, !rm, m, n, s->A64.as<double>(), st);
+        cx.Ar = s->A64.as<double>();
+      }
+      s->gram.run(cx.Ar, n, false, m, n, s->H.as<double>(), flag, st);
+    }
   }
 }
 
@@ -1122,7 +1266,8 @@ void solve_orthogonalize(mcnla_solver_s* s, hipStream_t st, SolveCtx& cx) {
   // the one eigen-solve it needs running on a second stream beside the integrator.  The
   // combining integrators depend on every basis and keep the eigen transforms.
   if (!via_a) {
-    s->gram.run(s->Y.p, false, m, nl, s->G.as<double>(), st);
+    s->gram.run(s->Y.p, nl, false, m, nl, s->G.as<double>(),
+                s->bad.as<int>() + mcnla_solver_s::kGramFlag, st);
   } else {  // G = Omega' (H Omega)
     GemmF64Args hp = plan_h_omega(n, nl, s->tune.h_omega, kern_bit(s->tune, kKernHOmega));
     hp.A = s->H.p;
@@ -1657,7 +1802,8 @@ mcnla_status mcnla_sketcher_run(mcnla_stage s, const void* A, int64_t lda, int a
     }
     k->core.generate(p, k->seed, k->mode, k->threads, col_block_chain(k->kind), st);
     k->timer.mark(st);
-    k->core.project(p, k->precision, A, lda, a_dtype, a_order, Y, st);
+    const ResidueScratch scratch = k->scratch(A, lda, a_dtype, a_order, Y);
+    k->core.project(p, k->precision, A, lda, a_dtype, a_order, Y, st, false, scratch);
     for (int64_t q = 0; q < k->exponent; ++q) {  // gaussian_projection_sketcher.hpp:96-100
       GemmF64Args t;  // Omega := A' Y  (n x Nl)
       t.M = p.ncol;
@@ -1679,7 +1825,8 @@ mcnla_status mcnla_sketcher_run(mcnla_stage s, const void* A, int64_t lda, int a
         t.partial = k->partial.as<double>();
       }
       gemm_f64(t, st);
-      k->core.project(p, k->precision, A, lda, a_dtype, a_order, Y, st);  // Y := A Omega
+      // Y := A Omega
+      k->core.project(p, k->precision, A, lda, a_dtype, a_order, Y, st, false, scratch);
     }
     k->timer.mark(st);
     k->computed = true;

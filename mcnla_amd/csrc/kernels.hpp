@@ -59,6 +59,31 @@ int64_t gemm_f64_splits_for(int64_t tiles, int64_t K, int64_t target_blocks);
 // the remaining rows (*tail_splits, 1 when none), whose last round would otherwise run a few
 // full-length workgroups on a mostly idle device.
 int64_t gemm_f64_dma_tail(int64_t M, int64_t N, int64_t K, int64_t* tail_splits);
+// ------------------------------------------------------------------------------------------------
+// FP64 products by residues on INT8 MFMA (gemm_residue.hip).
+struct ResidueArgs {
+  int64_t M = 0, N = 0, K = 0;
+  const void* A = nullptr;  // element (i, k) at A[i + k*lda] if a_mcontig else A[i*lda + k]
+  int64_t lda = 0;
+  bool a_mcontig = true;
+  bool a_f32 = false;
+  const double* B = nullptr;  // element (k, j) at B[k*ldb + j] if b_ncontig else B[k + j*ldb]
+  int64_t ldb = 0;
+  bool b_ncontig = true;
+  bool sym = false;           // C = A A' (N = M, B unused), both triangles written
+  double* C = nullptr;        // row-major, ldc
+  int64_t ldc = 0;
+};
+// Workspace of the product, at most `limit` bytes; 0 when it cannot run in that.  The result does
+// not depend on the workspace.
+size_t residue_bytes(const ResidueArgs& a, size_t limit, double* cost = nullptr);
+// Whether the product is faster by residues than on the FP64 kernels of gemm_f64, with a workspace
+// of `limit` bytes.
+bool residue_pays(const ResidueArgs& a, size_t limit);
+// Enqueues the product.  *flag (device) ends nonzero when an operand has a row without a scale (a
+// non-finite entry, or a norm out of range): C is undefined then, and the caller replaces it by
+// an FP64 product gated on the flag (gate_t = 1).  `ws` is 256-byte aligned.
+void gemm_residue(const ResidueArgs& a, void* ws, size_t ws_bytes, int* flag, hipStream_t st);
 // Compute units of the current device (cached per device).
 int compute_units();
 
