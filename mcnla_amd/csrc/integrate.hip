@@ -13,7 +13,6 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "small.hpp"
-#include "tall_direct.hpp"
 
 #include <algorithm>
 #include <climits>
@@ -24,11 +23,10 @@ namespace mcnla {
 struct IntegratorState {
   int converged_at;  // iteration index that met the stopping test, INT_MAX while running
   int nan_seen;      // a non-finite value appeared in the l x l step
-  int ticket;        // workgroups done with the current fused reduction (reset by the last one)
-  int pad;
   double res;        // last residual (KN: ||s - 1||_2, WY: mu)
   double taug, zeta, phi, mu;  // Wen-Yin scalars
 };
+static_assert(sizeof(IntegratorState) <= 256, "the state's slot in the workspace");
 
 namespace {
 
@@ -128,8 +126,14 @@ __global__ void reduce_partials_kernel(int t, const IntegratorState* st,
   out[q] = scale * sum_partials(P, nblk, count, q);
 }
 
+// A KN partial holds the lower triangles of Bc'Bc and of Bc'Bg + Bg'Bc over some rows, one after
+// the other, row by row: l (l + 1) doubles.
+__device__ __forceinline__ int tri(int i, int j) {
+  return i >= j ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i;
+}
+
 // The KN l x l step (row_block_kolmogorov_nagumo_integrator.hpp:146-201): Dc = Bc'Bc/N and
-// Dgc = Bc'Bgc/N from the per-block partials P (nblk blocks of [Bc'Bc, Bc'Bgc]), Z = Dgc - Dc^2,
+// Dgc = sym(Bc'Bgc)/N from the partials P (nblk of them, as above), Z = Dgc - Dc^2,
 // eig(Z), s = sqrt(1/2 + sqrt(1/4 - lambda)), C = V diag(s) V', Cinv = V diag(1/s) V',
 // F = C - Dc Cinv, convergence when !(||s - 1||_2 >= tol).
 //
@@ -139,267 +143,711 @@ __global__ void reduce_partials_kernel(int t, const IntegratorState* st,
 // semidefinite with lambda <= 1/4), and ||s - 1||_2 = ||C - I||_F.  Should an iteration not
 // converge (lambda at or above 1/4, non-finite input) the step falls back to a Jacobi
 // eigen-decomposition and the formulas above, which also reproduce the reference's NaN there.
-// Runs on NT threads (all of the workgroup).
-template <int NT>
-__device__ void kn_step_eigen(int t, IntegratorState* st, int l, double invN, double tol,
-                              const double* __restrict__ P, int64_t nblk, double* __restrict__ F,
-                              double* __restrict__ Cinv, double* dc, double* a, double* v,
-                              double* z) {
+// The series form of the step, for x = 4Z of small norm (all but the first few iterations: rho =
+// ||x||_F falls below 0.13 within five of 20 to 80 iterations on the workloads measured).  With
+// s = sqrt(1/2 + sqrt(1/4 - z)) = sqrt((1 + sqrt(1 - x)) / 2), the powers s^-r are
+// sum_k a_k x^k with a_0 = 1, a_{k+1} / a_k = (2k + r)(2k + r + 1) / (4 (k + 1)(k + r + 1)) (the
+// r-th power of the Catalan generating function): C is r = -1/2 and Cinv r = 1/2.  Both are
+// evaluated to degree 4b - 1 (Paterson-Stockmeyer with x, x^2, x^3, x^4), b the smallest whose
+// truncation is below 1.5e-17.
+constexpr int kSeriesMaxB = 10;
+struct SeriesTable {
+  double c[4 * kSeriesMaxB] = {}, ci[4 * kSeriesMaxB] = {};
+  constexpr SeriesTable() {
+    for (int which = 0; which < 2; ++which) {
+      const double r = which == 0 ? -0.5 : 0.5;
+      double a = 1.0;
+      for (int k = 0; k < 4 * kSeriesMaxB; ++k) {
+        (which == 0 ? c : ci)[k] = a;
+        a *= (2 * k + r) * (2 * k + r + 1) / (4 * (k + 1) * (k + r + 1));
+      }
+    }
+  }
+};
+__constant__ const SeriesTable kSeries;
+// rho up to which degree 4b - 1 suffices, b = 2, 3, ... (the tail sum a_k rho^k, k >= 4b, of Cinv
+// is 1.5e-17 there).
+__device__ __forceinline__ int series_blocks(double rho) {
+  constexpr double limit[kSeriesMaxB - 1] = {0.01435, 0.06178, 0.12669, 0.19394, 0.25695,
+                                             0.31369, 0.36401, 0.40845, 0.44771};
+  int b = 2;
+  for (; b <= kSeriesMaxB; ++b)
+    if (rho <= limit[b - 2]) return b;
+  return 0;  // also for a NaN
+}
+
+constexpr int kStepThreads = 512;
+constexpr int kStepWaves = kStepThreads / kWave;
+
+// Leading dimension of the np x np LDS matrices of the series step: rows and column walks of the
+// 16 x 16 x 4 fragments on distinct banks (at np = 64, where four matrices would not fit, pairs).
+template <int NP>
+__host__ __device__ constexpr int series_ld() {
+  return NP == 16 ? 18 : NP == 64 ? 66 : 50;
+}
+constexpr int kStepBuf = kMaxL * series_ld<kMaxL>();  // doubles per buffer
+static_assert(kMaxL * (kMaxL + 1) <= kStepBuf, "the other forms' buffers fit");
+
+// One 16 x 16 tile of A B + acc for symmetric A, B in LDS (both read along rows).
+template <int NP>
+__device__ __forceinline__ d4 sym_tile(const double* A, const double* B, int i0, int j0, d4 acc) {
+  constexpr int LD = series_ld<NP>();
+  const int lane = threadIdx.x & (kWave - 1), c = lane & 15, kq = lane >> 4;
+#pragma unroll
+  for (int k = 0; k < NP; k += 4)
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A[(k + kq) * LD + i0 + c], B[(k + kq) * LD + j0 + c],
+                                               acc, 0, 0, 0);
+  return acc;
+}
+
+// Writes a tile of the lower triangle and its mirror image.
+template <int NP>
+__device__ __forceinline__ void put_sym(double* X, int i0, int j0, const d4& v) {
+  constexpr int LD = series_ld<NP>();
+  const int lane = threadIdx.x & (kWave - 1);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int i = i0 + (lane >> 4) + 4 * r, j = j0 + (lane & 15);
+    X[i * LD + j] = v[r];
+    if (i0 != j0) X[j * LD + i] = v[r];
+  }
+}
+
+// The lower-triangle tile q (0, 1, ... row by row): its origin.
+__device__ __forceinline__ void lower_tile(int q, int& i0, int& j0) {
+  const int ti = q >= 6 ? 3 : q >= 3 ? 2 : q >= 1 ? 1 : 0;
+  i0 = ti * 16;
+  j0 = (q - ti * (ti + 1) / 2) * 16;
+}
+
+// All forms of the step run on kStepThreads threads (the whole workgroup) with four buffers of
+// kStepBuf doubles in smem, and leave Cinv in the second and F in the third (leading dimension
+// series_ld<NP>(); F is zero past l).  They return ||C - I||_F (NaN or infinite when Z is not).
+
+// The eigen-decomposition form.
+template <int NP>
+__device__ double kn_step_eigen(int l, double invN, const double* __restrict__ P, int64_t nblk,
+                                double* smem) {
   __shared__ double s[kMaxL];
   __shared__ double cs[2 * kMaxL];
   __shared__ int pq[2 * kMaxL];
   __shared__ double red[8];
-  const int ld = lds_ld(l);
-  const int ll = l * l;
-  for (int e = threadIdx.x; e < 2 * ll; e += NT) {  // Dc into dc, Dgc into a
-    const double x = invN * sum_partials(P, nblk, 2 * ll, e);
-    const int q = e % ll;
-    (e < ll ? dc : a)[(q / l) * ld + q % l] = x;
+  constexpr int LD = series_ld<NP>(), EP = (NP * NP + kStepThreads - 1) / kStepThreads;
+  double* z = smem;
+  double* v = smem + kStepBuf;
+  double* a = smem + 2 * kStepBuf;
+  double* dc = smem + 3 * kStepBuf;
+  const int ld = lds_ld(l), ll = l * l, half = l * (l + 1) / 2;
+  for (int e = threadIdx.x; e < ll; e += kStepThreads) {  // Dc into dc, Dgc into a
+    const int i = e / l, j = e % l, q = tri(i, j);
+    dc[i * ld + j] = invN * sum_partials(P, nblk, 2 * half, q);
+    a[i * ld + j] = 0.5 * invN * sum_partials(P, nblk, 2 * half, half + q);
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < ll; e += NT) {  // Z = sym(Dgc) - Dc Dc'
+  for (int e = threadIdx.x; e < ll; e += kStepThreads) {  // Z = Dgc - Dc Dc'
     const int i = e / l, j = e % l;
-    double x = 0.5 * (a[i * ld + j] + a[j * ld + i]);
+    double x = a[i * ld + j];
     for (int q = 0; q < l; ++q) x -= dc[i * ld + q] * dc[j * ld + q];
     z[i * ld + j] = x;
   }
   __syncthreads();
   lds_jacobi(l, z, v, true, cs, pq, red);
-  for (int i = threadIdx.x; i < l; i += NT) s[i] = sqrt(0.5 + sqrt(0.25 - z[i * ld + i]));
+  for (int i = threadIdx.x; i < l; i += kStepThreads)
+    s[i] = sqrt(0.5 + sqrt(0.25 - z[i * ld + i]));
   __syncthreads();
-  for (int e = threadIdx.x; e < ll; e += NT) {  // Cinv into `a`
+  for (int e = threadIdx.x; e < ll; e += kStepThreads) {  // Cinv into `a`
     const int i = e / l, j = e % l;
     double ci = 0.0;
     for (int q = 0; q < l; ++q) ci += v[i * ld + q] * v[j * ld + q] / s[q];
     a[i * ld + j] = ci;
-    Cinv[e] = ci;
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < ll; e += NT) {  // F = C - Dc Cinv, C on the fly
-    const int i = e / l, j = e % l;
-    double c = 0.0;
-    for (int q = 0; q < l; ++q) c += v[i * ld + q] * v[j * ld + q] * s[q];
-    double dci = 0.0;
-    for (int q = 0; q < l; ++q) dci += dc[i * ld + q] * a[q * ld + j];
-    F[e] = c - dci;
-  }
-  if (threadIdx.x == 0) {
-    double r = 0.0;
-    bool bad = false;
-    for (int q = 0; q < l; ++q) {
-      r += (s[q] - 1.0) * (s[q] - 1.0);
-      if (!isfinite(s[q])) bad = true;
+  double f[EP], ci[EP];  // F = C - Dc Cinv, C on the fly
+#pragma unroll
+  for (int u = 0; u < EP; ++u) {
+    const int e = threadIdx.x + u * kStepThreads, i = e / NP, j = e % NP;
+    f[u] = 0.0;
+    ci[u] = 0.0;
+    if (i < l && j < l) {
+      double c = 0.0, dci = 0.0;
+      for (int q = 0; q < l; ++q) {
+        c += v[i * ld + q] * v[j * ld + q] * s[q];
+        dci += dc[i * ld + q] * a[q * ld + j];
+      }
+      f[u] = c - dci;
+      ci[u] = a[i * ld + j];
     }
-    r = sqrt(r);
-    st->res = r;
-    if (bad) st->nan_seen = 1;
-    if (!(r >= tol)) st->converged_at = t;
   }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < EP; ++u) {
+    const int e = threadIdx.x + u * kStepThreads, i = e / NP, j = e % NP;
+    if (i >= NP) break;
+    smem[kStepBuf + i * LD + j] = ci[u];
+    smem[2 * kStepBuf + i * LD + j] = f[u];
+  }
+  __syncthreads();
+  double r = 0.0;
+  for (int q = 0; q < l; ++q) r += (s[q] - 1.0) * (s[q] - 1.0);
+  return sqrt(r);
 }
 
-// The NS form of the step; smem holds four (kMaxL x (kMaxL+1)) buffers, red NT/64 doubles.
-template <int NT>
-__device__ void kn_step_ns(int t, IntegratorState* st, int l, double invN, double tol,
-                           const double* __restrict__ P, int64_t nblk, double* __restrict__ F,
-                           double* __restrict__ Cinv, double* smem, double* red) {
-  constexpr int NW = NT / kWave;
-  constexpr int kBuf = kMaxL * (kMaxL + 1);
-  double* sDc = smem;
-  double* sY = smem + kBuf;
-  double* sW = smem + 2 * kBuf;
-  double* sT = smem + 3 * kBuf;
-  const int np = pad16(l), ld = np + 1, ll = l * l;
+// The Newton-Schulz form: X = (I - 4Z)^{1/2}, C = ((I + X)/2)^{1/2}, Cinv = C^{-1}.
+template <int NP>
+__device__ double kn_step_ns(int l, double invN, const double* __restrict__ P, int64_t nblk,
+                             double* smem, double* red) {
+  constexpr int LD = series_ld<NP>(), NT1 = NP / 16;
+  double* sY = smem;
+  double* sW = smem + kStepBuf;
+  double* sT = smem + 2 * kStepBuf;
+  double* sDc = smem + 3 * kStepBuf;
+  const int half = l * (l + 1) / 2;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid & (kWave - 1);
-  const int nt1 = np / 16, ntiles = nt1 * nt1;
-  // Dc into sDc, Dgc into sT, both zero-padded to np x np
-  for (int e = tid; e < np * np; e += NT) {
-    const int i = e / np, j = e % np;
+  // Dc into sDc, Dgc into sT, both zero-padded
+  for (int e = tid; e < NP * NP; e += kStepThreads) {
+    const int i = e / NP, j = e % NP, q = tri(i, j);
     double dc = 0.0, dgc = 0.0;
-    if (i < l && j < l) sum_partials2(P, nblk, 2 * ll, i * l + j, ll + i * l + j, dc, dgc);
-    sDc[i * ld + j] = invN * dc;
-    sT[i * ld + j] = invN * dgc;
+    if (i < l && j < l) sum_partials2(P, nblk, 2 * half, q, half + q, dc, dgc);
+    sDc[i * LD + j] = invN * dc;
+    sT[i * LD + j] = 0.5 * invN * dgc;
   }
   __syncthreads();
-  // Y = I - 4Z with Z = sym(Dgc) - Dc Dc'
-  for (int tile = wave; tile < ntiles; tile += NW) {
-    const int i0 = (tile / nt1) * 16, j0 = (tile % nt1) * 16;
-    const d4 acc = lds_mfma_tile<false, true>(np, ld, sDc, sDc, i0, j0);
+  // Y = I - 4Z with Z = Dgc - Dc Dc'
+  for (int tile = wave; tile < NT1 * NT1; tile += kStepWaves) {
+    const int i0 = (tile / NT1) * 16, j0 = (tile % NT1) * 16;
+    const d4 acc = lds_mfma_tile<false, true>(NP, LD, sDc, sDc, i0, j0);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = i0 + (lane >> 4) + 4 * r, j = j0 + (lane & 15);
-      const double zz = 0.5 * (sT[i * ld + j] + sT[j * ld + i]) - acc[r];
-      sY[i * ld + j] = ((i == j) ? 1.0 : 0.0) - 4.0 * zz;
+      sY[i * LD + j] = ((i == j) ? 1.0 : 0.0) - 4.0 * (sT[i * LD + j] - acc[r]);
     }
   }
   __syncthreads();
-  int ok = lds_ns_sqrt<NW>(np, ld, sY, sW, sT, red, 60);
+  int ok = lds_ns_sqrt<kStepWaves>(NP, LD, sY, sW, sT, red, 60);
   if (ok > 0) {
-    for (int e = tid; e < np * np; e += NT) {
-      const int i = e / np, j = e % np;
-      sY[i * ld + j] = 0.5 * (((i == j) ? 1.0 : 0.0) + sY[i * ld + j]);
+    for (int e = tid; e < NP * NP; e += kStepThreads) {
+      const int i = e / NP, j = e % NP;
+      sY[i * LD + j] = 0.5 * (((i == j) ? 1.0 : 0.0) + sY[i * LD + j]);
     }
     __syncthreads();
-    ok = lds_ns_sqrt<NW>(np, ld, sY, sW, sT, red, 60);
+    ok = lds_ns_sqrt<kStepWaves>(NP, LD, sY, sW, sT, red, 60);
   }
-  if (ok <= 0) {  // rare: eigen-decomposition instead (uses its own layout of the buffers)
-    kn_step_eigen<NT>(t, st, l, invN, tol, P, nblk, F, Cinv, sDc, sT, sW, sY);
-    return;
+  if (ok <= 0) {  // rare: eigen-decomposition instead
+    __syncthreads();
+    return kn_step_eigen<NP>(l, invN, P, nblk, smem);
   }
-  // C = sY, Cinv = sW; F = C - Dc Cinv; ||C - I||_F
+  // C = sY, Cinv = sW; F = C - Dc Cinv; ||C - I||_F (the padding of C is the identity)
   double rs = 0.0;
-  for (int tile = wave; tile < ntiles; tile += NW) {
-    const int i0 = (tile / nt1) * 16, j0 = (tile % nt1) * 16;
-    const d4 acc = lds_mfma_tile<false, false>(np, ld, sDc, sW, i0, j0);
+  for (int tile = wave; tile < NT1 * NT1; tile += kStepWaves) {
+    const int i0 = (tile / NT1) * 16, j0 = (tile % NT1) * 16;
+    const d4 acc = lds_mfma_tile<false, false>(NP, LD, sDc, sW, i0, j0);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = i0 + (lane >> 4) + 4 * r, j = j0 + (lane & 15);
-      if (i < l && j < l) {
-        const double c = sY[i * ld + j];
-        F[i * l + j] = c - acc[r];
-        Cinv[i * l + j] = sW[i * ld + j];
-        const double d = c - ((i == j) ? 1.0 : 0.0);
-        rs += d * d;
-      }
+      const double c = sY[i * LD + j];
+      sT[i * LD + j] = i < l && j < l ? c - acc[r] : 0.0;
+      const double d = c - ((i == j) ? 1.0 : 0.0);
+      rs += d * d;
     }
   }
   rs = wave_sum(rs);
   __syncthreads();  // red is reused
   if (lane == 0) red[wave] = rs;
   __syncthreads();
-  if (tid == 0) {
-    double tot = 0.0;
-    for (int w = 0; w < NW; ++w) tot += red[w];
-    const double r = sqrt(tot);
-    st->res = r;
-    if (!isfinite(r)) st->nan_seen = 1;
-    if (!(r >= tol)) st->converged_at = t;
-  }
+  double tot = 0.0;
+  for (int w = 0; w < kStepWaves; ++w) tot += red[w];
+  return sqrt(tot);
 }
 
-// One KN iteration's reductions and l x l step in one launch (after the split-K GEMM that
-// leaves Pbg[s] = partial Bs * Bc over the s-th K range):
-//   1. workgroup b owns rows [64 b, 64 b + 64) of the Nl x l matrices: Bgc = invN sum_s Pbg[s]
-//      (fixed order), written out, and its block partials Bc'Bc, Bc'Bgc -> P[b] (f64 MFMA);
-//   2. the last workgroup to finish (a ticket counter, taken after a device-scope fence; no
-//      waiting) sums P over blocks in block order and runs the NS step above.
-// The result is deterministic: no sum depends on which workgroup finishes last.
-constexpr int kStepThreads = 512;
-constexpr int kStepRows = 64;
-
-// Workgroup `blk` of nblk (kStepThreads threads).
-__device__ __forceinline__ void kn_reduce_step_body(
-    int t, IntegratorState* st, int64_t nl, int l, double invN, double tol,
-    const double* __restrict__ Pbg, int64_t splits, const double* __restrict__ B,
-    double* __restrict__ Bg, double* __restrict__ P, int64_t nblk, double* __restrict__ F,
-    double* __restrict__ Cinv, int64_t blk) {
-  if (skip(st, t)) return;
-  constexpr int kBuf = kMaxL * (kMaxL + 1);
-  static_assert(2 * kStepRows * (kMaxL + 1) <= 4 * kBuf, "row blocks fit the step buffers");
-  __shared__ double smem[4 * kBuf];
-  __shared__ double red[kStepThreads / kWave];
-  __shared__ int last;
-  const int tid = threadIdx.x;
-  const int ldr = kMaxL + 1;
-  double* sB = smem;
-  double* sG = smem + kStepRows * ldr;
-  const int64_t r0 = blk * kStepRows;
-  const int64_t per = nl * l;
-  // elements e and e + kStepThreads together, so two sums' loads are in flight at once
-  for (int e = tid; e < kStepRows * l; e += 2 * kStepThreads) {
-    const int e2 = e + kStepThreads;
-    const int64_t ra = r0 + e / l, rb = r0 + e2 / l;
-    const bool va = ra < nl, vb = e2 < kStepRows * l && rb < nl;
-    const int64_t oa = ra * l + e % l, ob = rb * l + e2 % l;
-    double ga = 0.0, gb = 0.0;
-    if (va) sum_partials2(Pbg, splits, per, oa, vb ? ob : -1, ga, gb);
-    if (va) {
-      ga *= invN;
-      Bg[oa] = ga;
-    }
-    sB[(e / l) * ldr + e % l] = va ? B[oa] : 0.0;
-    sG[(e / l) * ldr + e % l] = va ? ga : 0.0;
-    if (e2 < kStepRows * l) {
-      if (vb) {
-        gb *= invN;
-        Bg[ob] = gb;
-      }
-      sB[(e2 / l) * ldr + e2 % l] = vb ? B[ob] : 0.0;
-      sG[(e2 / l) * ldr + e2 % l] = vb ? gb : 0.0;
-    }
-  }
-  __syncthreads();
-  const int ll = l * l;
-  double* Pb = P + blk * (2 * ll);
-  {  // [B'B, B'G] over the block's rows on f64 MFMA tiles: 2 (np/16)^2 tiles over the waves
-    constexpr int NW = kStepThreads / kWave;
-    const int wave = tid / kWave, lane = tid % kWave;
-    const int nt1 = pad16(l) / 16, tiles = nt1 * nt1;
-    for (int tile = wave; tile < 2 * tiles; tile += NW) {
-      const int part = tile / tiles, i0 = ((tile % tiles) / nt1) * 16, j0 = (tile % nt1) * 16;
-      const double* y = part == 0 ? sB : sG;
-      d4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-      for (int k0 = 0; k0 < kStepRows; k0 += 4) {
-        const int k = k0 + lane / 16;
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(sB[k * ldr + i0 + lane % 16],
-                                                   y[k * ldr + j0 + lane % 16], acc, 0, 0, 0);
-      }
+// Returns false (uniformly, with nothing written) when x is too large for the series.  Waves own
+// lower-triangle tiles of the results: all matrices are symmetric polynomials of Z (and Dc), so
+// only those tiles are computed, six MFMA chains of NP / 4 where the square-root iterations take
+// eighteen; every barrier is one of about 5 + 2b.
+template <int NP>
+__device__ bool kn_step_series(int l, double invN, const double* __restrict__ P, int64_t nblk,
+                               double* smem, double* red, double* res) {
+  constexpr int LD = series_ld<NP>(), NT1 = NP / 16, NTL = NT1 * (NT1 + 1) / 2;
+  constexpr int Q1 = (NTL + kStepWaves - 1) / kStepWaves;      // tiles per wave
+  constexpr int Q2 = (2 * NTL + kStepWaves - 1) / kStepWaves;  // tiles of C and Cinv per wave
+  double* bX = smem;                  // x, then the polynomial of C
+  double* bX2 = smem + kStepBuf;      // x^2, then the polynomial of Cinv
+  double* bX4 = smem + 2 * kStepBuf;  // Dgc, then x^4
+  double* bDc = smem + 3 * kStepBuf;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid & (kWave - 1);
+  const int half = l * (l + 1) / 2;
+  const d4 zero = {0.0, 0.0, 0.0, 0.0};
+  // Dc into bDc, Dgc into bX4: job q < NTL is the tile q of Dc, the rest those of Dgc; the loads of
+  // all of a wave's jobs and of four partials are in flight together
+  {
+    d4 sum[Q2];
+    int off[Q2][4];
+    bool in[Q2][4];
+#pragma unroll
+    for (int q = 0; q < Q2; ++q) {
+      const int job = wave + q * kStepWaves;
+      int i0, j0;
+      lower_tile(job < NTL ? job : job - NTL, i0, j0);
+      sum[q] = zero;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int i = i0 + lane / 16 + 4 * r, j = j0 + lane % 16;
-        if (i < l && j < l) Pb[part * ll + i * l + j] = acc[r];
+        const int i = i0 + (lane >> 4) + 4 * r, j = j0 + (lane & 15);
+        in[q][r] = job < 2 * NTL && i < l && j < l;
+        off[q][r] = in[q][r] ? (job < NTL ? 0 : half) + tri(i, j) : 0;
       }
     }
+    constexpr int UB = Q2 == 1 ? 16 : Q2 == 2 ? 8 : 4;
+    for (int64_t b = 0; b < nblk; b += UB) {
+      double v[UB][Q2][4];
+#pragma unroll
+      for (int u = 0; u < UB; ++u) {
+        const double* Pb = P + (b + u < nblk ? b + u : b) * 2 * half;
+#pragma unroll
+        for (int q = 0; q < Q2; ++q)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[u][q][r] = Pb[off[q][r]];
+      }
+#pragma unroll
+      for (int u = 0; u < UB; ++u)
+        if (b + u < nblk) {
+#pragma unroll
+          for (int q = 0; q < Q2; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sum[q][r] += v[u][q][r];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < Q2; ++q) {
+      const int job = wave + q * kStepWaves;
+      if (job >= 2 * NTL) continue;
+      int i0, j0;
+      lower_tile(job < NTL ? job : job - NTL, i0, j0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sum[q][r] = in[q][r] ? (job < NTL ? invN : 0.5 * invN) * sum[q][r] : 0.0;
+      put_sym<NP>(job < NTL ? bDc : bX4, i0, j0, sum[q]);
+    }
   }
-  __threadfence();
   __syncthreads();
-  if (tid == 0) last = (atomicAdd(&st->ticket, 1) == static_cast<int>(nblk) - 1);
+  // x = 4 (Dgc - Dc^2) and rho^2 = ||x||_F^2
+  double ss = 0.0;
+#pragma unroll
+  for (int q = 0; q < Q1; ++q) {
+    const int tile = wave + q * kStepWaves;
+    if (tile >= NTL) continue;
+    int i0, j0;
+    lower_tile(tile, i0, j0);
+    const d4 d = sym_tile<NP>(bDc, bDc, i0, j0, zero);
+    d4 x;
+    double s4 = 0.0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      x[r] = 4.0 * (bX4[(i0 + (lane >> 4) + 4 * r) * LD + j0 + (lane & 15)] - d[r]);
+      s4 += x[r] * x[r];
+    }
+    ss += i0 != j0 ? 2.0 * s4 : s4;
+    put_sym<NP>(bX, i0, j0, x);
+  }
+  ss = wave_sum(ss);
+  if (lane == 0) red[wave] = ss;
   __syncthreads();
-  if (!last) return;
-  __threadfence();
-  if (tid == 0) st->ticket = 0;  // ready for the next iteration's launch
-  kn_step_ns<kStepThreads>(t, st, l, invN, tol, P, nblk, F, Cinv, smem, red);
+  double rho2 = 0.0;
+#pragma unroll
+  for (int w = 0; w < kStepWaves; ++w) rho2 += red[w];
+  const int nb = series_blocks(sqrt(rho2));
+  if (nb == 0) {
+    __syncthreads();  // the buffers are reused
+    return false;
+  }
+#pragma unroll
+  for (int q = 0; q < Q1; ++q) {  // x^2
+    const int tile = wave + q * kStepWaves;
+    if (tile >= NTL) continue;
+    int i0, j0;
+    lower_tile(tile, i0, j0);
+    put_sym<NP>(bX2, i0, j0, sym_tile<NP>(bX, bX, i0, j0, zero));
+  }
+  __syncthreads();
+  // x^4 into LDS; every owner of a tile of C (jobs 0 .. NTL - 1) or Cinv (the rest) keeps the
+  // tile of x, x^2 and x^3
+  d4 x1[Q2], x2[Q2], x3[Q2];
+#pragma unroll
+  for (int q = 0; q < Q2; ++q) {
+    const int job = wave + q * kStepWaves;
+    if (job >= 2 * NTL) continue;
+    int i0, j0;
+    lower_tile(job < NTL ? job : job - NTL, i0, j0);
+    if (job < NTL) put_sym<NP>(bX4, i0, j0, sym_tile<NP>(bX2, bX2, i0, j0, zero));
+    x3[q] = sym_tile<NP>(bX, bX2, i0, j0, zero);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = i0 + (lane >> 4) + 4 * r, j = j0 + (lane & 15);
+      x1[q][r] = bX[i * LD + j];
+      x2[q][r] = bX2[i * LD + j];
+    }
+  }
+  __syncthreads();
+  for (int b = nb - 1; b >= 0; --b) {  // P := P x^4 + a_4b I + ... + a_4b+3 x^3
+    d4 acc[Q2];
+#pragma unroll
+    for (int q = 0; q < Q2; ++q) {
+      const int job = wave + q * kStepWaves;
+      if (job >= 2 * NTL) continue;
+      const bool inv = job >= NTL;
+      int i0, j0;
+      lower_tile(inv ? job - NTL : job, i0, j0);
+      const double* a = (inv ? kSeries.ci : kSeries.c) + 4 * b;
+      const double a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = i0 + (lane >> 4) + 4 * r, j = j0 + (lane & 15);
+        acc[q][r] = fma(a3, x3[q][r], fma(a2, x2[q][r], fma(a1, x1[q][r], i == j ? a0 : 0.0)));
+      }
+      if (b != nb - 1) acc[q] = sym_tile<NP>(inv ? bX2 : bX, bX4, i0, j0, acc[q]);
+    }
+    if (b != nb - 1) __syncthreads();
+#pragma unroll
+    for (int q = 0; q < Q2; ++q) {
+      const int job = wave + q * kStepWaves;
+      if (job >= 2 * NTL) continue;
+      int i0, j0;
+      lower_tile(job < NTL ? job : job - NTL, i0, j0);
+      put_sym<NP>(job < NTL ? bX : bX2, i0, j0, acc[q]);
+    }
+    __syncthreads();
+  }
+  // F = C - Dc Cinv over x^4, ||C - I||_F
+  double rs = 0.0;
+  for (int tile = wave; tile < NT1 * NT1; tile += kStepWaves) {
+    const int i0 = (tile / NT1) * 16, j0 = (tile % NT1) * 16;
+    const d4 acc = sym_tile<NP>(bDc, bX2, i0, j0, zero);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = i0 + (lane >> 4) + 4 * r, j = j0 + (lane & 15);
+      const double c = bX[i * LD + j];
+      bX4[i * LD + j] = i < l && j < l ? c - acc[r] : 0.0;
+      const double d = c - ((i == j) ? 1.0 : 0.0);
+      rs += d * d;  // the padding of C is the identity
+    }
+  }
+  rs = wave_sum(rs);
+  if (lane == 0) red[wave] = rs;
+  __syncthreads();
+  double tot = 0.0;
+  for (int w = 0; w < kStepWaves; ++w) tot += red[w];
+  *res = sqrt(tot);
+  return true;
 }
 
-// B+ = Bc F + Bg Cinv; E+ = Ec F + invN Bc Cinv; FF+ = FFc F (block 0).  Workgroup `blk` of
-// nblocks (kThreads threads), a grid-stride loop over the elements: every element is one dot
-// product in a fixed order, whatever the grid.
-__device__ __forceinline__ void kn_update_body(
-    int t, const IntegratorState* st, int64_t nl, int l, double invN,
-    const double* __restrict__ Bc, const double* __restrict__ Bg, double* __restrict__ Bp,
-    const double* __restrict__ Ec, double* __restrict__ Ep, const double* __restrict__ FFc,
-    double* __restrict__ FFp, const double* __restrict__ F, const double* __restrict__ Cinv,
-    int64_t blk, int64_t nblocks) {
+// A KN iteration is two or three launches:
+//   1. product: workgroup b owns rows [R b, R b + R) of the Nl x l matrices and forms Bg = Bs Bc / N
+//      on them: its 8 waves take an eighth of K each, both operands straight from L2 into MFMA
+//      registers, and sum their tiles through LDS in wave order; then its partial
+//      [Bc'Bc, Bc'Bg + Bg'Bc] -> P[b] (f64 MFMA, lower triangles);
+//   2. from nine workgroups on, kn_sum sums the partials element by element, in block order;
+//   3. update: every workgroup runs the l x l step for itself and updates its rows of B and E.
+// All sums are in a fixed order.  Repeating the step (6 us at l = 32, 17 us at l = 64) in every
+// workgroup costs no time; doing it once, in the last workgroup of the product to finish, cost a
+// ticket and a device-scope fence (4 us, twice with two levels of partials), one CU summing all
+// partials (45 GB/s: 8 us at Nl = 2048 and l = 32, 25 us at Nl = 8192 and l = 64) and F and Cinv
+// through memory.
+
+// Rows per workgroup of the product: 16, so that the chip fills, while that makes at most 256
+// workgroups, then 32 (twice the use of each line of Bc).
+int step_rows(int64_t nl) { return nl <= 4096 ? 16 : 32; }
+
+// Partials that the update sums itself.
+constexpr int64_t kDirectPartials = 8;
+
+// sums[e] = sum_b P[b][e]: 64 elements per workgroup, a quarter of the blocks per wave.
+__device__ __forceinline__ void kn_sum_body(const double* __restrict__ P, int64_t nblk, int count,
+                                            double* __restrict__ sums, int64_t blk) {
+  __shared__ double part[kThreads];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int64_t e = blk * kWave + lane;
+  const int64_t per = (nblk + 3) / 4, b0 = wave * per < nblk ? wave * per : nblk;
+  const int64_t n = b0 + per < nblk ? per : nblk - b0;
+  part[threadIdx.x] = e < count ? sum_partials(P + b0 * count, n, count, e) : 0.0;
+  __syncthreads();
+  if (wave == 0 && e < count)
+    sums[e] = ((part[lane] + part[64 + lane]) + part[128 + lane]) + part[192 + lane];
+}
+
+// The tile of Bs Bc of one wave: RB rows from r0 by NP columns over k in [k0, k1), in stages of
+// 16 k.  In a stage, lane group kq takes k = 4 kq .. 4 kq + 3 (the
+// same in both operands), so that a lane's four entries of Bs are 32 contiguous bytes and a row's
+// 16 are one line (VEC: 16-byte loads; Bs 16-byte aligned and nl even).  Columns past l and rows
+// past nl repeat valid ones (their results are not used); k past k1 enters as zero.
+template <int NP, int RB, bool VEC>
+__device__ __forceinline__ void kn_product(const double* __restrict__ Bs,
+                                           const double* __restrict__ B, int nl, int l, int r0,
+                                           int k0, int k1, d4 (&acc)[RB / 16][NP / 16]) {
+  constexpr int NT = NP / 16, RT = RB / 16;
+  const int lane = threadIdx.x & (kWave - 1), c = lane & 15, kq = lane >> 4;
+  const double* row[RT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    const int r = r0 + 16 * i + c;
+    row[i] = Bs + static_cast<int64_t>(r < nl ? r : nl - 1) * nl;
+  }
+  int col[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) col[j] = j * 16 + c < l ? j * 16 + c : l - 1;
+  // D stages of 16 k in registers: a stage's loads are issued D - 1 stages ahead (past the last
+  // whole stage they repeat it), with no branch in the loop that would make the compiler wait
+  constexpr int D = RT * NT <= 3 ? 4 : 3;
+  double a[D][RT][4], b[D][4][NT];
+  auto load = [&](int k, double (&x)[RT][4], double (&y)[4][NT]) {
+    const int kk = k + 4 * kq;
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      if constexpr (VEC) {
+        const double2 p = *reinterpret_cast<const double2*>(row[i] + kk);
+        const double2 q = *reinterpret_cast<const double2*>(row[i] + kk + 2);
+        x[i][0] = p.x;
+        x[i][1] = p.y;
+        x[i][2] = q.x;
+        x[i][3] = q.y;
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[i][u] = row[i][kk + u];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) y[u][j] = B[static_cast<int64_t>(kk + u) * l + col[j]];
+  };
+  auto mul = [&](const double (&x)[RT][4], const double (&y)[4][NT]) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i][u], y[u][j], acc[i][j], 0, 0, 0);
+  };
+  const int n = (k1 - k0) / 16;  // whole stages
+  if (n > 0) {
+#pragma unroll
+    for (int s = 0; s < D - 1; ++s) load(k0 + 16 * (s < n ? s : n - 1), a[s], b[s]);
+    int s0 = 0;
+    for (; s0 + D <= n; s0 += D) {
+#pragma unroll
+      for (int s = 0; s < D; ++s) {
+        const int ahead = s0 + s + D - 1;
+        load(k0 + 16 * (ahead < n ? ahead : n - 1), a[(s + D - 1) % D], b[(s + D - 1) % D]);
+        mul(a[s], b[s]);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < D - 1; ++s)
+      if (s0 + s < n) mul(a[s], b[s]);
+  }
+  if (k0 + 16 * n < k1) {  // the last, partial stage
+    const int kk = k0 + 16 * n + 4 * kq;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const bool in = kk + u < k1;
+      const int kc = in ? kk + u : k0;
+#pragma unroll
+      for (int i = 0; i < RT; ++i) a[0][i][u] = in ? row[i][kc] : 0.0;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) b[0][u][j] = B[static_cast<int64_t>(kc) * l + col[j]];
+    }
+    mul(a[0], b[0]);
+  }
+}
+
+// A wave's product tile, written to LDS (leading dimension NP + 2).
+template <int NP, int RB>
+__device__ __forceinline__ void kn_product_tile(const double* __restrict__ Bs,
+                                                const double* __restrict__ B, int nl, int l,
+                                                bool vec, int r0, int k0, int k1, double* out) {
+  constexpr int NT = NP / 16, RT = RB / 16;
+  const int lane = threadIdx.x & (kWave - 1);
+  d4 acc[RT][NT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+  if (vec)
+    kn_product<NP, RB, true>(Bs, B, nl, l, r0, k0, k1, acc);
+  else
+    kn_product<NP, RB, false>(Bs, B, nl, l, r0, k0, k1, acc);
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        out[(16 * i + (lane >> 4) + 4 * r) * (NP + 2) + 16 * j + (lane & 15)] = acc[i][j][r];
+}
+
+// Workgroup `blk` of the product (kStepThreads threads), `rows` (16 or 32) rows each; l <= NP.
+template <int NP>
+__device__ __forceinline__ void kn_product_body(int t, const IntegratorState* st, int nl, int l,
+                                                int rows, bool vec, double invN,
+                                                const double* __restrict__ Bs,
+                                                const double* __restrict__ B,
+                                                double* __restrict__ Bg, double* __restrict__ P,
+                                                int64_t blk) {
   if (skip(st, t)) return;
-  __shared__ double sF[kMaxL * kMaxL];
-  __shared__ double sC[kMaxL * kMaxL];
-  for (int e = threadIdx.x; e < l * l; e += kThreads) {
-    sF[e] = F[e];
-    sC[e] = Cinv[e];
+  constexpr int NT = NP / 16, LT = NP + 2;
+  __shared__ double smem[kStepWaves * 32 * LT];
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const int r0 = static_cast<int>(blk) * rows;
+  const int per = (nl + 16 * kStepWaves - 1) / (16 * kStepWaves) * 16;  // k per wave
+  const int k0 = wave * per < nl ? wave * per : nl, k1 = k0 + per < nl ? k0 + per : nl;
+  const int tile = rows * LT;
+  if (rows == 16)
+    kn_product_tile<NP, 16>(Bs, B, nl, l, vec, r0, k0, k1, smem + wave * tile);
+  else
+    kn_product_tile<NP, 32>(Bs, B, nl, l, vec, r0, k0, k1, smem + wave * tile);
+  __syncthreads();
+  // the rows of Bg (summed in wave order, written out) and of B, then side by side in LDS
+  constexpr int EP = 32 * NP / kStepThreads;  // elements per thread, at most
+  double gv[EP], bv[EP];
+#pragma unroll
+  for (int u = 0; u < EP; ++u) {
+    const int e = tid + u * kStepThreads, rr = e / NP, j = e % NP;
+    const bool in = rr < rows && r0 + rr < nl && j < l;
+    const int64_t o = static_cast<int64_t>(r0 + rr) * l + j;
+    bv[u] = in ? B[o] : 0.0;
+    double g = 0.0;
+    if (rr < rows) {
+#pragma unroll
+      for (int w = 0; w < kStepWaves; ++w) g += smem[w * tile + rr * LT + j];
+    }
+    gv[u] = in ? invN * g : 0.0;
+    if (in) Bg[o] = gv[u];
   }
   __syncthreads();
-  const int64_t total = nl * l;
-  for (int64_t e = blk * kThreads + threadIdx.x; e < total; e += nblocks * kThreads) {
-    const int64_t r = e / l;
-    const int j = e % l;
-    const double* bc = Bc + r * l;
-    const double* bg = Bg + r * l;
-    const double* ec = Ec + r * l;
-    double b = 0.0, ee = 0.0;
-    for (int q = 0; q < l; ++q) {
-      const double f = sF[q * l + j], ci = sC[q * l + j];
-      b += bc[q] * f + bg[q] * ci;
-      ee += ec[q] * f + invN * bc[q] * ci;
-    }
-    Bp[e] = b;
-    Ep[e] = ee;
+  constexpr int ldr = NP + 16;  // rows k, k + 1 half the banks apart
+  double* sB = smem;
+  double* sG = smem + 32 * ldr;
+#pragma unroll
+  for (int u = 0; u < EP; ++u) {
+    const int e = tid + u * kStepThreads, rr = e / NP, j = e % NP;
+    if (rr >= rows) break;
+    sB[rr * ldr + j] = bv[u];
+    sG[rr * ldr + j] = gv[u];
   }
-  if (blk == 0) {
-    for (int e = threadIdx.x; e < l * l; e += kThreads) {
-      const int i = e / l, j = e % l;
-      double acc = 0.0;
-      for (int q = 0; q < l; ++q) acc += FFc[i * l + q] * sF[q * l + j];
-      FFp[e] = acc;
+  __syncthreads();
+  const int half = l * (l + 1) / 2;
+  double* Pb = P + blk * (2 * half);
+  // lower-triangle tiles of B'B and B'G + G'B over the block's rows; the two-product jobs first
+  constexpr int NTL = NT * (NT + 1) / 2;
+  for (int job = wave; job < 2 * NTL; job += kStepWaves) {
+    const bool cross = job < NTL;
+    int i0, j0;
+    lower_tile(cross ? job : job - NTL, i0, j0);
+    const int ci = i0 + lane % 16, cj = j0 + lane % 16;
+    d4 p = {0.0, 0.0, 0.0, 0.0};
+    if (cross) {
+#pragma unroll 4
+      for (int q = 0; q < rows; q += 4) {
+        const int k = (q + lane / 16) * ldr;
+        p = __builtin_amdgcn_mfma_f64_16x16x4f64(sB[k + ci], sG[k + cj], p, 0, 0, 0);
+        p = __builtin_amdgcn_mfma_f64_16x16x4f64(sG[k + ci], sB[k + cj], p, 0, 0, 0);
+      }
+    } else {
+#pragma unroll 4
+      for (int q = 0; q < rows; q += 4) {
+        const int k = (q + lane / 16) * ldr;
+        p = __builtin_amdgcn_mfma_f64_16x16x4f64(sB[k + ci], sB[k + cj], p, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = i0 + lane / 16 + 4 * r;
+      if (i < l && cj <= i) Pb[(cross ? half : 0) + i * (i + 1) / 2 + cj] = p[r];
+    }
+  }
+}
+
+// The l x l step and B+ = Bc F + Bg Cinv, E+ = Ec F + invN Bc Cinv on kUpdRows rows per workgroup
+// (f64 MFMA tiles; the rows are loaded before the step and go to LDS after it); the last workgroup
+// makes FF+ = FFc F.  Every element is one chain of MFMAs over k, whatever the grid.
+constexpr int kUpdRows = 32;
+
+// Workgroups of the update: the row blocks and one for FF+.
+int64_t kn_update_blocks(int64_t nl) { return ceil_div(nl, kUpdRows) + 1; }
+
+template <int NP>
+__device__ __forceinline__ void kn_update_body(
+    int t, IntegratorState* st, int64_t nl, int l, double invN, double tol,
+    const double* __restrict__ P, int64_t nblk, const double* __restrict__ Bc,
+    const double* __restrict__ Bg, double* __restrict__ Bp, const double* __restrict__ Ec,
+    double* __restrict__ Ep, const double* __restrict__ FFc, double* __restrict__ FFp, int64_t blk,
+    int64_t nblocks) {
+  if (skip(st, t)) return;
+  constexpr int LD = series_ld<NP>(), NT = NP / 16, ER = kUpdRows * NP / kStepThreads;
+  static_assert(2 * kUpdRows * LD <= kStepBuf, "two row blocks fit a step buffer");
+  __shared__ double smem[4 * kStepBuf];
+  __shared__ double red[kStepWaves];
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, c = lane & 15,
+            kq = lane >> 4;
+  const bool ff = blk == nblocks - 1;
+  const int64_t r0 = blk * kUpdRows;
+  double v[3][ER];
+#pragma unroll
+  for (int u = 0; u < ER; ++u) {
+    const int e = tid + u * kStepThreads, r = e / NP, j = e % NP;
+    const bool in = !ff && r0 + r < nl && j < l;
+    const int64_t o = in ? (r0 + r) * l + j : 0;
+    v[0][u] = in ? Bc[o] : 0.0;
+    v[1][u] = in ? Bg[o] : 0.0;
+    v[2][u] = in ? Ec[o] : 0.0;
+  }
+  double res;
+  if (!kn_step_series<NP>(l, invN, P, nblk, smem, red, &res))
+    res = kn_step_ns<NP>(l, invN, P, nblk, smem, red);
+  if (blk == 0 && tid == 0) {
+    st->res = res;
+    if (!isfinite(res)) st->nan_seen = 1;
+    if (!(res >= tol)) st->converged_at = t;
+  }
+  double* sBc = smem;  // over C
+  double* sBg = smem + kUpdRows * LD;
+  const double* sC = smem + kStepBuf;
+  const double* sF = smem + 2 * kStepBuf;
+  double* sEc = smem + 3 * kStepBuf;  // over Dc
+  __syncthreads();
+  if (ff) {
+    for (int e = tid; e < NP * NP; e += kStepThreads) {
+      const int i = e / NP, j = e % NP;
+      sEc[i * LD + j] = i < l && j < l ? FFc[i * l + j] : 0.0;
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < ER; ++u) {
+      const int e = tid + u * kStepThreads, r = e / NP, j = e % NP;
+      sBc[r * LD + j] = v[0][u];
+      sBg[r * LD + j] = v[1][u];
+      sEc[r * LD + j] = v[2][u];
+    }
+  }
+  __syncthreads();
+  const int tiles = (ff ? NT : kUpdRows / 16) * NT;
+  const int64_t rows = ff ? l : (nl - r0 < kUpdRows ? nl - r0 : kUpdRows);
+  for (int job = wave; job < (ff ? tiles : 2 * tiles); job += kStepWaves) {
+    const bool eside = job < tiles;
+    const int tile = eside ? job : job - tiles, i0 = (tile / NT) * 16, j0 = (tile % NT) * 16;
+    const double* x = (eside ? sEc : sBc) + (i0 + c) * LD;  // times F
+    const double* y = (eside ? sBc : sBg) + (i0 + c) * LD;  // times Cinv
+    d4 p = {0.0, 0.0, 0.0, 0.0}, q = p;
+#pragma unroll
+    for (int k0 = 0; k0 < NP; k0 += 4) {
+      const int k = k0 + kq;
+      p = __builtin_amdgcn_mfma_f64_16x16x4f64(x[k], sF[k * LD + j0 + c], p, 0, 0, 0);
+      if (!ff) q = __builtin_amdgcn_mfma_f64_16x16x4f64(y[k], sC[k * LD + j0 + c], q, 0, 0, 0);
+    }
+    double* out = ff ? FFp : eside ? Ep : Bp;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = i0 + kq + 4 * r, j = j0 + c;
+      if (i < rows && j < l)
+        out[(ff ? i : r0 + i) * l + j] = eside ? p[r] + invN * q[r] : p[r] + q[r];
     }
   }
 }
@@ -415,18 +863,16 @@ __device__ __forceinline__ void kn_update_body(
 
 struct KnMember {
   const double* Bs;   // Nl x Nl
-  double* Pbg;        // bs_splits split-K partials of Bs * B
   double* B[2];
   double* Bg;
   double* E[2];
   double* FF[2];
-  double* P;          // block partials of the step
-  double* F;
-  double* C;          // Cinv
+  double* P;          // partials of the product's workgroups
+  double* sums;       // their sums (P itself when the update sums them)
   IntegratorState* st;
-  int64_t nl, kchunk, bs_splits, bs_blocks, nblk_s, upd_blocks;
+  int64_t nl, nblk, nsum, upd_blocks;  // nsum: partials left at `sums`
   double invN, tol;
-  int l, vec;
+  int l, rows, vec;   // rows per product workgroup; Bs takes 16-byte loads
   int t;              // the member's iteration index in this launch
 };
 
@@ -436,46 +882,32 @@ struct KnGroup {
 };
 static_assert(sizeof(KnGroup) <= 4096, "the member table fits the kernel arguments");
 
-// Bg partials of iteration t: Pbg[s] = Bs(:, K range s) * Bc(K range s, :) on the tall-skinny
-// FP64-MFMA tiles (the alpha = 1/N scaling is applied where the partials are summed).
-template <int LP>
-__global__ __launch_bounds__(256, LP == 32 ? 3 : 2) void kn_bs_group_kernel(KnGroup g) {
+// The product and the update are launched once per class of l present (NP = l rounded up to 32, 48
+// or 64).
+template <int NP>
+__global__ __launch_bounds__(kStepThreads) void kn_product_group_kernel(KnGroup g) {
   const KnMember& m = g.m[blockIdx.y];
-  const int t = m.t;
-  if (blockIdx.x >= m.bs_blocks || skip(m.st, t)) return;
-  GemmF64Args p;
-  p.M = m.nl;
-  p.N = m.l;
-  p.K = m.nl;
-  p.A = m.Bs;
-  p.lda = m.nl;
-  p.a_mcontig = false;
-  p.B = m.B[t & 1];
-  p.ldb = m.l;
-  p.splits = m.bs_splits;
-  p.kchunk = m.kchunk;
-  p.partial = m.Pbg;
-  if (m.vec)
-    tall_direct_tile<double, double, LP, true>(p, blockIdx.x);
-  else
-    tall_direct_tile<double, double, LP, false>(p, blockIdx.x);
+  if (blockIdx.x >= m.nblk) return;
+  kn_product_body<NP>(m.t, m.st, static_cast<int>(m.nl), m.l, m.rows, m.vec != 0, m.invN, m.Bs,
+                      m.B[m.t & 1], m.Bg, m.P, blockIdx.x);
 }
 
-__global__ __launch_bounds__(kStepThreads) void kn_reduce_step_group_kernel(KnGroup g) {
+__global__ __launch_bounds__(kThreads) void kn_sum_group_kernel(KnGroup g) {
   const KnMember& m = g.m[blockIdx.y];
-  const int t = m.t;
-  if (blockIdx.x >= m.nblk_s) return;
-  kn_reduce_step_body(t, m.st, m.nl, m.l, m.invN, m.tol, m.Pbg, m.bs_splits, m.B[t & 1], m.Bg,
-                      m.P, m.nblk_s, m.F, m.C, blockIdx.x);
+  const int count = m.l * (m.l + 1);
+  if (m.nsum == m.nblk || static_cast<int64_t>(blockIdx.x) * kWave >= count || skip(m.st, m.t))
+    return;
+  kn_sum_body(m.P, m.nblk, count, m.sums, blockIdx.x);
 }
 
-__global__ __launch_bounds__(kThreads) void kn_update_group_kernel(KnGroup g) {
+template <int NP>
+__global__ __launch_bounds__(kStepThreads) void kn_update_group_kernel(KnGroup g) {
   const KnMember& m = g.m[blockIdx.y];
   const int t = m.t;
   if (blockIdx.x >= m.upd_blocks) return;
   const int c = t & 1, p = c ^ 1;
-  kn_update_body(t, m.st, m.nl, m.l, m.invN, m.B[c], m.Bg, m.B[p], m.E[c], m.E[p], m.FF[c],
-                 m.FF[p], m.F, m.C, blockIdx.x, m.upd_blocks);
+  kn_update_body<NP>(t, m.st, m.nl, m.l, m.invN, m.tol, m.sums, m.nsum, m.B[c], m.Bg, m.B[p],
+                     m.E[c], m.E[p], m.FF[c], m.FF[p], blockIdx.x, m.upd_blocks);
 }
 
 // out[2i] = converged_at, out[2i + 1] = nan_seen of member i (one read-back for the group).
@@ -1038,7 +1470,6 @@ __global__ __launch_bounds__(kWyThreads) void wy_tau_kernel(int t, IntegratorSta
 __global__ void init_state_kernel(IntegratorState* st) {
   st->converged_at = INT_MAX;
   st->nan_seen = 0;
-  st->ticket = 0;
   st->res = 0.0;
   st->taug = WyConst::tau0;
   st->zeta = 1.0;
@@ -1213,6 +1644,7 @@ Layout layout(char* base, int64_t N, int l) {
   L.BsU1 = take(nll);
   const size_t pp = static_cast<size_t>(L.nblk_p) * 3 * ll;
   const size_t pt = static_cast<size_t>(L.nblk_t) * (3 * ll + 2);
+  // (a KN iteration's (ceil(nl / 16) + 1) l (l + 1) doubles of partials and their sums fit pt)
   L.P = take(pp > pt ? pp : pt);
   L.Pbg = take(static_cast<size_t>(L.splits + 1) * nll);
   L.T = take(3 * ll + 2);
@@ -1313,7 +1745,6 @@ KnMember kn_member(const GramIntegrator& g, const Layout& L) {
   KnMember m{};
   const int64_t nl = L.nl;
   m.Bs = g.Bs;
-  m.Pbg = L.Pbg;
   m.B[0] = L.B[0];
   m.B[1] = L.B[1];
   m.Bg = L.Bg[0];
@@ -1322,59 +1753,50 @@ KnMember kn_member(const GramIntegrator& g, const Layout& L) {
   m.FF[0] = L.FF[0];
   m.FF[1] = L.FF[1];
   m.P = L.P;
-  m.F = L.F;
-  m.C = L.C;
   m.st = L.st;
   m.nl = nl;
   m.l = g.l;
-  m.kchunk = ceil_div(ceil_div(nl, L.splits), 16) * 16;  // whole 16-deep K tiles per split
-  m.bs_splits = ceil_div(nl, m.kchunk);
-  m.bs_blocks = ceil_div(nl, 128) * m.bs_splits;
-  m.nblk_s = ceil_div(nl, kStepRows);
-  m.upd_blocks = grid_elems(nl * g.l);
+  m.rows = step_rows(nl);
+  m.nblk = ceil_div(nl, m.rows);
+  const bool direct = m.nblk <= kDirectPartials;
+  m.nsum = direct ? m.nblk : 1;
+  m.sums = direct ? L.P : L.P + m.nblk * g.l * (g.l + 1);
+  m.vec = (reinterpret_cast<uintptr_t>(g.Bs) % 16 == 0 && nl % 2 == 0) ? 1 : 0;
+  m.upd_blocks = kn_update_blocks(nl);
   m.invN = 1.0 / static_cast<double>(g.N);
   m.tol = g.tol;
-  m.vec = (reinterpret_cast<uintptr_t>(g.Bs) % 16 == 0 && nl % 2 == 0) ? 1 : 0;
   return m;
 }
 
-// One KN iteration of the members in `act` (member i at its iteration act.m[i].t): the split-K
-// Bs products (a launch per tile-width class present), then the reductions + l x l steps, then
-// the updates.
+// One KN iteration of the members in `act` (member i at its iteration act.m[i].t): the products (a
+// launch per class of l present), the sums of their partials, then the l x l steps and updates.
 void launch_kn_iteration(const KnGroup& act, hipStream_t st) {
-  KnGroup narrow, wide;
-  narrow.count = wide.count = 0;
-  int64_t bn = 0, bw = 0, bs = 0, bu = 0;
+  KnGroup cls[3];
+  int64_t bp[3] = {0, 0, 0}, bu[3] = {0, 0, 0}, bs = 0;
+  for (auto& c : cls) c.count = 0;
   for (int i = 0; i < act.count; ++i) {
     const KnMember& m = act.m[i];
-    if (m.l <= 32) {
-      narrow.m[narrow.count++] = m;
-      bn = std::max(bn, m.bs_blocks);
-    } else {
-      wide.m[wide.count++] = m;
-      bw = std::max(bw, m.bs_blocks);
-    }
-    bs = std::max(bs, m.nblk_s);
-    bu = std::max(bu, m.upd_blocks);
+    const int c = m.l <= 32 ? 0 : m.l <= 48 ? 1 : 2;
+    cls[c].m[cls[c].count++] = m;
+    bp[c] = std::max(bp[c], m.nblk);
+    bu[c] = std::max(bu[c], m.upd_blocks);
+    if (m.nsum != m.nblk)
+      bs = std::max<int64_t>(bs, ceil_div(static_cast<int64_t>(m.l) * (m.l + 1), kWave));
+    MCNLA_REQUIRE(m.nl < (1LL << 31), MCNLA_ERR_INVALID, "integrator grid too large");
   }
-  MCNLA_REQUIRE(bn < (1LL << 31) && bw < (1LL << 31) && bs < (1LL << 31), MCNLA_ERR_INVALID,
-                "integrator grid too large");
-  if (narrow.count) {
-    hipLaunchKernelGGL(kn_bs_group_kernel<32>, dim3(static_cast<unsigned>(bn), narrow.count),
-                       dim3(256), 0, st, narrow);
+  auto launch = [&](auto kernel, const KnGroup& g, int64_t blocks, int threads) {
+    if (g.count == 0 || blocks == 0) return;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks), g.count), dim3(threads), 0, st,
+                       g);
     MCNLA_LAUNCHED();
-  }
-  if (wide.count) {
-    hipLaunchKernelGGL(kn_bs_group_kernel<64>, dim3(static_cast<unsigned>(bw), wide.count),
-                       dim3(256), 0, st, wide);
-    MCNLA_LAUNCHED();
-  }
-  hipLaunchKernelGGL(kn_reduce_step_group_kernel, dim3(static_cast<unsigned>(bs), act.count),
-                     dim3(kStepThreads), 0, st, act);
-  MCNLA_LAUNCHED();
-  hipLaunchKernelGGL(kn_update_group_kernel, dim3(static_cast<unsigned>(bu), act.count),
-                     dim3(kThreads), 0, st, act);
-  MCNLA_LAUNCHED();
+  };
+  launch(kn_product_group_kernel<32>, cls[0], bp[0], kStepThreads);
+  launch(kn_product_group_kernel<48>, cls[1], bp[1], kStepThreads);
+  launch(kn_product_group_kernel<64>, cls[2], bp[2], kStepThreads);
+  launch(kn_sum_group_kernel, act, bs, kThreads);
+  launch(kn_update_group_kernel<32>, cls[0], bu[0], kStepThreads);
+  launch(kn_update_group_kernel<48>, cls[1], bu[1], kStepThreads);
+  launch(kn_update_group_kernel<64>, cls[2], bu[2], kStepThreads);
 }
 
 // The KN loop of a group.  `graphs` (a group of one only) records each chunk once and replays it.
