@@ -127,58 +127,58 @@ __global__ __launch_bounds__(256) void congruence_kernel(const double* __restric
 // that Y_i T_i has orthonormal columns when W_i = Y_i' Y_i.  L_0 is also written to L0 (lower
 // triangle, zeros above).  A pivot that is not above l eps of W_i's largest diagonal entry flags
 // *bad.
-__global__ __launch_bounds__(256) void cholesky_transforms_kernel(const double* __restrict__ W,
-                                                                 double* __restrict__ T,
-                                                                 double* __restrict__ L0, int l,
-                                                                 int* bad) {
+//
+// One elimination makes both: step k subtracts a_ik / d_k times row k from the rows below it, in
+// the trailing lower triangle of A (D = diag(d) in the end, L = A D^-1/2) and in X, which starts
+// as I and ends as D^1/2 L^-1.  1024 threads own an entry of every 16th column each; one barrier
+// per step, 0.5 us (12.8 us at l = 20, 25 at l = 40; factorization, division and a substitution by
+// one thread per column, three barriers a step, took 25 and 65).
+__global__ __launch_bounds__(kSyevThreads) void cholesky_transforms_kernel(
+    const double* __restrict__ W, double* __restrict__ T, double* __restrict__ L0, int l,
+    int* bad) {
   __shared__ double a[kLds];
   __shared__ double x[kLds];
+  __shared__ double rs[kMaxL];  // 1 / sqrt(d)
   const int ld = lds_ld(l);
   const int64_t b = blockIdx.x;
   const double* Wb = W + b * l * l;
   const int tid = threadIdx.x;
-  for (int e = tid; e < l * l; e += blockDim.x) {
+  for (int e = tid; e < l * l; e += kSyevThreads) {
     const int i = e / l, j = e % l;
     a[i * ld + j] = (i >= j) ? Wb[i * l + j] : 0.0;
-    x[i * ld + j] = 0.0;
+    x[i * ld + j] = i == j ? 1.0 : 0.0;
   }
   __syncthreads();
   // A pivot at or below l eps of the largest diagonal entry is zero at working precision: the
   // sketch does not have full column rank (or W holds NaN / Inf, which fails the test too).
   double wmax = 0.0;
-  for (int i = 0; i < l; ++i) wmax = fmax(wmax, Wb[i * l + i]);
+  for (int i = 0; i < l; ++i) wmax = fmax(wmax, a[i * ld + i]);
   const double floor_piv = l * 0x1p-52 * wmax;
-  bool fail = false;
-  for (int j = 0; j < l; ++j) {
-    const double d = a[j * ld + j];
-    const double piv = (d > 0.0) ? sqrt(d) : 1.0;
-    fail = fail || !(d > floor_piv);
-    __syncthreads();  // every thread has read the pivot before it is overwritten
-    if (tid == 0) a[j * ld + j] = piv;
-    for (int r = j + 1 + tid; r < l; r += blockDim.x) a[r * ld + j] /= piv;
-    __syncthreads();
-    const int w = l - 1 - j;
-    for (int e = tid; e < w * w; e += blockDim.x) {
-      const int r = j + 1 + e / w, c = j + 1 + e % w;
-      if (c <= r) a[r * ld + c] -= a[r * ld + j] * a[c * ld + j];
-    }
-    __syncthreads();
-  }
-  // X = L^{-1}: thread c solves L x = e_c by forward substitution (column c of X in LDS)
-  for (int c = tid; c < l; c += blockDim.x) {
-    x[c * ld + c] = 1.0 / a[c * ld + c];
-    for (int r = c + 1; r < l; ++r) {
-      double s = 0.0;
-      for (int q = c; q < r; ++q) s += a[r * ld + q] * x[q * ld + c];
-      x[r * ld + c] = -s / a[r * ld + r];
-    }
-  }
   __syncthreads();
+  bool fail = false;
+  const int r = tid >> 4, c0 = tid & 15;
+  for (int k = 0; k < l; ++k) {
+    const double akk = a[k * ld + k], d = (akk > 0.0) ? akk : 1.0;
+    fail = fail || !(akk > floor_piv);
+    if (tid == 0) rs[k] = 1.0 / sqrt(d);
+    if (r > k && r < l) {
+      const double f = a[r * ld + k] / d;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int c = c0 + 16 * j;
+        if (c <= k)
+          x[r * ld + c] -= f * x[k * ld + c];
+        else if (c <= r)
+          a[r * ld + c] -= f * a[c * ld + k];
+      }
+    }
+    __syncthreads();
+  }
   double* Tb = T + b * l * l;
-  for (int e = tid; e < l * l; e += blockDim.x) {
+  for (int e = tid; e < l * l; e += kSyevThreads) {
     const int i = e / l, j = e % l;
-    Tb[e] = x[j * ld + i];  // T = X'
-    if (b == 0 && L0 != nullptr) L0[e] = (i >= j) ? a[i * ld + j] : 0.0;
+    Tb[e] = i <= j ? x[j * ld + i] * rs[j] : 0.0;  // T = X'
+    if (b == 0 && L0 != nullptr) L0[e] = (i >= j) ? a[i * ld + j] * rs[j] : 0.0;
   }
   if (fail && tid == 0) atomicAdd(bad, 1);
 }
@@ -395,8 +395,8 @@ void cholesky_transforms(const double* W, int64_t N, int l, double* Tst, double*
                          hipStream_t st) {
   MCNLA_REQUIRE(l >= 1 && l <= kMaxL, MCNLA_ERR_INVALID, "l > 64");
   if (N <= 0) return;
-  hipLaunchKernelGGL(cholesky_transforms_kernel, dim3(static_cast<unsigned>(N)), dim3(256), 0, st,
-                     W, Tst, L0, l, bad);
+  hipLaunchKernelGGL(cholesky_transforms_kernel, dim3(static_cast<unsigned>(N)), dim3(kSyevThreads),
+                     0, st, W, Tst, L0, l, bad);
   MCNLA_LAUNCHED();
 }
 

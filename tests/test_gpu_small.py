@@ -46,3 +46,23 @@ def test_orthogonalizer_edges(l, m, precision):
     assert bad == 0
     sign = np.sign(np.sum(q * ref, axis=0))
     assert np.abs(q * sign - ref).max() < (1e-8 if precision == mc.PREC_F64 else 2e-7)
+
+
+@pytest.mark.parametrize("k,p,N", [(1, 0, 3), (8, 7, 3), (10, 6, 3), (10, 7, 2), (20, 11, 3),
+                                   (20, 12, 2), (20, 13, 2), (30, 17, 2), (30, 18, 2), (30, 19, 2),
+                                   (50, 13, 2), (50, 14, 3)])
+def test_solve_edges(k, p, N):
+    """The Cholesky route of a solve against the oracle's eigen transforms."""
+    m, n, l = 400, 150, k + p
+    rng = np.random.default_rng(l)
+    A = (basis(rng, m, n) * 0.9 ** np.arange(n)) @ basis(rng, n, n).T
+    om = oracle.omega_ref(3, n, N * l, col_block=True)
+    Q, _ = oracle.gramian_orthogonalize(oracle.sketch(A, om), l, N)
+    Qb, iters = oracle.kn_rowblock(Q, l, N, 256, 1e-4)
+    S, U, _ = oracle.svd_former(A, Qb, k)
+    P = mc.Parameters().setSize(m, n).setRank(k).setOverRank(p).setNumSketch(N)
+    s = mc.Solver(P, seed=3, omega_mode=mc.OMEGA_REFERENCE)
+    s.solve(mc.DeviceArray.from_numpy(np.asfortranarray(A)))
+    assert abs(s.iteration() - iters) <= 1
+    assert np.max(np.abs(s.vectorS() - S) / S) < 1e-9
+    assert np.abs(U @ U.T - s.matrixU() @ s.matrixU().T).max() < 1e-8
