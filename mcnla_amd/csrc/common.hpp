@@ -66,4 +66,21 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// The sum over a row of 16 lanes, the same in each of them, by DPP rotations (VALU moves: a shuffle
+// goes through LDS).
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_mov_dpp(static_cast<int>(b), CTRL, 0xf, 0xf, true);
+  const uint32_t hi = __builtin_amdgcn_mov_dpp(static_cast<int>(b >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, static_cast<uint64_t>(hi) << 32 | lo);
+}
+__device__ __forceinline__ double row_sum(double v) {
+  v += dpp_move<0x128>(v);  // row_ror:8, 4, 2, 1
+  v += dpp_move<0x124>(v);
+  v += dpp_move<0x122>(v);
+  v += dpp_move<0x121>(v);
+  return v;
+}
+
 }  // namespace mcnla

@@ -11,32 +11,75 @@ namespace {
 
 constexpr int kSmallThreads = 256;
 constexpr int kLds = kMaxL * (kMaxL + 1);
-// A Jacobi round applies up to (l/2)^2 + (l/2) l = 3072 work items at l = 64: 1024 threads take
-// three each (256 threads took twelve, one after another, each waiting on its LDS reads).
-constexpr int kSyevThreads = 1024;
+
+// LDS of one eigen-problem.
+struct EigLds {
+  double a[kLds];
+  double v[kLds];
+  double cs[2 * kMaxL];  // lds_jacobi's rotations; lds_psd_eig's d and nrm
+  int pq[2 * kMaxL];
+  double red[2 * (kEigThreads / kWave)];
+  int ord[kMaxL];
+};
+
+// Eigen-decomposition of the symmetric n x n matrix in sh.a (both triangles): w (descending) and
+// V as batched_syev gives them.  A matrix that is positive definite at working precision goes
+// through its Cholesky factor, any other one (the symmetric former's, a rank-deficient or
+// non-finite Gram matrix) through the two-sided Jacobi.  The matrix is first scaled by a power of
+// two to a largest diagonal entry in [1/2, 1).
+__device__ void eig_sorted(int n, bool definite, EigLds& sh, double* w, double* V) {
+  const int ld = lds_ld(n), tid = threadIdx.x;
+  double* d = sh.cs;
+  double* nrm = sh.cs + kMaxL;
+  double mx = 0.0;
+  for (int i = 0; i < n; ++i) mx = fmax(mx, sh.a[i * ld + i]);
+  int e = 0;
+  if (definite && mx > 0.0 && isfinite(mx)) {
+    (void)frexp(mx, &e);
+    __syncthreads();
+    for (int q = tid; q < n * n; q += kEigThreads) {
+      double* x = &sh.a[(q / n) * ld + q % n];
+      *x = ldexp(*x, -e);
+    }
+    __syncthreads();
+    if (lds_psd_eig(n, sh.a, sh.v, d, nrm, sh.pq)) {
+      lds_psd_eig_sorted(n, sh.v, sh.a, nrm, sh.ord, ldexp(1.0, e), w, V);
+      return;
+    }
+    __syncthreads();
+    for (int q = tid; q < n * n; q += kEigThreads) {  // the matrix again, unscaled
+      const int i = q / n, j = q % n;
+      if (i >= j) {
+        const double x = ldexp(i == j ? d[i] : sh.a[j * ld + i], e);
+        sh.a[i * ld + j] = x;
+      }
+    }
+    __syncthreads();
+    for (int q = tid; q < n * n; q += kEigThreads) {
+      const int i = q / n, j = q % n;
+      if (i < j) sh.a[i * ld + j] = sh.a[j * ld + i];
+    }
+  }
+  __syncthreads();
+  lds_jacobi(n, sh.a, sh.v, true, sh.cs, sh.pq, sh.red);
+  lds_eig_sorted(n, sh.a, sh.v, w, V, sh.ord);
+}
 
 // One workgroup per matrix: W[b] -> (w[b] descending, V[b]).
-__global__ __launch_bounds__(kSyevThreads) void batched_syev_kernel(const double* __restrict__ W,
-                                                                   double* __restrict__ w,
-                                                                   double* __restrict__ V,
-                                                                   int n) {
-  __shared__ double a[kLds];
-  __shared__ double v[kLds];
-  __shared__ double cs[2 * kMaxL];
-  __shared__ int pq[2 * kMaxL];
-  __shared__ double red[2 * (kSyevThreads / kWave)];
-  __shared__ int ord[kMaxL];
+__global__ __launch_bounds__(kEigThreads) void batched_syev_kernel(const double* __restrict__ W,
+                                                                  double* __restrict__ w,
+                                                                  double* __restrict__ V, int n) {
+  __shared__ EigLds sh;
   const int64_t b = blockIdx.x;
   const double* Wb = W + b * n * n;
   const int ld = lds_ld(n);
-  for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
+  for (int e = threadIdx.x; e < n * n; e += kEigThreads) {
     const int i = e / n, j = e % n;
     // symmetrize from the lower triangle (i >= j)
-    a[i * ld + j] = (i >= j) ? Wb[i * n + j] : Wb[j * n + i];
+    sh.a[i * ld + j] = (i >= j) ? Wb[i * n + j] : Wb[j * n + i];
   }
   __syncthreads();
-  lds_jacobi(n, a, v, true, cs, pq, red);
-  lds_eig_sorted(n, a, v, w + b * n, V + b * n * n, ord);
+  eig_sorted(n, true, sh, w + b * n, V + b * n * n);
 }
 
 // T_i = V_i diag(1/sqrt(w_i)) into rows [i*l, (i+1)*l) of the Nl x l stack.
@@ -133,7 +176,7 @@ __global__ __launch_bounds__(256) void congruence_kernel(const double* __restric
 // as I and ends as D^1/2 L^-1.  1024 threads own an entry of every 16th column each; one barrier
 // per step, 0.5 us (12.8 us at l = 20, 25 at l = 40; factorization, division and a substitution by
 // one thread per column, three barriers a step, took 25 and 65).
-__global__ __launch_bounds__(kSyevThreads) void cholesky_transforms_kernel(
+__global__ __launch_bounds__(kEigThreads) void cholesky_transforms_kernel(
     const double* __restrict__ W, double* __restrict__ T, double* __restrict__ L0, int l,
     int* bad) {
   __shared__ double a[kLds];
@@ -143,7 +186,7 @@ __global__ __launch_bounds__(kSyevThreads) void cholesky_transforms_kernel(
   const int64_t b = blockIdx.x;
   const double* Wb = W + b * l * l;
   const int tid = threadIdx.x;
-  for (int e = tid; e < l * l; e += kSyevThreads) {
+  for (int e = tid; e < l * l; e += kEigThreads) {
     const int i = e / l, j = e % l;
     a[i * ld + j] = (i >= j) ? Wb[i * l + j] : 0.0;
     x[i * ld + j] = i == j ? 1.0 : 0.0;
@@ -175,7 +218,7 @@ __global__ __launch_bounds__(kSyevThreads) void cholesky_transforms_kernel(
     __syncthreads();
   }
   double* Tb = T + b * l * l;
-  for (int e = tid; e < l * l; e += kSyevThreads) {
+  for (int e = tid; e < l * l; e += kEigThreads) {
     const int i = e / l, j = e % l;
     Tb[e] = i <= j ? x[j * ld + i] * rs[j] : 0.0;  // T = X'
     if (b == 0 && L0 != nullptr) L0[e] = (i >= j) ? a[i * ld + j] * rs[j] : 0.0;
@@ -266,29 +309,21 @@ __global__ __launch_bounds__(256) void apply_blockdiag_kernel(T* __restrict__ Y,
 // Former: eig of Wg (l x l) -> eigw (descending), eigv; Wk = eigv[:, :k]; S = sqrt(eigw[:k]).
 // symmetric (Wg = Qbar' A Qbar of a symmetric A): the k largest eigenpairs in ascending order,
 // S = the eigenvalues themselves (row_block_symmetric_former.hpp:65-66,127-130).
-// One l x l problem on one workgroup: 16 waves share each Jacobi round's work.
-constexpr int kFormerThreads = 1024;
-
-__global__ __launch_bounds__(kFormerThreads) void former_small_kernel(const double* __restrict__ Wg,
-                                                                    int l, int k, bool symmetric,
-                                                                    double* __restrict__ eigw,
-                                                                    double* __restrict__ eigv,
-                                                                    double* __restrict__ Wk,
-                                                                    double* __restrict__ S) {
-  __shared__ double a[kLds];
-  __shared__ double v[kLds];
-  __shared__ double cs[2 * kMaxL];
-  __shared__ int pq[2 * kMaxL];
-  __shared__ double red[2 * (kFormerThreads / kWave)];
-  __shared__ int ord[kMaxL];
+// One l x l problem on one workgroup.
+__global__ __launch_bounds__(kEigThreads) void former_small_kernel(const double* __restrict__ Wg,
+                                                                  int l, int k, bool symmetric,
+                                                                  double* __restrict__ eigw,
+                                                                  double* __restrict__ eigv,
+                                                                  double* __restrict__ Wk,
+                                                                  double* __restrict__ S) {
+  __shared__ EigLds sh;
   const int ld = lds_ld(l);
-  for (int e = threadIdx.x; e < l * l; e += blockDim.x) {
+  for (int e = threadIdx.x; e < l * l; e += kEigThreads) {
     const int i = e / l, j = e % l;
-    a[i * ld + j] = 0.5 * (Wg[i * l + j] + Wg[j * l + i]);
+    sh.a[i * ld + j] = 0.5 * (Wg[i * l + j] + Wg[j * l + i]);
   }
   __syncthreads();
-  lds_jacobi(l, a, v, true, cs, pq, red);
-  lds_eig_sorted(l, a, v, eigw, eigv, ord);
+  eig_sorted(l, !symmetric, sh, eigw, eigv);
   for (int e = threadIdx.x; e < l * k; e += blockDim.x) {
     const int i = e / k, j = e % k;
     Wk[e] = eigv[i * l + (symmetric ? k - 1 - j : j)];
@@ -339,7 +374,7 @@ unsigned grid_for(int64_t total, int threads = 256, int64_t cap = 16384) {
 void batched_syev(const double* W, double* w, double* V, int64_t batch, int n, hipStream_t st) {
   MCNLA_REQUIRE(n >= 1 && n <= kMaxL, MCNLA_ERR_INVALID, "eigen problem larger than 64");
   if (batch <= 0) return;
-  hipLaunchKernelGGL(batched_syev_kernel, dim3(static_cast<unsigned>(batch)), dim3(kSyevThreads),
+  hipLaunchKernelGGL(batched_syev_kernel, dim3(static_cast<unsigned>(batch)), dim3(kEigThreads),
                      0, st, W, w, V, n);
   MCNLA_LAUNCHED();
 }
@@ -395,7 +430,7 @@ void cholesky_transforms(const double* W, int64_t N, int l, double* Tst, double*
                          hipStream_t st) {
   MCNLA_REQUIRE(l >= 1 && l <= kMaxL, MCNLA_ERR_INVALID, "l > 64");
   if (N <= 0) return;
-  hipLaunchKernelGGL(cholesky_transforms_kernel, dim3(static_cast<unsigned>(N)), dim3(kSyevThreads),
+  hipLaunchKernelGGL(cholesky_transforms_kernel, dim3(static_cast<unsigned>(N)), dim3(kEigThreads),
                      0, st, W, Tst, L0, l, bad);
   MCNLA_LAUNCHED();
 }
@@ -423,7 +458,7 @@ void apply_blockdiag(void* Y, bool y_f32, int64_t m, int64_t N, int l, const dou
 void former_small(const double* Wg, int l, int k, double* eigw, double* eigv, double* Wk,
                   double* S, hipStream_t st, bool symmetric) {
   MCNLA_REQUIRE(l >= 1 && l <= kMaxL && k >= 1 && k <= l, MCNLA_ERR_INVALID, "former sizes");
-  hipLaunchKernelGGL(former_small_kernel, dim3(1), dim3(kFormerThreads), 0, st, Wg, l, k, symmetric,
+  hipLaunchKernelGGL(former_small_kernel, dim3(1), dim3(kEigThreads), 0, st, Wg, l, k, symmetric,
                      eigw, eigv, Wk, S);
   MCNLA_LAUNCHED();
 }

@@ -6,6 +6,8 @@
 
 namespace mcnla {
 
+__host__ __device__ constexpr int pad16(int n) { return (n + 15) & ~15; }
+
 // Leading dimension used for an n x n matrix kept in LDS (odd stride avoids bank conflicts on
 // column walks).
 __host__ __device__ constexpr int lds_ld(int n) { return n + 1; }
@@ -132,6 +134,200 @@ __device__ inline int lds_jacobi(int n, double* a, double* v, bool init_v, doubl
   return sweeps;
 }
 
+constexpr int kEigThreads = 1024;
+constexpr int kEigStride = 65;
+
+// One-sided Jacobi on the n columns of u (16 R rows, those past n zero): rotations from the right
+// until every pair has |u_p . u_q| <= 1e-15 |u_p| |u_q|.  16 lanes hold a pair, R rows each, four
+// pairs to a wave, so that a round -- two columns read, their inner product by DPP adds, the
+// rotation, two columns written, one barrier -- is one pass at every n, on 8 waves at most: what
+// bounds it is the length of that chain (0.3 us; lds_jacobi's two passes over two matrices take
+// 1 to 1.5 us, and a wave per pair, which repeats the rotation's arithmetic four times as often,
+// 0.65 to 1).  nrm: 64 doubles, flags: 2 ints of LDS.
+template <int R>
+__device__ inline void lds_one_sided(int n, double* u, double* nrm, int* flags) {
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const int g = tid >> 4, row = tid & 15;  // 64 groups of 16 lanes
+  const int np = (n + 1) & ~1, npairs = np / 2;
+  for (int sweep = 0; sweep < 30; ++sweep) {
+    if (tid == 0) flags[0] = flags[1] = 0;
+    if (g < n) {
+      double s = 0.0;
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        const double x = u[g * kEigStride + row + 16 * j];
+        s += x * x;
+      }
+      s = row_sum(s);
+      if (row == 0) nrm[g] = s;
+    }
+    __syncthreads();
+    for (int round = 0; round < np - 1; ++round) {
+      int x = g == 0 ? 0 : g + round, y = np - 1 - g + round;
+      if (x >= np) x -= np - 1;
+      if (y >= np) y -= np - 1;
+      const int p = x < y ? x : y, q = x < y ? y : x;
+      if (g < npairs && q < n) {  // q = n: the bye of an odd n
+        double* cp = u + p * kEigStride + row;
+        double* cq = u + q * kEigStride + row;
+        double up[R], uq[R], apq = 0.0;
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          up[j] = cp[16 * j];
+          uq[j] = cq[16 * j];
+          apq += up[j] * uq[j];
+        }
+        const double app = nrm[p], aqq = nrm[q];
+        apq = row_sum(apq);
+        if (apq * apq > 1e-30 * (app * aqq)) {
+          // theta = (aqq - app) / (2 apq), t its smaller root.  t may be off by the 2^-24 of the
+          // hardware's reciprocals (that much of a_pq is left); c^2 + s^2 = 1 may not.
+          const double dd = aqq - app, h = 2.0 * apq;
+          const double ri = __builtin_amdgcn_rsq(fma(dd, dd, h * h));
+          double t = fabs(h) * ri * __builtin_amdgcn_rcp(fma(fabs(dd), ri, 1.0));
+          if ((dd < 0.0) != (apq < 0.0)) t = -t;
+          const double w = fma(t, t, 1.0), y0 = __builtin_amdgcn_rsq(w);
+          const double e = fma(-w * y0, y0, 1.0);
+          const double c = fma(y0 * e, fma(0.375, e, 0.5), y0), s = t * c;
+#pragma unroll
+          for (int j = 0; j < R; ++j) {
+            cp[16 * j] = c * up[j] - s * uq[j];
+            cq[16 * j] = s * up[j] + c * uq[j];
+          }
+          if (row == 0) {
+            nrm[p] = app - t * apq;
+            nrm[q] = aqq + t * apq;
+            flags[0] = 1;
+          }
+        }
+      }
+      __syncthreads();
+    }
+    if (!flags[0]) return;
+    bool again = sweep < 3;
+    if (!again) {
+      // would the next sweep rotate any pair?  All inner products at once on f64 MFMA tiles
+      const int tiles = R * (R + 1) / 2;
+      if (wave < tiles) {
+        int ti = 0;
+        while ((ti + 1) * (ti + 2) / 2 <= wave) ++ti;
+        const int i0 = ti * 16, j0 = (wave - ti * (ti + 1) / 2) * 16, cc = lane & 15,
+                  kq = lane >> 4;
+        const int ci = i0 + cc < n ? i0 + cc : n - 1, cj = j0 + cc < n ? j0 + cc : n - 1;
+        d4 f = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 16 * R; k += 4)
+          f = __builtin_amdgcn_mfma_f64_16x16x4f64(u[ci * kEigStride + k + kq],
+                                                   u[cj * kEigStride + k + kq], f, 0, 0, 0);
+        bool more = false;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = i0 + kq + 4 * r, j = j0 + cc;
+          if (i < n && j < i) more = more || f[r] * f[r] > 1e-30 * (nrm[i] * nrm[j]);
+        }
+        if (more) flags[1] = 1;
+      }
+      __syncthreads();
+      again = flags[1] != 0;
+    }
+    __syncthreads();  // flags are reset, nrm is renewed
+    if (!again) return;
+  }
+}
+
+// Eigen-decomposition of a positive definite n x n matrix (n <= 64) by one-sided Jacobi on its
+// Cholesky factor (Veselic & Hari, Numer. Math. 56, 1989): A = L L', and rotations from the right
+// that make the columns of L orthogonal leave them as the eigenvectors times the square roots of
+// the eigenvalues -- to lds_jacobi's threshold, in the same tournament.
+// a: the matrix (LDS, ld = n + 1, both triangles; diagonal at most 1); its lower triangle and
+// diagonal are overwritten.  u: 64 columns of 65 doubles of LDS, the result.  d, nrm: 64 doubles,
+// flags: 2 ints of LDS.  Every thread of the workgroup of 1024 must call this.  Returns false
+// (uniformly) when a pivot is not above n 2^-50 times the largest diagonal entry; `a` then has its
+// upper triangle intact and the diagonal is in d.
+__device__ inline bool lds_psd_eig(int n, double* a, double* u, double* d, double* nrm,
+                                   int* flags) {
+  const int ld = lds_ld(n), tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  constexpr int NW = kEigThreads / kWave;
+  if (tid < n) d[tid] = a[tid * ld + tid];
+  __syncthreads();
+  double floor_piv = 0.0;
+  for (int i = 0; i < n; ++i) floor_piv = fmax(floor_piv, d[i]);
+  floor_piv *= n * 0x1p-50;
+  // LDL': column k stays unscaled below its pivot
+  const int r = tid >> 4, c0 = tid & 15;
+  for (int k = 0; k < n; ++k) {
+    const double dk = a[k * ld + k];
+    if (!(dk > floor_piv)) return false;  // also for a NaN
+    if (r > k && r < n) {
+      const double f = a[r * ld + k] / dk;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int c = c0 + 16 * j;
+        if (c > k && c <= r) a[r * ld + c] -= f * a[c * ld + k];
+      }
+    }
+    __syncthreads();
+  }
+  for (int c = wave; c < n; c += NW) {
+    const double s = rsqrt(a[c * ld + c]);
+    u[c * kEigStride + lane] = (lane >= c && lane < n) ? a[lane * ld + c] * s : 0.0;
+  }
+  __syncthreads();
+  if (n <= 16) lds_one_sided<1>(n, u, nrm, flags);
+  else if (n <= 32) lds_one_sided<2>(n, u, nrm, flags);
+  else if (n <= 48) lds_one_sided<3>(n, u, nrm, flags);
+  else lds_one_sided<4>(n, u, nrm, flags);
+  __syncthreads();
+  return true;
+}
+
+// The eigenpairs lds_psd_eig left in u, in DESCENDING order and each with its largest-magnitude
+// entry positive (the first of equal ones): w (n, times `scale`) and vout (global, row-major n x n,
+// vectors in columns).  a: n (n + 1) doubles, nrm: 64 doubles, ord: 64 ints of LDS.
+__device__ inline void lds_psd_eig_sorted(int n, const double* u, double* a, double* nrm, int* ord,
+                                          double scale, double* w, double* vout) {
+  const int ld = lds_ld(n), tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  constexpr int NW = kEigThreads / kWave;
+  if ((tid >> 4) < n) {
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const double x = u[(tid >> 4) * kEigStride + (tid & 15) + 16 * j];
+      s += x * x;
+    }
+    s = row_sum(s);
+    if ((tid & 15) == 0) nrm[tid >> 4] = s;
+  }
+  __syncthreads();
+  if (tid < n) {
+    const double di = nrm[tid];
+    int rank = 0;
+    for (int j = 0; j < n; ++j) rank += (nrm[j] > di || (nrm[j] == di && j < tid)) ? 1 : 0;
+    ord[rank] = tid;
+  }
+  __syncthreads();
+  for (int j = wave; j < n; j += NW) {
+    const int src = ord[j];
+    const double x = u[src * kEigStride + lane];
+    double key = lane < n ? fabs(x) : -1.0;
+    int at = lane;
+    for (int off = 32; off > 0; off >>= 1) {
+      const double ok = __shfl_xor(key, off, kWave);
+      const int oi = __shfl_xor(at, off, kWave);
+      if (ok > key || (ok == key && oi < at)) {
+        key = ok;
+        at = oi;
+      }
+    }
+    const double sg = __shfl(x, at, kWave) < 0.0 ? -1.0 : 1.0;
+    if (lane < n) a[lane * ld + j] = sg * rsqrt(nrm[src]) * x;
+    if (lane == 0) w[j] = nrm[src] * scale;
+  }
+  __syncthreads();
+  for (int e = tid; e < n * n; e += kEigThreads) vout[e] = a[(e / n) * ld + e % n];
+  __syncthreads();
+}
+
 // c = a' * b for n x n LDS matrices (ld = n+1); c must not alias a or b.
 __device__ inline void lds_matmul_tn(int n, const double* a, const double* b, double* c) {
   const int ld = lds_ld(n);
@@ -158,8 +354,6 @@ __device__ inline void lds_matmul_nn(int n, const double* a, const double* b, do
 // np x np matrices (np a multiple of 16, at most 64) kept row-major in LDS with leading dimension
 // ld.  Matrices of order l < np are embedded as diag(X, I) so that products, square roots and
 // inverses leave the padding block equal to the identity.
-
-__host__ __device__ constexpr int pad16(int n) { return (n + 15) & ~15; }
 
 // One 16 x 16 tile of op(A) op(B) on v_mfma_f64_16x16x4f64 (the whole wave must call it).  Slot r
 // of lane L holds element (i0 + L/16 + 4r, j0 + L%16) of the product.

@@ -48,6 +48,26 @@ def test_orthogonalizer_edges(l, m, precision):
     assert np.abs(q * sign - ref).max() < (1e-8 if precision == mc.PREC_F64 else 2e-7)
 
 
+@pytest.mark.parametrize("l", EDGES)
+@pytest.mark.parametrize("decades", [6, 8])
+def test_former_edges(l, decades):
+    """Singular values 1 .. 10^-decades: sigma_j = ||Z w_j|| with w_j from the Gram matrix, whose
+    rounding tilts w_j towards the larger ones by about eps / sigma_j.  At 1e-6 the pivots pass; LAPACK's
+    eigensolver leaves 6.4e-10 there at l = 64, six times that is allowed.  At 1e-8 the smallest
+    eigenvalues drown in rounding and the pivots fail: only the leading half (1e-4) is compared."""
+    rng = np.random.default_rng(l)
+    m, n = 300, 200
+    W, s = graded(rng, n, l, decades)
+    Q = basis(rng, m, l)
+    f = mc.SvdFormer(params(m, n, l, 1), True)
+    f(mc.DeviceArray.from_numpy(np.asfortranarray(Q @ W.T)), mc.DeviceArray.from_numpy(Q))
+    S, U = f.vectorS(), f.matrixU()
+    keep = l if decades == 6 else (l + 1) // 2
+    err = np.abs(S - s) / s
+    assert np.max(err[:keep]) < (4e-9 if decades == 6 else 2e-8)
+    assert np.abs(U.T @ U - np.eye(l)).max() < 1e-12
+
+
 @pytest.mark.parametrize("k,p,N", [(1, 0, 3), (8, 7, 3), (10, 6, 3), (10, 7, 2), (20, 11, 3),
                                    (20, 12, 2), (20, 13, 2), (30, 17, 2), (30, 18, 2), (30, 19, 2),
                                    (50, 13, 2), (50, 14, 3)])
