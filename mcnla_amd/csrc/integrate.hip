@@ -4,7 +4,7 @@
 // every iteration works on Nl x l and l x l matrices that stay in L2 (the reference's Gramian
 // forms, row_block_gramian_kolmogorov_nagumo_integrator.hpp:106-226 and
 // row_block_gramian_wen_yin_integrator.hpp:114-328).  The basis is carried as coefficients:
-// Qc = Q0 F~ + Qs E~, so Qbar = Qs * M with M = E~ + [F~; 0].
+// Qc = Q0 F~ + Qs E~, so Qbar = Qs * M with M = E~ + [F~; 0] (KN keeps that sum itself, in E).
 //
 // Every iteration t is a fixed sequence of kernels gated by st->converged_at: a kernel of
 // iteration t does nothing once convergence was detected at an earlier iteration, so the host can
@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 #include <vector>
 
 namespace mcnla {
@@ -166,14 +167,11 @@ struct SeriesTable {
 };
 __constant__ const SeriesTable kSeries;
 // rho up to which degree 4b - 1 suffices, b = 2, 3, ... (the tail sum a_k rho^k, k >= 4b, of Cinv
-// is 1.5e-17 there).
+// is 1.5e-17 there); 0 beyond the last, and for a NaN.
 __device__ __forceinline__ int series_blocks(double rho) {
-  constexpr double limit[kSeriesMaxB - 1] = {0.01435, 0.06178, 0.12669, 0.19394, 0.25695,
-                                             0.31369, 0.36401, 0.40845, 0.44771};
-  int b = 2;
-  for (; b <= kSeriesMaxB; ++b)
-    if (rho <= limit[b - 2]) return b;
-  return 0;  // also for a NaN
+  const int b = 2 + (rho > 0.01435) + (rho > 0.06178) + (rho > 0.12669) + (rho > 0.19394) +
+                (rho > 0.25695) + (rho > 0.31369) + (rho > 0.36401) + (rho > 0.40845);
+  return rho <= 0.44771 ? b : 0;
 }
 
 constexpr int kStepThreads = 512;
@@ -221,12 +219,13 @@ __device__ __forceinline__ void lower_tile(int q, int& i0, int& j0) {
 }
 
 // All forms of the step run on kStepThreads threads (the whole workgroup) with four buffers of
-// kStepBuf doubles in smem, and leave Cinv in the second and F in the third (leading dimension
-// series_ld<NP>(); F is zero past l).  They return ||C - I||_F (NaN or infinite when Z is not).
+// kStepBuf doubles in smem, and leave C in the first and Cinv in the second (leading dimension
+// series_ld<NP>(); past l they are not used).  They return ||C - I||_F (NaN or infinite when Z is
+// not).
 
 // The eigen-decomposition form.
 template <int NP>
-__device__ double kn_step_eigen(int l, double invN, const double* __restrict__ P, int64_t nblk,
+__device__ __forceinline__ double kn_step_eigen(int l, double invN, const double* __restrict__ P, int64_t nblk,
                                 double* smem) {
   __shared__ double s[kMaxL];
   __shared__ double cs[2 * kMaxL];
@@ -255,36 +254,26 @@ __device__ double kn_step_eigen(int l, double invN, const double* __restrict__ P
   for (int i = threadIdx.x; i < l; i += kStepThreads)
     s[i] = sqrt(0.5 + sqrt(0.25 - z[i * ld + i]));
   __syncthreads();
-  for (int e = threadIdx.x; e < ll; e += kStepThreads) {  // Cinv into `a`
-    const int i = e / l, j = e % l;
-    double ci = 0.0;
-    for (int q = 0; q < l; ++q) ci += v[i * ld + q] * v[j * ld + q] / s[q];
-    a[i * ld + j] = ci;
-  }
-  __syncthreads();
-  double f[EP], ci[EP];  // F = C - Dc Cinv, C on the fly
+  double ce[EP], ci[EP];
 #pragma unroll
   for (int u = 0; u < EP; ++u) {
     const int e = threadIdx.x + u * kStepThreads, i = e / NP, j = e % NP;
-    f[u] = 0.0;
+    ce[u] = 0.0;
     ci[u] = 0.0;
-    if (i < l && j < l) {
-      double c = 0.0, dci = 0.0;
+    if (i < l && j < l)
       for (int q = 0; q < l; ++q) {
-        c += v[i * ld + q] * v[j * ld + q] * s[q];
-        dci += dc[i * ld + q] * a[q * ld + j];
+        const double vv = v[i * ld + q] * v[j * ld + q];
+        ce[u] += vv * s[q];
+        ci[u] += vv / s[q];
       }
-      f[u] = c - dci;
-      ci[u] = a[i * ld + j];
-    }
   }
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < EP; ++u) {
     const int e = threadIdx.x + u * kStepThreads, i = e / NP, j = e % NP;
     if (i >= NP) break;
+    smem[i * LD + j] = ce[u];
     smem[kStepBuf + i * LD + j] = ci[u];
-    smem[2 * kStepBuf + i * LD + j] = f[u];
   }
   __syncthreads();
   double r = 0.0;
@@ -294,7 +283,7 @@ __device__ double kn_step_eigen(int l, double invN, const double* __restrict__ P
 
 // The Newton-Schulz form: X = (I - 4Z)^{1/2}, C = ((I + X)/2)^{1/2}, Cinv = C^{-1}.
 template <int NP>
-__device__ double kn_step_ns(int l, double invN, const double* __restrict__ P, int64_t nblk,
+__device__ __forceinline__ double kn_step_ns(int l, double invN, const double* __restrict__ P, int64_t nblk,
                              double* smem, double* red) {
   constexpr int LD = series_ld<NP>(), NT1 = NP / 16;
   double* sY = smem;
@@ -336,19 +325,12 @@ __device__ double kn_step_ns(int l, double invN, const double* __restrict__ P, i
     __syncthreads();
     return kn_step_eigen<NP>(l, invN, P, nblk, smem);
   }
-  // C = sY, Cinv = sW; F = C - Dc Cinv; ||C - I||_F (the padding of C is the identity)
+  // C = sY, Cinv = sW; ||C - I||_F (the padding of C is the identity)
   double rs = 0.0;
-  for (int tile = wave; tile < NT1 * NT1; tile += kStepWaves) {
-    const int i0 = (tile / NT1) * 16, j0 = (tile % NT1) * 16;
-    const d4 acc = lds_mfma_tile<false, false>(NP, LD, sDc, sW, i0, j0);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = i0 + (lane >> 4) + 4 * r, j = j0 + (lane & 15);
-      const double c = sY[i * LD + j];
-      sT[i * LD + j] = i < l && j < l ? c - acc[r] : 0.0;
-      const double d = c - ((i == j) ? 1.0 : 0.0);
-      rs += d * d;
-    }
+  for (int e = tid; e < NP * NP; e += kStepThreads) {
+    const int i = e / NP, j = e % NP;
+    const double d = sY[i * LD + j] - ((i == j) ? 1.0 : 0.0);
+    rs += d * d;
   }
   rs = wave_sum(rs);
   __syncthreads();  // red is reused
@@ -359,245 +341,94 @@ __device__ double kn_step_ns(int l, double invN, const double* __restrict__ P, i
   return sqrt(tot);
 }
 
-// Returns false (uniformly, with nothing written) when x is too large for the series.  Waves own
-// lower-triangle tiles of the results: all matrices are symmetric polynomials of Z (and Dc), so
-// only those tiles are computed, six MFMA chains of NP / 4 where the square-root iterations take
-// eighteen; every barrier is one of about 5 + 2b.
-template <int NP>
-__device__ bool kn_step_series(int l, double invN, const double* __restrict__ P, int64_t nblk,
-                               double* smem, double* red, double* res) {
-  constexpr int LD = series_ld<NP>(), NT1 = NP / 16, NTL = NT1 * (NT1 + 1) / 2;
-  constexpr int Q1 = (NTL + kStepWaves - 1) / kStepWaves;      // tiles per wave
-  constexpr int Q2 = (2 * NTL + kStepWaves - 1) / kStepWaves;  // tiles of C and Cinv per wave
-  double* bX = smem;                  // x, then the polynomial of C
-  double* bX2 = smem + kStepBuf;      // x^2, then the polynomial of Cinv
-  double* bX4 = smem + 2 * kStepBuf;  // Dgc, then x^4
-  double* bDc = smem + 3 * kStepBuf;
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid & (kWave - 1);
-  const int half = l * (l + 1) / 2;
-  const d4 zero = {0.0, 0.0, 0.0, 0.0};
-  // Dc into bDc, Dgc into bX4: job q < NTL is the tile q of Dc, the rest those of Dgc; the loads of
-  // all of a wave's jobs and of four partials are in flight together
-  {
-    d4 sum[Q2];
-    int off[Q2][4];
-    bool in[Q2][4];
-#pragma unroll
-    for (int q = 0; q < Q2; ++q) {
-      const int job = wave + q * kStepWaves;
-      int i0, j0;
-      lower_tile(job < NTL ? job : job - NTL, i0, j0);
-      sum[q] = zero;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = i0 + (lane >> 4) + 4 * r, j = j0 + (lane & 15);
-        in[q][r] = job < 2 * NTL && i < l && j < l;
-        off[q][r] = in[q][r] ? (job < NTL ? 0 : half) + tri(i, j) : 0;
-      }
-    }
-    constexpr int UB = Q2 == 1 ? 16 : Q2 == 2 ? 8 : 4;
-    for (int64_t b = 0; b < nblk; b += UB) {
-      double v[UB][Q2][4];
-#pragma unroll
-      for (int u = 0; u < UB; ++u) {
-        const double* Pb = P + (b + u < nblk ? b + u : b) * 2 * half;
-#pragma unroll
-        for (int q = 0; q < Q2; ++q)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[u][q][r] = Pb[off[q][r]];
-      }
-#pragma unroll
-      for (int u = 0; u < UB; ++u)
-        if (b + u < nblk) {
-#pragma unroll
-          for (int q = 0; q < Q2; ++q)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sum[q][r] += v[u][q][r];
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < Q2; ++q) {
-      const int job = wave + q * kStepWaves;
-      if (job >= 2 * NTL) continue;
-      int i0, j0;
-      lower_tile(job < NTL ? job : job - NTL, i0, j0);
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        sum[q][r] = in[q][r] ? (job < NTL ? invN : 0.5 * invN) * sum[q][r] : 0.0;
-      put_sym<NP>(job < NTL ? bDc : bX4, i0, j0, sum[q]);
-    }
-  }
-  __syncthreads();
-  // x = 4 (Dgc - Dc^2) and rho^2 = ||x||_F^2
-  double ss = 0.0;
-#pragma unroll
-  for (int q = 0; q < Q1; ++q) {
-    const int tile = wave + q * kStepWaves;
-    if (tile >= NTL) continue;
-    int i0, j0;
-    lower_tile(tile, i0, j0);
-    const d4 d = sym_tile<NP>(bDc, bDc, i0, j0, zero);
-    d4 x;
-    double s4 = 0.0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      x[r] = 4.0 * (bX4[(i0 + (lane >> 4) + 4 * r) * LD + j0 + (lane & 15)] - d[r]);
-      s4 += x[r] * x[r];
-    }
-    ss += i0 != j0 ? 2.0 * s4 : s4;
-    put_sym<NP>(bX, i0, j0, x);
-  }
-  ss = wave_sum(ss);
-  if (lane == 0) red[wave] = ss;
-  __syncthreads();
-  double rho2 = 0.0;
-#pragma unroll
-  for (int w = 0; w < kStepWaves; ++w) rho2 += red[w];
-  const int nb = series_blocks(sqrt(rho2));
-  if (nb == 0) {
-    __syncthreads();  // the buffers are reused
-    return false;
-  }
-#pragma unroll
-  for (int q = 0; q < Q1; ++q) {  // x^2
-    const int tile = wave + q * kStepWaves;
-    if (tile >= NTL) continue;
-    int i0, j0;
-    lower_tile(tile, i0, j0);
-    put_sym<NP>(bX2, i0, j0, sym_tile<NP>(bX, bX, i0, j0, zero));
-  }
-  __syncthreads();
-  // x^4 into LDS; every owner of a tile of C (jobs 0 .. NTL - 1) or Cinv (the rest) keeps the
-  // tile of x, x^2 and x^3
-  d4 x1[Q2], x2[Q2], x3[Q2];
-#pragma unroll
-  for (int q = 0; q < Q2; ++q) {
-    const int job = wave + q * kStepWaves;
-    if (job >= 2 * NTL) continue;
-    int i0, j0;
-    lower_tile(job < NTL ? job : job - NTL, i0, j0);
-    if (job < NTL) put_sym<NP>(bX4, i0, j0, sym_tile<NP>(bX2, bX2, i0, j0, zero));
-    x3[q] = sym_tile<NP>(bX, bX2, i0, j0, zero);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = i0 + (lane >> 4) + 4 * r, j = j0 + (lane & 15);
-      x1[q][r] = bX[i * LD + j];
-      x2[q][r] = bX2[i * LD + j];
-    }
-  }
-  __syncthreads();
-  for (int b = nb - 1; b >= 0; --b) {  // P := P x^4 + a_4b I + ... + a_4b+3 x^3
-    d4 acc[Q2];
-#pragma unroll
-    for (int q = 0; q < Q2; ++q) {
-      const int job = wave + q * kStepWaves;
-      if (job >= 2 * NTL) continue;
-      const bool inv = job >= NTL;
-      int i0, j0;
-      lower_tile(inv ? job - NTL : job, i0, j0);
-      const double* a = (inv ? kSeries.ci : kSeries.c) + 4 * b;
-      const double a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = i0 + (lane >> 4) + 4 * r, j = j0 + (lane & 15);
-        acc[q][r] = fma(a3, x3[q][r], fma(a2, x2[q][r], fma(a1, x1[q][r], i == j ? a0 : 0.0)));
-      }
-      if (b != nb - 1) acc[q] = sym_tile<NP>(inv ? bX2 : bX, bX4, i0, j0, acc[q]);
-    }
-    if (b != nb - 1) __syncthreads();
-#pragma unroll
-    for (int q = 0; q < Q2; ++q) {
-      const int job = wave + q * kStepWaves;
-      if (job >= 2 * NTL) continue;
-      int i0, j0;
-      lower_tile(job < NTL ? job : job - NTL, i0, j0);
-      put_sym<NP>(job < NTL ? bX : bX2, i0, j0, acc[q]);
-    }
-    __syncthreads();
-  }
-  // F = C - Dc Cinv over x^4, ||C - I||_F
-  double rs = 0.0;
-  for (int tile = wave; tile < NT1 * NT1; tile += kStepWaves) {
-    const int i0 = (tile / NT1) * 16, j0 = (tile % NT1) * 16;
-    const d4 acc = sym_tile<NP>(bDc, bX2, i0, j0, zero);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = i0 + (lane >> 4) + 4 * r, j = j0 + (lane & 15);
-      const double c = bX[i * LD + j];
-      bX4[i * LD + j] = i < l && j < l ? c - acc[r] : 0.0;
-      const double d = c - ((i == j) ? 1.0 : 0.0);
-      rs += d * d;  // the padding of C is the identity
-    }
-  }
-  rs = wave_sum(rs);
-  if (lane == 0) red[wave] = rs;
-  __syncthreads();
-  double tot = 0.0;
-  for (int w = 0; w < kStepWaves; ++w) tot += red[w];
-  *res = sqrt(tot);
-  return true;
-}
+// The lower-triangle job of slot q of a wave: tiles are dealt to the waves round robin.
+__device__ __forceinline__ int slot_job(int q) { return threadIdx.x / kWave + q * kStepWaves; }
 
 // A KN iteration is two or three launches:
-//   1. product: workgroup b owns rows [R b, R b + R) of the Nl x l matrices and forms Bg = Bs Bc / N
-//      on them: its 8 waves take an eighth of K each, both operands straight from L2 into MFMA
-//      registers, and sum their tiles through LDS in wave order; then its partial
-//      [Bc'Bc, Bc'Bg + Bg'Bc] -> P[b] (f64 MFMA, lower triangles);
-//   2. from nine workgroups on, kn_sum sums the partials element by element, in block order;
+//   1. product: a workgroup owns rows [R b, R b + R) of the Nl x l matrices, and all or a part of
+//      their columns, and forms Bg = Bs Bc / N there: its 8 waves take every eighth 16 of K, both
+//      operands straight from L2 into MFMA registers, and sum their tiles through LDS in wave
+//      order; then its partial of Bc'Bc and Bc'Bg -> P[b] (f64 MFMA);
+//   2. from nine row blocks on, kn_sum sums the partials element by element, in block order;
 //   3. update: every workgroup runs the l x l step for itself and updates its rows of B and E.
-// All sums are in a fixed order.  Repeating the step (6 us at l = 32, 17 us at l = 64) in every
+// All sums are in a fixed order.  Repeating the step (5 us at l = 32, 13 us at l = 64) in every
 // workgroup costs no time; doing it once, in the last workgroup of the product to finish, cost a
 // ticket and a device-scope fence (4 us, twice with two levels of partials), one CU summing all
 // partials (45 GB/s: 8 us at Nl = 2048 and l = 32, 25 us at Nl = 8192 and l = 64) and F and Cinv
 // through memory.
 
-// Rows per workgroup of the product: 16, so that the chip fills, while that makes at most 256
-// workgroups, then 32 (twice the use of each line of Bc).
-int step_rows(int64_t nl) { return nl <= 4096 ? 16 : 32; }
-
 // Partials that the update sums itself.
 constexpr int64_t kDirectPartials = 8;
 
-// sums[e] = sum_b P[b][e]: 64 elements per workgroup, a quarter of the blocks per wave.
-__device__ __forceinline__ void kn_sum_body(const double* __restrict__ P, int64_t nblk, int count,
-                                            double* __restrict__ sums, int64_t blk) {
-  __shared__ double part[kThreads];
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int64_t e = blk * kWave + lane;
-  const int64_t per = (nblk + 3) / 4, b0 = wave * per < nblk ? wave * per : nblk;
-  const int64_t n = b0 + per < nblk ? per : nblk - b0;
-  part[threadIdx.x] = e < count ? sum_partials(P + b0 * count, n, count, e) : 0.0;
-  __syncthreads();
-  if (wave == 0 && e < count)
-    sums[e] = ((part[lane] + part[64 + lane]) + part[128 + lane]) + part[192 + lane];
+// Rows per workgroup of the product and of the update: 16, so that the chip fills, while that makes
+// at most 256 workgroups, then 32 (in the product, twice the use of each line of Bc).
+int step_rows(int64_t nl) { return nl <= 4096 ? 16 : 32; }
+
+// Parts the columns of a product's row block are cut into.  Below 256 row blocks of 16 the product
+// is bound by the matrix cores of the few CUs that have one, so the blocks are cut while the parts
+// keep to one per CU and to whole 16-wide tiles: Nl = 740, l = 37 (47 blocks) 13.5 -> 8.0 us, Nl =
+// 1920, l = 60 28.9 -> 22.3, Nl = 2048, l = 32 21.2 -> 19.4 (one product after another).  Up to
+// kDirectPartials blocks the update reads the partials itself, uncut.
+int step_parts(int64_t nblk, int l) {
+  if (nblk <= kDirectPartials || l <= 16) return 1;
+  if (l <= 32) return nblk <= 128 ? 2 : 1;
+  if (l <= 48) return nblk <= 85 ? 3 : 1;
+  return nblk <= 64 ? 4 : nblk <= 128 ? 2 : 1;
 }
 
-// The tile of Bs Bc of one wave: RB rows from r0 by NP columns over k in [k0, k1), in stages of
-// 16 k.  In a stage, lane group kq takes k = 4 kq .. 4 kq + 3 (the
-// same in both operands), so that a lane's four entries of Bs are 32 contiguous bytes and a row's
-// 16 are one line (VEC: 16-byte loads; Bs 16-byte aligned and nl even).  Columns past l and rows
-// past nl repeat valid ones (their results are not used); k past k1 enters as zero.
-template <int NP, int RB, bool VEC>
+// sums = the sum over the blocks of the partials: 64 elements per workgroup, a quarter of the blocks
+// per wave.  A partial of a product in parts holds Bc'Bg's two triangles side by side (each with
+// the diagonal), which are added here.
+__device__ __forceinline__ void kn_sum_body(const double* __restrict__ P, int64_t nblk, int half,
+                                            bool parts, double* __restrict__ sums, int64_t blk) {
+  __shared__ double part[2][kThreads];
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int64_t e = blk * kWave + lane, count = (parts ? 3 : 2) * half;
+  const int64_t per = (nblk + 3) / 4, b0 = wave * per < nblk ? wave * per : nblk;
+  const int64_t n = b0 + per < nblk ? per : nblk - b0;
+  const bool both = parts && e >= half && e < 2 * half;
+  double x = 0.0, y = 0.0;
+  if (e < 2 * half) sum_partials2(P + b0 * count, n, count, e, both ? e + half : -1, x, y);
+  part[0][threadIdx.x] = x;
+  part[1][threadIdx.x] = y;
+  __syncthreads();
+  if (wave == 0 && e < 2 * half) {
+    x = ((part[0][lane] + part[0][64 + lane]) + part[0][128 + lane]) + part[0][192 + lane];
+    y = ((part[1][lane] + part[1][64 + lane]) + part[1][128 + lane]) + part[1][192 + lane];
+    sums[e] = x + y;
+  }
+}
+
+// The tile of Bs Bc of one wave: RB rows from r0 by the NTW 16-wide column tiles from ct0, over the
+// 16-wide stages `wave`, wave + 8, ... of K, so that the workgroup walks 1 KB of every row at a
+// time.  In a stage, lane group kq takes k = 4 kq .. 4 kq + 3 (the same in both operands), so that
+// a lane's four entries of Bs are 32 contiguous bytes and a row's 16 are one line (VEC: 16-byte
+// loads; Bs 16-byte aligned and nl even).  Columns past l and rows past nl repeat valid ones (their
+// results are not used); k past nl enters as zero.  At Nl = 8192 and l = 64 it is bound by Bs from
+// HBM and the matrix cores together: 162 us, of which 120 are either's at its measured rate.
+template <int NTW, int RB, bool VEC>
 __device__ __forceinline__ void kn_product(const double* __restrict__ Bs,
                                            const double* __restrict__ B, int nl, int l, int r0,
-                                           int k0, int k1, d4 (&acc)[RB / 16][NP / 16]) {
-  constexpr int NT = NP / 16, RT = RB / 16;
+                                           int ct0, d4 (&acc)[RB / 16][NTW]) {
+  constexpr int RT = RB / 16;
   const int lane = threadIdx.x & (kWave - 1), c = lane & 15, kq = lane >> 4;
+  const int wave = threadIdx.x / kWave;
   const double* row[RT];
 #pragma unroll
   for (int i = 0; i < RT; ++i) {
     const int r = r0 + 16 * i + c;
     row[i] = Bs + static_cast<int64_t>(r < nl ? r : nl - 1) * nl;
   }
-  int col[NT];
+  int col[NTW];
 #pragma unroll
-  for (int j = 0; j < NT; ++j) col[j] = j * 16 + c < l ? j * 16 + c : l - 1;
-  // D stages of 16 k in registers: a stage's loads are issued D - 1 stages ahead (past the last
-  // whole stage they repeat it), with no branch in the loop that would make the compiler wait
-  constexpr int D = RT * NT <= 3 ? 4 : 3;
-  double a[D][RT][4], b[D][4][NT];
-  auto load = [&](int k, double (&x)[RT][4], double (&y)[4][NT]) {
-    const int kk = k + 4 * kq;
+  for (int j = 0; j < NTW; ++j) col[j] = (ct0 + j) * 16 + c < l ? (ct0 + j) * 16 + c : l - 1;
+  // D stages in registers: a stage's loads are issued D - 1 stages ahead (in the loop, past the
+  // last whole stage they repeat it), with no branch there that would make the compiler wait.  At
+  // 32 rows by 64 columns a third stage spills (190 us where two take 162).
+  constexpr int D = RT * NTW == 1 ? 8 : RT * NTW == 2 ? 5 : RT * NTW <= 3 ? 4 : RT * NTW <= 6 ? 3 : 2;
+  double a[D][RT][4], b[D][4][NTW];
+  auto load = [&](int s, double (&x)[RT][4], double (&y)[4][NTW]) {
+    const int kk = 16 * (wave + kStepWaves * s) + 4 * kq;
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
       if constexpr (VEC) {
@@ -615,27 +446,29 @@ __device__ __forceinline__ void kn_product(const double* __restrict__ Bs,
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int j = 0; j < NT; ++j) y[u][j] = B[static_cast<int64_t>(kk + u) * l + col[j]];
+      for (int j = 0; j < NTW; ++j) y[u][j] = B[static_cast<unsigned>((kk + u) * l + col[j])];
   };
-  auto mul = [&](const double (&x)[RT][4], const double (&y)[4][NT]) {
+  auto mul = [&](const double (&x)[RT][4], const double (&y)[4][NTW]) {
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
       for (int i = 0; i < RT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+        for (int j = 0; j < NTW; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i][u], y[u][j], acc[i][j], 0, 0, 0);
   };
-  const int n = (k1 - k0) / 16;  // whole stages
+  const int whole = nl / 16;
+  const int n = whole > wave ? (whole - wave + kStepWaves - 1) / kStepWaves : 0;
   if (n > 0) {
 #pragma unroll
-    for (int s = 0; s < D - 1; ++s) load(k0 + 16 * (s < n ? s : n - 1), a[s], b[s]);
+    for (int s = 0; s < D - 1; ++s)
+      if (s < n) load(s, a[s], b[s]);
     int s0 = 0;
     for (; s0 + D <= n; s0 += D) {
 #pragma unroll
       for (int s = 0; s < D; ++s) {
         const int ahead = s0 + s + D - 1;
-        load(k0 + 16 * (ahead < n ? ahead : n - 1), a[(s + D - 1) % D], b[(s + D - 1) % D]);
+        load(ahead < n ? ahead : n - 1, a[(s + D - 1) % D], b[(s + D - 1) % D]);
         mul(a[s], b[s]);
       }
     }
@@ -643,211 +476,477 @@ __device__ __forceinline__ void kn_product(const double* __restrict__ Bs,
     for (int s = 0; s < D - 1; ++s)
       if (s0 + s < n) mul(a[s], b[s]);
   }
-  if (k0 + 16 * n < k1) {  // the last, partial stage
-    const int kk = k0 + 16 * n + 4 * kq;
+  if (nl % 16 != 0 && whole % kStepWaves == wave) {  // the last, partial stage
+    const int kk = 16 * whole + 4 * kq;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const bool in = kk + u < k1;
-      const int kc = in ? kk + u : k0;
+      const bool in = kk + u < nl;
+      const int kc = in ? kk + u : 0;
 #pragma unroll
       for (int i = 0; i < RT; ++i) a[0][i][u] = in ? row[i][kc] : 0.0;
 #pragma unroll
-      for (int j = 0; j < NT; ++j) b[0][u][j] = B[static_cast<int64_t>(kc) * l + col[j]];
+      for (int j = 0; j < NTW; ++j) b[0][u][j] = B[static_cast<int64_t>(kc) * l + col[j]];
     }
     mul(a[0], b[0]);
   }
 }
 
-// A wave's product tile, written to LDS (leading dimension NP + 2).
-template <int NP, int RB>
+// A wave's product tile, written to LDS (leading dimension 16 NTW + 2).
+template <int NTW, int RB>
 __device__ __forceinline__ void kn_product_tile(const double* __restrict__ Bs,
                                                 const double* __restrict__ B, int nl, int l,
-                                                bool vec, int r0, int k0, int k1, double* out) {
-  constexpr int NT = NP / 16, RT = RB / 16;
+                                                bool vec, int r0, int ct0, double* out) {
+  constexpr int RT = RB / 16;
   const int lane = threadIdx.x & (kWave - 1);
-  d4 acc[RT][NT];
+  d4 acc[RT][NTW];
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+    for (int j = 0; j < NTW; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
   if (vec)
-    kn_product<NP, RB, true>(Bs, B, nl, l, r0, k0, k1, acc);
+    kn_product<NTW, RB, true>(Bs, B, nl, l, r0, ct0, acc);
   else
-    kn_product<NP, RB, false>(Bs, B, nl, l, r0, k0, k1, acc);
+    kn_product<NTW, RB, false>(Bs, B, nl, l, r0, ct0, acc);
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+    for (int j = 0; j < NTW; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        out[(16 * i + (lane >> 4) + 4 * r) * (NP + 2) + 16 * j + (lane & 15)] = acc[i][j][r];
+        out[(16 * i + (lane >> 4) + 4 * r) * (16 * NTW + 2) + 16 * j + (lane & 15)] = acc[i][j][r];
 }
 
-// Workgroup `blk` of the product (kStepThreads threads), `rows` (16 or 32) rows each; l <= NP.
-template <int NP>
-__device__ __forceinline__ void kn_product_body(int t, const IntegratorState* st, int nl, int l,
-                                                int rows, bool vec, double invN,
+// Row block `blk` of the product (kStepThreads threads), `rows` (16 or 32) rows, the NTW column
+// tiles from ct0; l <= NP.  NTW = NP / 16 is the whole row block.  smem: product_lds<NP, rows>()
+// doubles.
+template <int NP, int rows>
+__host__ __device__ constexpr int product_lds() {
+  return kStepWaves * rows * (NP + 2);
+}
+
+template <int NP, int rows, int NTW>
+__device__ __forceinline__ void kn_product_body(int nl, int l, bool vec, double invN,
                                                 const double* __restrict__ Bs,
                                                 const double* __restrict__ B,
                                                 double* __restrict__ Bg, double* __restrict__ P,
-                                                int64_t blk) {
-  if (skip(st, t)) return;
-  constexpr int NT = NP / 16, LT = NP + 2;
-  __shared__ double smem[kStepWaves * 32 * LT];
+                                                int64_t blk, int ct0, double* smem) {
+  constexpr int NT = NP / 16, W = 16 * NTW, LT = W + 2;
+  constexpr bool whole = NTW == NT;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   const int r0 = static_cast<int>(blk) * rows;
-  const int per = (nl + 16 * kStepWaves - 1) / (16 * kStepWaves) * 16;  // k per wave
-  const int k0 = wave * per < nl ? wave * per : nl, k1 = k0 + per < nl ? k0 + per : nl;
   const int tile = rows * LT;
-  if (rows == 16)
-    kn_product_tile<NP, 16>(Bs, B, nl, l, vec, r0, k0, k1, smem + wave * tile);
-  else
-    kn_product_tile<NP, 32>(Bs, B, nl, l, vec, r0, k0, k1, smem + wave * tile);
-  __syncthreads();
-  // the rows of Bg (summed in wave order, written out) and of B, then side by side in LDS
-  constexpr int EP = 32 * NP / kStepThreads;  // elements per thread, at most
-  double gv[EP], bv[EP];
+  kn_product_tile<NTW, rows>(Bs, B, nl, l, vec, r0, ct0, smem + wave * tile);
+  // the rows of B and, summed in wave order and written out, of Bg, then side by side in LDS
+  constexpr int EB = (rows * NP + kStepThreads - 1) / kStepThreads;  // elements per thread
+  constexpr int EG = (rows * W + kStepThreads - 1) / kStepThreads;
+  double gv[EG], bv[EB];
 #pragma unroll
-  for (int u = 0; u < EP; ++u) {
+  for (int u = 0; u < EB; ++u) {
     const int e = tid + u * kStepThreads, rr = e / NP, j = e % NP;
     const bool in = rr < rows && r0 + rr < nl && j < l;
-    const int64_t o = static_cast<int64_t>(r0 + rr) * l + j;
-    bv[u] = in ? B[o] : 0.0;
+    bv[u] = in ? B[static_cast<int64_t>(r0 + rr) * l + j] : 0.0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < EG; ++u) {
+    const int e = tid + u * kStepThreads, rr = e / W, j = 16 * ct0 + e % W;
+    const bool in = rr < rows && r0 + rr < nl && j < l;
     double g = 0.0;
     if (rr < rows) {
 #pragma unroll
-      for (int w = 0; w < kStepWaves; ++w) g += smem[w * tile + rr * LT + j];
+      for (int w = 0; w < kStepWaves; ++w) g += smem[w * tile + rr * LT + e % W];
     }
     gv[u] = in ? invN * g : 0.0;
-    if (in) Bg[o] = gv[u];
+    if (in) Bg[static_cast<int64_t>(r0 + rr) * l + j] = gv[u];
   }
   __syncthreads();
   constexpr int ldr = NP + 16;  // rows k, k + 1 half the banks apart
   double* sB = smem;
-  double* sG = smem + 32 * ldr;
+  double* sG = smem + rows * ldr;
 #pragma unroll
-  for (int u = 0; u < EP; ++u) {
+  for (int u = 0; u < EB; ++u) {
     const int e = tid + u * kStepThreads, rr = e / NP, j = e % NP;
-    if (rr >= rows) break;
-    sB[rr * ldr + j] = bv[u];
-    sG[rr * ldr + j] = gv[u];
+    if (rr < rows) sB[rr * ldr + j] = bv[u];
+  }
+#pragma unroll
+  for (int u = 0; u < EG; ++u) {
+    const int e = tid + u * kStepThreads, rr = e / W;
+    if (rr < rows) sG[rr * ldr + 16 * ct0 + e % W] = gv[u];
   }
   __syncthreads();
   const int half = l * (l + 1) / 2;
-  double* Pb = P + blk * (2 * half);
-  // lower-triangle tiles of B'B and B'G + G'B over the block's rows; the two-product jobs first
-  constexpr int NTL = NT * (NT + 1) / 2;
-  for (int job = wave; job < 2 * NTL; job += kStepWaves) {
-    const bool cross = job < NTL;
-    int i0, j0;
-    lower_tile(cross ? job : job - NTL, i0, j0);
-    const int ci = i0 + lane % 16, cj = j0 + lane % 16;
-    d4 p = {0.0, 0.0, 0.0, 0.0};
-    if (cross) {
-#pragma unroll 4
-      for (int q = 0; q < rows; q += 4) {
-        const int k = (q + lane / 16) * ldr;
-        p = __builtin_amdgcn_mfma_f64_16x16x4f64(sB[k + ci], sG[k + cj], p, 0, 0, 0);
-        p = __builtin_amdgcn_mfma_f64_16x16x4f64(sG[k + ci], sB[k + cj], p, 0, 0, 0);
+  if constexpr (whole) {
+    // lower-triangle tiles of B'B and B'G + G'B over the block's rows; the two-product jobs first
+    double* Pb = P + blk * (2 * half);
+    constexpr int NTL = NT * (NT + 1) / 2;
+    for (int job = wave; job < 2 * NTL; job += kStepWaves) {
+      const bool cross = job < NTL;
+      int i0, j0;
+      lower_tile(cross ? job : job - NTL, i0, j0);
+      const int ci = i0 + lane % 16, cj = j0 + lane % 16;
+      d4 p = {0.0, 0.0, 0.0, 0.0};
+      if (cross) {
+#pragma unroll
+        for (int q = 0; q < rows; q += 4) {
+          const int k = (q + lane / 16) * ldr;
+          p = __builtin_amdgcn_mfma_f64_16x16x4f64(sB[k + ci], sG[k + cj], p, 0, 0, 0);
+          p = __builtin_amdgcn_mfma_f64_16x16x4f64(sG[k + ci], sB[k + cj], p, 0, 0, 0);
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < rows; q += 4) {
+          const int k = (q + lane / 16) * ldr;
+          p = __builtin_amdgcn_mfma_f64_16x16x4f64(sB[k + ci], sB[k + cj], p, 0, 0, 0);
+        }
       }
-    } else {
-#pragma unroll 4
-      for (int q = 0; q < rows; q += 4) {
-        const int k = (q + lane / 16) * ldr;
-        p = __builtin_amdgcn_mfma_f64_16x16x4f64(sB[k + ci], sB[k + cj], p, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = i0 + lane / 16 + 4 * r;
+        if (i < l && cj <= i) Pb[(cross ? half : 0) + i * (i + 1) / 2 + cj] = p[r];
       }
     }
+  } else {
+    // its columns of B'G, both triangles, and of the lower triangle of B'B
+    double* Pb = P + blk * (3 * half);
+    for (int job = wave; job < 2 * NT * NTW; job += kStepWaves) {
+      const bool cross = job < NT * NTW;
+      const int q0 = cross ? job : job - NT * NTW, i0 = (q0 % NT) * 16, j0 = (ct0 + q0 / NT) * 16;
+      if (!cross && i0 < j0) continue;
+      const double* right = cross ? sG : sB;
+      const int ci = i0 + lane % 16, cj = j0 + lane % 16;
+      d4 p = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = i0 + lane / 16 + 4 * r;
-      if (i < l && cj <= i) Pb[(cross ? half : 0) + i * (i + 1) / 2 + cj] = p[r];
+      for (int q = 0; q < 16; q += 4) {
+        const int k = (q + lane / 16) * ldr;
+        p = __builtin_amdgcn_mfma_f64_16x16x4f64(sB[k + ci], right[k + cj], p, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = i0 + lane / 16 + 4 * r;
+        if (i >= l || cj >= l) continue;
+        if (cj <= i) Pb[(cross ? half : 0) + i * (i + 1) / 2 + cj] = p[r];
+        if (cross && cj >= i) Pb[2 * half + cj * (cj + 1) / 2 + i] = p[r];
+      }
     }
   }
 }
 
-// The l x l step and B+ = Bc F + Bg Cinv, E+ = Ec F + invN Bc Cinv on kUpdRows rows per workgroup
-// (f64 MFMA tiles; the rows are loaded before the step and go to LDS after it); the last workgroup
-// makes FF+ = FFc F.  Every element is one chain of MFMAs over k, whatever the grid.
-constexpr int kUpdRows = 32;
-
-// Workgroups of the update: the row blocks and one for FF+.
-int64_t kn_update_blocks(int64_t nl) { return ceil_div(nl, kUpdRows) + 1; }
-
-template <int NP>
+// The l x l step and B+ = Bc F + Bg Cinv, E+ = Ec F + invN Bc Cinv, F = C - Dc Cinv, on R rows per
+// workgroup, as B+ = Bc C + (Bg - Bc Dc) Cinv and likewise for E: the products with Dc do not wait
+// for the polynomials, and F, another l x l product and barrier for everyone, is not formed.
+// E0 = [I; 0] makes E the coefficients of the integrated basis by itself.
+//
+// The series form of the step.  All matrices are symmetric polynomials of Z (and Dc), so only
+// lower-triangle tiles are computed, tile slot_job(q) by the wave that keeps x, x^2 and x^3 there
+// (Dgc too, which no one else needs).  What bounds it is a chain of stages, each NP / 4 MFMAs of
+// 64 cycles per tile of the fullest SIMD and 0.3 us of LDS reads, writes and a barrier, after 1.8
+// us for the first loads: 12 us inside the kernel at l = 37 and Nl = 740 (18.5 with F formed, x^3
+// twice, 32 rows a workgroup and the partials' loads repeated to a fixed number), 9.6 at l = 20 (11.7),
+// 20 at l = 60 (26.5).
+// Every element is one chain of MFMAs over k, whatever the grid.
+template <int NP, int R>
 __device__ __forceinline__ void kn_update_body(
     int t, IntegratorState* st, int64_t nl, int l, double invN, double tol,
     const double* __restrict__ P, int64_t nblk, const double* __restrict__ Bc,
     const double* __restrict__ Bg, double* __restrict__ Bp, const double* __restrict__ Ec,
-    double* __restrict__ Ep, const double* __restrict__ FFc, double* __restrict__ FFp, int64_t blk,
-    int64_t nblocks) {
-  if (skip(st, t)) return;
-  constexpr int LD = series_ld<NP>(), NT = NP / 16, ER = kUpdRows * NP / kStepThreads;
-  static_assert(2 * kUpdRows * LD <= kStepBuf, "two row blocks fit a step buffer");
-  __shared__ double smem[4 * kStepBuf];
-  __shared__ double red[kStepWaves];
+    double* __restrict__ Ep, int64_t blk, double* smem, double* red, double (*coef)[4 * kSeriesMaxB]) {
+  constexpr int LD = series_ld<NP>(), NT = NP / 16, NTL = NT * (NT + 1) / 2, RT = R / 16;
+  constexpr int ER = (R * NP + kStepThreads - 1) / kStepThreads;  // row elements per thread
+  constexpr int Q1 = (NTL + kStepWaves - 1) / kStepWaves;         // tiles per wave
+  constexpr int JU = 2 * RT * NT;  // tiles of Bc Dc, then those of Ec Dc; of B+, E+
+  constexpr int QU = (NTL + JU + kStepWaves - 1) / kStepWaves;
+  static_assert(2 * R * LD <= kStepBuf, "two row blocks fit a step buffer");
+  double* bX = smem;                  // x, then the polynomial of C
+  double* bX2 = smem + kStepBuf;      // rows of Bc and Ec, x^2, then the polynomial of Cinv
+  double* bX4 = smem + 2 * kStepBuf;  // x^4, then rows of Bg - Bc Dc and invN Bc - Ec Dc
+  double* bDc = smem + 3 * kStepBuf;  // Dc, then rows of Bc and Ec
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, c = lane & 15,
             kq = lane >> 4;
-  const bool ff = blk == nblocks - 1;
-  const int64_t r0 = blk * kUpdRows;
-  double v[3][ER];
+  const int half = l * (l + 1) / 2;
+  const int64_t r0 = blk * R;
+  const int rows = nl - r0 < R ? static_cast<int>(nl - r0) : R;
+  Bc += r0 * l;
+  Bg += r0 * l;
+  Ec += r0 * l;
+  Bp += r0 * l;
+  Ep += r0 * l;
+  const d4 zero = {0.0, 0.0, 0.0, 0.0};
+  // everything this workgroup reads, in flight together: the tiles of Dc and Dgc, the rows of Bc
+  // and Ec, and the tiles of Bg
+  d4 dc[Q1], g[Q1], uv[QU];
+  double v[2][ER];
+  auto load = [&] {
+    unsigned off[Q1][4];
+    bool in[Q1][4];
 #pragma unroll
-  for (int u = 0; u < ER; ++u) {
-    const int e = tid + u * kStepThreads, r = e / NP, j = e % NP;
-    const bool in = !ff && r0 + r < nl && j < l;
-    const int64_t o = in ? (r0 + r) * l + j : 0;
-    v[0][u] = in ? Bc[o] : 0.0;
-    v[1][u] = in ? Bg[o] : 0.0;
-    v[2][u] = in ? Ec[o] : 0.0;
+    for (int q = 0; q < Q1; ++q) {
+      const int job = slot_job(q);
+      int i0, j0;
+      lower_tile(job < NTL ? job : 0, i0, j0);
+      dc[q] = zero;
+      g[q] = zero;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = i0 + kq + 4 * r, j = j0 + c;
+        in[q][r] = job < NTL && i < l && j < l;
+        off[q][r] = in[q][r] ? tri(i, j) : 0;
+      }
+    }
+    constexpr int UB = NP == 32 ? 6 : 4 / Q1;  // one, or some of a product's without kn_sum
+    for (int64_t b = 0; b < nblk; b += UB) {
+      double x[UB][Q1][4], y[UB][Q1][4];
+#pragma unroll
+      for (int u = 0; u < UB; ++u)
+        if (b + u < nblk) {
+          const double* Pb = P + (b + u) * 2 * half;
+#pragma unroll
+          for (int q = 0; q < Q1; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              x[u][q][r] = Pb[off[q][r]];
+              y[u][q][r] = Pb[off[q][r] + half];
+            }
+        }
+#pragma unroll
+      for (int u = 0; u < UB; ++u)
+        if (b + u < nblk) {
+#pragma unroll
+          for (int q = 0; q < Q1; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              dc[q][r] += x[u][q][r];
+              g[q][r] += y[u][q][r];
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < Q1; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        dc[q][r] = in[q][r] ? invN * dc[q][r] : 0.0;
+        g[q][r] = in[q][r] ? 0.5 * invN * g[q][r] : 0.0;
+      }
+#pragma unroll
+    for (int u = 0; u < ER; ++u) {
+      const int e = tid + u * kStepThreads, r = e / NP, j = e % NP;
+      const bool use = r < rows && j < l;
+      const unsigned o = use ? r * l + j : 0;
+      v[0][u] = use ? Bc[o] : 0.0;
+      v[1][u] = use ? Ec[o] : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < QU; ++q) {
+      const int job = slot_job(q) - NTL;
+      uv[q] = zero;
+      if (job >= 0 && job < JU / 2) {
+        const int i0 = job / NT * 16, j = job % NT * 16 + c;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = i0 + kq + 4 * r;
+          const bool use = i < rows && j < l;
+          uv[q][r] = use ? Bg[static_cast<unsigned>(i * l + j)] : 0.0;
+        }
+      }
+    }
+  };
+  auto put_dc = [&] {
+#pragma unroll
+    for (int q = 0; q < Q1; ++q) {
+      const int job = slot_job(q);
+      int i0, j0;
+      lower_tile(job < NTL ? job : 0, i0, j0);
+      if (job < NTL) put_sym<NP>(bDc, i0, j0, dc[q]);
+    }
+  };
+  auto put_rows = [&](double* buf) {
+#pragma unroll
+    for (int u = 0; u < ER; ++u) {
+      const int e = tid + u * kStepThreads, r = e / NP, j = e % NP;
+      if (r < R) {
+        buf[r * LD + j] = v[0][u];
+        buf[(R + r) * LD + j] = v[1][u];
+      }
+    }
+  };
+  // Bg - Bc Dc and invN Bc - Ec Dc from the rows in buf
+  auto take_dc = [&](int q, const double* buf) {
+    const int u = slot_job(q) - NTL;
+    if (u < 0 || u >= JU) return;
+    const int side = u / (RT * NT), i0 = u % (RT * NT) / NT * 16, j0 = u % NT * 16;
+    const double* a = buf + (side * R + i0 + c) * LD;
+    d4 d = zero;
+#pragma unroll
+    for (int k = 0; k < NP; k += 4)
+      d = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k + kq], bDc[(k + kq) * LD + j0 + c], d, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const double w = side == 0 ? uv[q][r] : invN * buf[(i0 + kq + 4 * r) * LD + j0 + c];
+      uv[q][r] = w - d[r];
+    }
+  };
+  auto put_uv = [&](double* buf) {
+#pragma unroll
+    for (int q = 0; q < QU; ++q) {
+      const int job = slot_job(q) - NTL;
+      if (job < 0 || job >= JU) continue;
+      const int i0 = job / NT * 16, j = job % NT * 16 + c;  // the second side's rows follow
+#pragma unroll
+      for (int r = 0; r < 4; ++r) buf[(i0 + kq + 4 * r) * LD + j] = uv[q][r];
+    }
+  };
+  load();
+  if (tid < 4 * kSeriesMaxB) {
+    coef[0][tid] = kSeries.c[tid];
+    coef[1][tid] = kSeries.ci[tid];
   }
-  double res;
-  if (!kn_step_series<NP>(l, invN, P, nblk, smem, red, &res))
+  put_dc();
+  put_rows(bX2);
+  __syncthreads();
+  // x = 4 (Dgc - Dc^2) and rho^2 = ||x||_F^2
+  d4 x1[Q1], x2[Q1], x3[Q1];
+  double ss = 0.0;
+#pragma unroll
+  for (int q = 0; q < Q1; ++q) {
+    const int job = slot_job(q);
+    if (job >= NTL) continue;
+    int i0, j0;
+    lower_tile(job, i0, j0);
+    const d4 d = sym_tile<NP>(bDc, bDc, i0, j0, zero);
+    double s4 = 0.0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      x1[q][r] = 4.0 * (g[q][r] - d[r]);
+      s4 += x1[q][r] * x1[q][r];
+    }
+    ss += i0 != j0 ? 2.0 * s4 : s4;
+    put_sym<NP>(bX, i0, j0, x1[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < QU; ++q) take_dc(q, bX2);
+  ss = wave_sum(ss);
+  if (lane == 0) red[wave] = ss;
+  __syncthreads();
+  double rho2 = 0.0;
+#pragma unroll
+  for (int w = 0; w < kStepWaves; ++w) rho2 += red[w];
+  const int nb = series_blocks(sqrt(rho2));
+  double res = 0.0;
+  if (nb == 0) {
+    __syncthreads();  // the buffers are reused
     res = kn_step_ns<NP>(l, invN, P, nblk, smem, red);
+    load();  // not kept in registers over the square-root iterations, which need them all
+    __syncthreads();
+    put_dc();
+    put_rows(bX4);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < QU; ++q) take_dc(q, bX4);
+    __syncthreads();
+    put_rows(bDc);
+    put_uv(bX4);
+  } else {
+    put_rows(bDc);
+#pragma unroll
+    for (int q = 0; q < Q1; ++q) {  // x^2
+      const int job = slot_job(q);
+      if (job >= NTL) continue;
+      int i0, j0;
+      lower_tile(job, i0, j0);
+      x2[q] = sym_tile<NP>(bX, bX, i0, j0, zero);
+      put_sym<NP>(bX2, i0, j0, x2[q]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < (2 * NTL + kStepWaves - 1) / kStepWaves; ++q) {  // x^3, then x^4 into LDS
+      const int job = slot_job(q);
+      int i0, j0;
+      if (job < NTL) {
+        lower_tile(job, i0, j0);
+        x3[q < Q1 ? q : 0] = sym_tile<NP>(bX, bX2, i0, j0, zero);
+      } else if (job < 2 * NTL) {
+        lower_tile(job - NTL, i0, j0);
+        put_sym<NP>(bX4, i0, j0, sym_tile<NP>(bX2, bX2, i0, j0, zero));
+      }
+    }
+    __syncthreads();
+    for (int b = nb - 1; b >= 0; --b) {  // P := P x^4 + a_4b I + ... + a_4b+3 x^3
+      d4 acc[2][Q1];
+#pragma unroll
+      for (int q = 0; q < Q1; ++q) {
+        const int job = slot_job(q);
+        if (job >= NTL) continue;
+        int i0, j0;
+        lower_tile(job, i0, j0);
+#pragma unroll
+        for (int inv = 0; inv < 2; ++inv) {
+          const double* a = coef[inv] + 4 * b;
+          const double a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int i = i0 + kq + 4 * r, j = j0 + c;
+            acc[inv][q][r] =
+                fma(a3, x3[q][r], fma(a2, x2[q][r], fma(a1, x1[q][r], i == j ? a0 : 0.0)));
+          }
+        }
+        if (b != nb - 1) {
+          acc[0][q] = sym_tile<NP>(bX, bX4, i0, j0, acc[0][q]);
+          acc[1][q] = sym_tile<NP>(bX2, bX4, i0, j0, acc[1][q]);
+        }
+      }
+      if (b != nb - 1) __syncthreads();
+      double rs = 0.0;
+#pragma unroll
+      for (int q = 0; q < Q1; ++q) {
+        const int job = slot_job(q);
+        if (job >= NTL) continue;
+        int i0, j0;
+        lower_tile(job, i0, j0);
+        put_sym<NP>(bX, i0, j0, acc[0][q]);
+        put_sym<NP>(bX2, i0, j0, acc[1][q]);
+        double s4 = 0.0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const double d = acc[0][q][r] - (i0 + kq + 4 * r == j0 + c ? 1.0 : 0.0);
+          s4 += d * d;  // the padding of C is the identity
+        }
+        rs += i0 != j0 ? 2.0 * s4 : s4;
+      }
+      if (b == 0) {
+        put_uv(bX4);
+        if (blk == 0) {  // ||C - I||_F
+          rs = wave_sum(rs);
+          if (lane == 0) red[wave] = rs;
+        }
+      }
+      __syncthreads();
+    }
+    if (blk == 0) {
+      for (int w = 0; w < kStepWaves; ++w) res += red[w];
+      res = sqrt(res);
+    }
+  }
   if (blk == 0 && tid == 0) {
     st->res = res;
     if (!isfinite(res)) st->nan_seen = 1;
     if (!(res >= tol)) st->converged_at = t;
   }
-  double* sBc = smem;  // over C
-  double* sBg = smem + kUpdRows * LD;
-  const double* sC = smem + kStepBuf;
-  const double* sF = smem + 2 * kStepBuf;
-  double* sEc = smem + 3 * kStepBuf;  // over Dc
-  __syncthreads();
-  if (ff) {
-    for (int e = tid; e < NP * NP; e += kStepThreads) {
-      const int i = e / NP, j = e % NP;
-      sEc[i * LD + j] = i < l && j < l ? FFc[i * l + j] : 0.0;
-    }
-  } else {
+  if (nb == 0) __syncthreads();
+  for (int job = wave; job < JU; job += kStepWaves) {
+    const int side = job / (RT * NT), i0 = job % (RT * NT) / NT * 16, j0 = job % NT * 16;
+    const double* x = bDc + (side * R + i0 + c) * LD + kq;  // times C
+    const double* y = bX4 + (side * R + i0 + c) * LD + kq;  // times Cinv
+    d4 p = zero, q = zero;
 #pragma unroll
-    for (int u = 0; u < ER; ++u) {
-      const int e = tid + u * kStepThreads, r = e / NP, j = e % NP;
-      sBc[r * LD + j] = v[0][u];
-      sBg[r * LD + j] = v[1][u];
-      sEc[r * LD + j] = v[2][u];
+    for (int k = 0; k < NP; k += 4) {
+      const int kk = (k + kq) * LD + j0 + c;
+      p = __builtin_amdgcn_mfma_f64_16x16x4f64(x[k], bX[kk], p, 0, 0, 0);
+      q = __builtin_amdgcn_mfma_f64_16x16x4f64(y[k], bX2[kk], q, 0, 0, 0);
     }
-  }
-  __syncthreads();
-  const int tiles = (ff ? NT : kUpdRows / 16) * NT;
-  const int64_t rows = ff ? l : (nl - r0 < kUpdRows ? nl - r0 : kUpdRows);
-  for (int job = wave; job < (ff ? tiles : 2 * tiles); job += kStepWaves) {
-    const bool eside = job < tiles;
-    const int tile = eside ? job : job - tiles, i0 = (tile / NT) * 16, j0 = (tile % NT) * 16;
-    const double* x = (eside ? sEc : sBc) + (i0 + c) * LD;  // times F
-    const double* y = (eside ? sBc : sBg) + (i0 + c) * LD;  // times Cinv
-    d4 p = {0.0, 0.0, 0.0, 0.0}, q = p;
-#pragma unroll
-    for (int k0 = 0; k0 < NP; k0 += 4) {
-      const int k = k0 + kq;
-      p = __builtin_amdgcn_mfma_f64_16x16x4f64(x[k], sF[k * LD + j0 + c], p, 0, 0, 0);
-      if (!ff) q = __builtin_amdgcn_mfma_f64_16x16x4f64(y[k], sC[k * LD + j0 + c], q, 0, 0, 0);
-    }
-    double* out = ff ? FFp : eside ? Ep : Bp;
+    double* out = side == 0 ? Bp : Ep;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = i0 + kq + 4 * r, j = j0 + c;
-      if (i < rows && j < l)
-        out[(ff ? i : r0 + i) * l + j] = eside ? p[r] + invN * q[r] : p[r] + q[r];
+      if (i < rows && j < l) out[static_cast<unsigned>(i * l + j)] = p[r] + q[r];
     }
   }
 }
@@ -866,13 +965,12 @@ struct KnMember {
   double* B[2];
   double* Bg;
   double* E[2];
-  double* FF[2];
-  double* P;          // partials of the product's workgroups
+  double* P;          // partials of the product's row blocks
   double* sums;       // their sums (P itself when the update sums them)
   IntegratorState* st;
-  int64_t nl, nblk, nsum, upd_blocks;  // nsum: partials left at `sums`
+  int64_t nl, nblk, nsum;  // row blocks of the product and the update; partials left at `sums`
   double invN, tol;
-  int l, rows, vec;   // rows per product workgroup; Bs takes 16-byte loads
+  int l, rows, parts, vec;  // rows per block, parts of a product's columns; Bs takes 16-byte loads
   int t;              // the member's iteration index in this launch
 };
 
@@ -882,14 +980,30 @@ struct KnGroup {
 };
 static_assert(sizeof(KnGroup) <= 4096, "the member table fits the kernel arguments");
 
-// The product and the update are launched once per class of l present (NP = l rounded up to 32, 48
-// or 64).
-template <int NP>
+// The product and the update are launched once per class of l (NP = l rounded up to 32, 48 or 64)
+// and rows per block (R) present.
+// A product's parts of one row block are eight workgroups apart, on the same XCD and its L2.
+template <int NP, int R>
 __global__ __launch_bounds__(kStepThreads) void kn_product_group_kernel(KnGroup g) {
+  constexpr int NT = NP / 16;
+  __shared__ double smem[product_lds<NP, R>()];
   const KnMember& m = g.m[blockIdx.y];
-  if (blockIdx.x >= m.nblk) return;
-  kn_product_body<NP>(m.t, m.st, static_cast<int>(m.nl), m.l, m.rows, m.vec != 0, m.invN, m.Bs,
-                      m.B[m.t & 1], m.Bg, m.P, blockIdx.x);
+  const int x = blockIdx.x, part = x / 8 % m.parts, blk = x / (8 * m.parts) * 8 + x % 8;
+  if (blk >= m.nblk || skip(m.st, m.t)) return;
+  const int nl = static_cast<int>(m.nl);
+  auto run = [&](auto ntw) {
+    constexpr int NTW = decltype(ntw)::value;
+    kn_product_body<NP, R, NTW>(nl, m.l, m.vec != 0, m.invN, m.Bs, m.B[m.t & 1], m.Bg, m.P, blk,
+                                part * NTW, smem);
+  };
+  if (R == 32 || m.parts == 1) {
+    run(std::integral_constant<int, NT>());
+  } else if constexpr (R == 16) {
+    if (m.parts == NT)
+      run(std::integral_constant<int, 1>());
+    else if constexpr (NT == 4)
+      run(std::integral_constant<int, 2>());
+  }
 }
 
 __global__ __launch_bounds__(kThreads) void kn_sum_group_kernel(KnGroup g) {
@@ -897,17 +1011,20 @@ __global__ __launch_bounds__(kThreads) void kn_sum_group_kernel(KnGroup g) {
   const int count = m.l * (m.l + 1);
   if (m.nsum == m.nblk || static_cast<int64_t>(blockIdx.x) * kWave >= count || skip(m.st, m.t))
     return;
-  kn_sum_body(m.P, m.nblk, count, m.sums, blockIdx.x);
+  kn_sum_body(m.P, m.nblk, count / 2, m.parts > 1, m.sums, blockIdx.x);
 }
 
-template <int NP>
+template <int NP, int R>
 __global__ __launch_bounds__(kStepThreads) void kn_update_group_kernel(KnGroup g) {
+  __shared__ double smem[4 * kStepBuf];
+  __shared__ double red[kStepWaves];
+  __shared__ double coef[2][4 * kSeriesMaxB];
   const KnMember& m = g.m[blockIdx.y];
   const int t = m.t;
-  if (blockIdx.x >= m.upd_blocks) return;
+  if (blockIdx.x >= m.nblk || skip(m.st, t)) return;
   const int c = t & 1, p = c ^ 1;
-  kn_update_body<NP>(t, m.st, m.nl, m.l, m.invN, m.tol, m.sums, m.nsum, m.B[c], m.Bg, m.B[p],
-                     m.E[c], m.E[p], m.FF[c], m.FF[p], blockIdx.x, m.upd_blocks);
+  kn_update_body<NP, R>(t, m.st, m.nl, m.l, m.invN, m.tol, m.sums, m.nsum, m.B[c], m.Bg, m.B[p],
+                        m.E[c], m.E[p], blockIdx.x, smem, red, coef);
 }
 
 // out[2i] = converged_at, out[2i + 1] = nan_seen of member i (one read-back for the group).
@@ -1477,7 +1594,7 @@ __global__ void init_state_kernel(IntegratorState* st) {
   st->mu = 0.0;
 }
 
-// B0 = first l columns of Bs; E0 = 0; FF0 = I.
+// B0 = first l columns of Bs; E0 = 0 and FF0 = I, or E0 = [I; 0] where FF0 is null.
 __global__ void init_coef_kernel(const double* __restrict__ Bs, int64_t nl, int l,
                                  double* __restrict__ B0, double* __restrict__ E0,
                                  double* __restrict__ FF0) {
@@ -1487,8 +1604,9 @@ __global__ void init_coef_kernel(const double* __restrict__ Bs, int64_t nl, int 
     const int64_t r = e / l;
     const int j = e % l;
     B0[e] = Bs[r * nl + j];
-    E0[e] = 0.0;
-    if (e < (int64_t)l * l) FF0[e] = ((e / l) == (e % l)) ? 1.0 : 0.0;
+    const double id = r == j ? 1.0 : 0.0;
+    E0[e] = FF0 == nullptr ? id : 0.0;
+    if (FF0 != nullptr && r < l) FF0[e] = id;
   }
 }
 
@@ -1644,7 +1762,8 @@ Layout layout(char* base, int64_t N, int l) {
   L.BsU1 = take(nll);
   const size_t pp = static_cast<size_t>(L.nblk_p) * 3 * ll;
   const size_t pt = static_cast<size_t>(L.nblk_t) * (3 * ll + 2);
-  // (a KN iteration's (ceil(nl / 16) + 1) l (l + 1) doubles of partials and their sums fit pt)
+  // (A KN iteration's partials, at most ceil(nl / 16) 3 l (l + 1) / 2 doubles, and their sums, l (l +
+  // 1), may run on into Pbg, which it does not use: 3 nl / 32 l^2 + 2 nl l doubles in all.)
   L.P = take(pp > pt ? pp : pt);
   L.Pbg = take(static_cast<size_t>(L.splits + 1) * nll);
   L.T = take(3 * ll + 2);
@@ -1710,33 +1829,37 @@ void check_integrator(const GramIntegrator& g, const Layout& L) {
   MCNLA_REQUIRE(g.ws_bytes >= L.bytes, MCNLA_ERR_INVALID, "integrator workspace too small");
 }
 
-// State reset, B0 = Bs(:, 0:l), E0 = 0, FF0 = I.
+// State reset, B0 = Bs(:, 0:l), and E0 + [FF0; 0] = [I; 0]: KN keeps all of it in E.
 void init_iteration(const GramIntegrator& g, const Layout& L, hipStream_t st) {
   hipLaunchKernelGGL(init_state_kernel, dim3(1), dim3(1), 0, st, L.st);
   MCNLA_LAUNCHED();
   hipLaunchKernelGGL(init_coef_kernel, dim3(grid_elems(L.nl * g.l)), dim3(kThreads), 0, st, g.Bs,
-                     L.nl, g.l, L.B[0], L.E[0], L.FF[0]);
+                     L.nl, g.l, L.B[0], L.E[0], g.wen_yin ? L.FF[0] : nullptr);
   MCNLA_LAUNCHED();
 }
 
 // The coefficients after `iters` iterations, re-orthonormalized: coef = M W with
-// M = E + [FF; 0] and W = (M' Bs M)^{-1/2}.
+// M = E (KN) or E + [FF; 0] and W = (M' Bs M)^{-1/2}.
 void finish_iteration(const GramIntegrator& g, const Layout& L, int64_t iters, double* coef,
                       hipStream_t st) {
   const int64_t nl = L.nl;
   const int l = g.l;
   const int fin = static_cast<int>(iters & 1);
-  hipLaunchKernelGGL(coef_kernel, dim3(grid_elems(nl * l)), dim3(kThreads), 0, st, L.E[fin],
-                     L.FF[fin], nl, l, L.U1);
-  MCNLA_LAUNCHED();
-  bs_product(g, L, L.U1, L.BsU1, -1, st);
+  const double* M = L.E[fin];
+  if (g.wen_yin) {
+    hipLaunchKernelGGL(coef_kernel, dim3(grid_elems(nl * l)), dim3(kThreads), 0, st, L.E[fin],
+                       L.FF[fin], nl, l, L.U1);
+    MCNLA_LAUNCHED();
+    M = L.U1;
+  }
+  bs_product(g, L, M, L.BsU1, -1, st);
   hipLaunchKernelGGL(gram_partials_kernel, dim3(static_cast<unsigned>(L.nblk_p)), dim3(kThreads),
-                     0, st, -1, L.st, nl, l, L.U1, L.BsU1, L.P, 2);
+                     0, st, -1, L.st, nl, l, M, L.BsU1, L.P, 2);
   MCNLA_LAUNCHED();
   hipLaunchKernelGGL(polish_kernel, dim3(1), dim3(kWyThreads), 0, st, l, static_cast<double>(g.N),
                      L.P, L.nblk_p, L.F);
   MCNLA_LAUNCHED();
-  hipLaunchKernelGGL(right_mul_kernel, dim3(grid_elems(nl * l)), dim3(kThreads), 0, st, nl, l, L.U1,
+  hipLaunchKernelGGL(right_mul_kernel, dim3(grid_elems(nl * l)), dim3(kThreads), 0, st, nl, l, M,
                      L.F, coef);
   MCNLA_LAUNCHED();
 }
@@ -1750,19 +1873,17 @@ KnMember kn_member(const GramIntegrator& g, const Layout& L) {
   m.Bg = L.Bg[0];
   m.E[0] = L.E[0];
   m.E[1] = L.E[1];
-  m.FF[0] = L.FF[0];
-  m.FF[1] = L.FF[1];
   m.P = L.P;
   m.st = L.st;
   m.nl = nl;
   m.l = g.l;
   m.rows = step_rows(nl);
   m.nblk = ceil_div(nl, m.rows);
+  m.parts = step_parts(m.nblk, g.l);
   const bool direct = m.nblk <= kDirectPartials;
   m.nsum = direct ? m.nblk : 1;
-  m.sums = direct ? L.P : L.P + m.nblk * g.l * (g.l + 1);
+  m.sums = direct ? L.P : L.P + m.nblk * g.l * (g.l + 1) / 2 * (m.parts > 1 ? 3 : 2);
   m.vec = (reinterpret_cast<uintptr_t>(g.Bs) % 16 == 0 && nl % 2 == 0) ? 1 : 0;
-  m.upd_blocks = kn_update_blocks(nl);
   m.invN = 1.0 / static_cast<double>(g.N);
   m.tol = g.tol;
   return m;
@@ -1771,15 +1892,15 @@ KnMember kn_member(const GramIntegrator& g, const Layout& L) {
 // One KN iteration of the members in `act` (member i at its iteration act.m[i].t): the products (a
 // launch per class of l present), the sums of their partials, then the l x l steps and updates.
 void launch_kn_iteration(const KnGroup& act, hipStream_t st) {
-  KnGroup cls[3];
-  int64_t bp[3] = {0, 0, 0}, bu[3] = {0, 0, 0}, bs = 0;
+  KnGroup cls[6];
+  int64_t bp[6] = {}, bu[6] = {}, bs = 0;
   for (auto& c : cls) c.count = 0;
   for (int i = 0; i < act.count; ++i) {
     const KnMember& m = act.m[i];
-    const int c = m.l <= 32 ? 0 : m.l <= 48 ? 1 : 2;
+    const int c = (m.l <= 32 ? 0 : m.l <= 48 ? 1 : 2) + (m.rows == 16 ? 0 : 3);
     cls[c].m[cls[c].count++] = m;
-    bp[c] = std::max(bp[c], m.nblk);
-    bu[c] = std::max(bu[c], m.upd_blocks);
+    bp[c] = std::max(bp[c], m.parts == 1 ? m.nblk : ceil_div(m.nblk, 8) * 8 * m.parts);
+    bu[c] = std::max(bu[c], m.nblk);
     if (m.nsum != m.nblk)
       bs = std::max<int64_t>(bs, ceil_div(static_cast<int64_t>(m.l) * (m.l + 1), kWave));
     MCNLA_REQUIRE(m.nl < (1LL << 31), MCNLA_ERR_INVALID, "integrator grid too large");
@@ -1790,13 +1911,19 @@ void launch_kn_iteration(const KnGroup& act, hipStream_t st) {
                        g);
     MCNLA_LAUNCHED();
   };
-  launch(kn_product_group_kernel<32>, cls[0], bp[0], kStepThreads);
-  launch(kn_product_group_kernel<48>, cls[1], bp[1], kStepThreads);
-  launch(kn_product_group_kernel<64>, cls[2], bp[2], kStepThreads);
+  launch(kn_product_group_kernel<32, 16>, cls[0], bp[0], kStepThreads);
+  launch(kn_product_group_kernel<48, 16>, cls[1], bp[1], kStepThreads);
+  launch(kn_product_group_kernel<64, 16>, cls[2], bp[2], kStepThreads);
+  launch(kn_product_group_kernel<32, 32>, cls[3], bp[3], kStepThreads);
+  launch(kn_product_group_kernel<48, 32>, cls[4], bp[4], kStepThreads);
+  launch(kn_product_group_kernel<64, 32>, cls[5], bp[5], kStepThreads);
   launch(kn_sum_group_kernel, act, bs, kThreads);
-  launch(kn_update_group_kernel<32>, cls[0], bu[0], kStepThreads);
-  launch(kn_update_group_kernel<48>, cls[1], bu[1], kStepThreads);
-  launch(kn_update_group_kernel<64>, cls[2], bu[2], kStepThreads);
+  launch(kn_update_group_kernel<32, 16>, cls[0], bu[0], kStepThreads);
+  launch(kn_update_group_kernel<48, 16>, cls[1], bu[1], kStepThreads);
+  launch(kn_update_group_kernel<64, 16>, cls[2], bu[2], kStepThreads);
+  launch(kn_update_group_kernel<32, 32>, cls[3], bu[3], kStepThreads);
+  launch(kn_update_group_kernel<48, 32>, cls[4], bu[4], kStepThreads);
+  launch(kn_update_group_kernel<64, 32>, cls[5], bu[5], kStepThreads);
 }
 
 // The KN loop of a group.  `graphs` (a group of one only) records each chunk once and replays it.

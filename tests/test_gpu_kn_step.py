@@ -39,3 +39,23 @@ def test_kn_iteration_edges(m, l, N, spread):
     ref, iters = oracle.kn_rowblock(Qs, l, N, 256, 1e-4)
     assert it.iteration() == iters
     assert np.max(np.abs(Qbar.numpy() - ref)) < 1e-8
+
+
+@pytest.mark.parametrize("l,N", [
+    (64, 20),   # Nl = 1280: the columns of a row block in two parts
+    (17, 130),  # Nl = 2210, uncut again
+    (37, 40),   # Nl = 1480
+    (49, 45),   # Nl = 2205, odd
+    (33, 128),  # Nl = 4224: 32-row workgroups
+    (20, 7),    # Nl = 140: the smallest in two parts
+])
+def test_kn_product_parts(l, N):
+    """The rule that cuts a product's row blocks by columns, on both sides of its lines."""
+    Qs = sketches(150, l, N, 0.5, seed=l + N)
+    P = mc.Parameters().setSize(150, 150).setRank(l).setOverRank(0).setNumSketch(N)
+    it = mc.RowBlockKolmogorovNagumoIntegrator(P, 256, 1e-4)
+    Qbar = P.createMatrixQbar()
+    it(mc.DeviceArray.from_numpy(Qs), Qbar)
+    ref, iters = oracle.kn_rowblock(Qs, l, N, 256, 1e-4)
+    assert it.iteration() == iters
+    assert np.max(np.abs(Qbar.numpy() - ref)) < 1e-8
