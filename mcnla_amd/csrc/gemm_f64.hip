@@ -11,6 +11,7 @@
 // Tiles are staged through LDS as [k][mn] (mn contiguous) so that every MFMA operand fragment is
 // one LDS row segment; v_mfma_f64_16x16x4f64 does the arithmetic.  Source elements may be FP32
 // (mixed precision collections); they are widened to FP64 on the way into LDS.
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -230,6 +231,156 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_f64_kernel(
           }
         }
       }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Products with few tiles, and those the DMA path cannot take: a wave computes a 32 x 32 tile with
+// its operands straight from L1/L2 into MFMA registers, D stages of 16 k deep, with no LDS and no
+// barrier in the loop.  WG x WG waves make a square tile of the workgroup (they share its operands
+// through L1), times WK waves that take every WK-th stage and are summed through LDS in order.
+//   WG = 1, WK = 8: a chip full of 32 x 32 tiles is 6 % of one full of 128 x 128 ones, so a product
+//     of a few tiles spreads over CUs and SIMDs instead of walking all of K in one wave.
+//   WG = 2, WK = 2: 64 x 64 tiles, where those fill the chip.
+template <typename T, bool CONTIG>
+struct WaveOperand {
+  const T* p[2];     // the lane's k = 4 kq of the split's first stage, rows i and i + 16
+  int64_t su;        // elements between k and k + 1
+  // x0 + i < count: the tile's rows (columns of B), repeated past the last
+  __device__ __forceinline__ WaveOperand(const void* base, int64_t ld, int64_t x0, int64_t count,
+                                         int64_t k) {
+    su = CONTIG ? ld : 1;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int64_t r = x0 + 16 * i + (threadIdx.x & 15), x = r < count ? r : count - 1;
+      p[i] = static_cast<const T*>(base) + (CONTIG ? x + k * ld : x * ld + k);
+    }
+  }
+};
+
+template <typename TA, typename TB, bool A_MC, bool B_NC, int WG, int WK>
+__global__ __launch_bounds__(WG* WG* WK * 64) void gemm_f64_wave_kernel(GemmF64Args p) {
+  constexpr int T = 32 * WG, D = 4, LD = 34;
+  __shared__ double sums[WK > 1 ? WG * WG * WK * 32 * LD : 1];
+  if (p.gate != nullptr && *p.gate < p.gate_t) return;
+  const int64_t tiles_m = ceil_div(p.M, T), tiles_n = ceil_div(p.N, T);
+  const int64_t ntiles = p.lower_only ? tiles_m * (tiles_m + 1) / 2 : tiles_m * tiles_n;
+  const int64_t logical = xcd_swizzle(blockIdx.x, ntiles * p.splits * p.batch);
+  const int64_t bat = logical / (ntiles * p.splits);
+  const int64_t split = (logical / ntiles) % p.splits, t = logical % ntiles;
+  int64_t tm, tn;
+  if (p.lower_only) {
+    tm = static_cast<int64_t>((sqrt(8.0 * static_cast<double>(t) + 1.0) - 1.0) * 0.5);
+    while (tm * (tm + 1) / 2 > t) --tm;
+    while ((tm + 1) * (tm + 2) / 2 <= t) ++tm;
+    tn = t - tm * (tm + 1) / 2;
+  } else {
+    tm = t / tiles_n;
+    tn = t % tiles_n;
+  }
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, c = lane & 15, kq = lane >> 4;
+  const int wk = wave / (WG * WG), wt = wave % (WG * WG);
+  const int64_t m0 = tm * T + wt / WG * 32, n0 = tn * T + wt % WG * 32;
+  const int64_t kbeg = split * p.kchunk;
+  const int64_t kend = (kbeg + p.kchunk < p.K) ? kbeg + p.kchunk : p.K;
+  d4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+  if (kbeg < kend && m0 < p.M && n0 < p.N) {
+    const WaveOperand<TA, A_MC> A(static_cast<const TA*>(p.A) + bat * p.stride_a, p.lda, m0, p.M,
+                                  kbeg + 4 * kq);
+    const WaveOperand<TB, B_NC> B(static_cast<const TB*>(p.B) + bat * p.stride_b, p.ldb, n0, p.N,
+                                  kbeg + 4 * kq);
+    TA a[D][2][4];
+    TB b[D][2][4];
+    auto load = [&](int64_t s, TA (&x)[2][4], TB (&y)[2][4]) {
+      const int64_t k = 16 * (wk + WK * s);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          x[i][u] = A.p[i][(k + u) * A.su];
+          y[i][u] = B.p[i][(k + u) * B.su];
+        }
+    };
+    auto mul = [&](const TA (&x)[2][4], const TB (&y)[2][4]) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                static_cast<double>(x[i][u]), static_cast<double>(y[j][u]), acc[i][j], 0, 0, 0);
+    };
+    const int64_t whole = (kend - kbeg) / 16;
+    const int64_t n = whole > wk ? (whole - wk + WK - 1) / WK : 0;
+#pragma unroll
+    for (int s = 0; s < D - 1; ++s)
+      if (s < n) load(s, a[s], b[s]);
+    int64_t s0 = 0;
+    for (; s0 + D <= n; s0 += D) {
+#pragma unroll
+      for (int s = 0; s < D; ++s) {
+        const int64_t ahead = s0 + s + D - 1;
+        load(ahead < n ? ahead : n - 1, a[(s + D - 1) % D], b[(s + D - 1) % D]);
+        mul(a[s], b[s]);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < D - 1; ++s)
+      if (s0 + s < n) mul(a[s], b[s]);
+    if ((kend - kbeg) % 16 != 0 && whole % WK == wk) {  // the last, partial stage
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t k = 16 * whole + 4 * kq + u;
+        const bool in = kbeg + k < kend;
+        const int64_t at = (in ? k : kend - kbeg - 1) - 4 * kq;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const TA x = A.p[i][at * A.su];
+          const TB y = B.p[i][at * B.su];
+          a[0][i][u] = in ? x : TA(0);
+          b[0][i][u] = in ? y : TB(0);
+        }
+      }
+      mul(a[0], b[0]);
+    }
+  }
+  double* __restrict__ C = p.partial ? p.partial + (bat * p.splits + split) * p.M * p.N
+                                     : p.C + bat * p.stride_c;
+  const int64_t ldc = p.partial ? p.N : p.ldc;
+  auto put = [&](int64_t gi, int64_t gj, double v) {
+    if (gi >= p.M || gj >= p.N) return;
+    double* x = C + gi * ldc + gj;
+    *x = p.partial ? v : (p.beta == 0.0) ? p.alpha * v : p.alpha * v + p.beta * *x;
+  };
+  if constexpr (WK == 1) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) put(m0 + 16 * i + kq + 4 * r, n0 + 16 * j + c, acc[i][j][r]);
+  } else {
+    double* own = sums + wave * 32 * LD;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) own[(16 * i + kq + 4 * r) * LD + 16 * j + c] = acc[i][j][r];
+    __syncthreads();
+    for (int e = threadIdx.x; e < T * T; e += WG * WG * WK * 64) {
+      const int i = e / T, j = e % T;
+      const double* x = sums + (i / 32 * WG + j / 32) * 32 * LD + i % 32 * LD + j % 32;
+      double v = 0.0;
+#pragma unroll
+      for (int w = 0; w < WK; ++w) v += x[w * WG * WG * 32 * LD];
+      put(tm * T + i, tn * T + j, v);
+    }
+  }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1116,34 +1267,94 @@ void launch_cfg(const GemmF64Args& p, hipStream_t st) {
 }
 
 template <typename TA, typename TB, bool A_MC, bool B_NC>
-void launch_shape(const GemmF64Args& p, hipStream_t st) {
-  switch (p.shape) {
-    case GemmShape::kSquare:  // 128 x 128 tiles, 4 waves of 64 x 64
-      launch_cfg<TA, TB, A_MC, B_NC, 128, 128, 16, 64, 64>(p, st);
-      break;
-    case GemmShape::kTallN32:  // 128 x 32 tiles, 4 waves stacked along M
-      launch_cfg<TA, TB, A_MC, B_NC, 128, 32, 16, 32, 32>(p, st);
-      break;
-    case GemmShape::kTallN64:
-      launch_cfg<TA, TB, A_MC, B_NC, 128, 64, 16, 32, 64>(p, st);
-      break;
-    case GemmShape::kWideM32:  // 32 x 128 tiles, 4 waves along N
-      launch_cfg<TA, TB, A_MC, B_NC, 32, 128, 16, 32, 32>(p, st);
-      break;
-    case GemmShape::kSmall:  // 32 x 32 tiles, 1 wave (tiny l x l products, split-K)
-      launch_cfg<TA, TB, A_MC, B_NC, 32, 32, 16, 32, 32>(p, st);
-      break;
+void launch_tall_tiles(const GemmF64Args& p, hipStream_t st) {
+  if (p.shape == GemmShape::kTallN32)  // 128 x 32 tiles, 4 waves stacked along M
+    launch_cfg<TA, TB, A_MC, B_NC, 128, 32, 16, 32, 32>(p, st);
+  else
+    launch_cfg<TA, TB, A_MC, B_NC, 128, 64, 16, 32, 64>(p, st);
+}
+
+// Workgroups of the wave kernel with tiles of 32 wg rows and columns.
+int64_t wave_blocks(const GemmF64Args& p, int wg, int64_t splits) {
+  const int64_t tm = ceil_div(p.M, 32 * wg), tn = ceil_div(p.N, 32 * wg);
+  return (p.lower_only ? tm * (tm + 1) / 2 : tm * tn) * splits * p.batch;
+}
+
+// What a grid of one workgroup per CU costs: whole rounds of tiles of `area` entries, kchunk deep,
+// at the rate (TFLOP/s) that the kernel reaches with the chip full, in units of 2 / 1e12 s.
+double rounds_cost(int64_t blocks, int64_t area, int64_t kchunk, double rate) {
+  const int64_t cus = device_cus();
+  return static_cast<double>(ceil_div(blocks, cus) * cus) * static_cast<double>(area) *
+         static_cast<double>(kchunk) / rate;
+}
+
+// Rates at which the choices below come out as measured (all FP64; DMA 256 x 128, wave 64 x 64 and
+// 32 x 32 tiles, us): 2000 x 160 x 1000 237 / 47 / 32, 4000 x 256 x 2000 462 / 90 / 106, 20000 x
+// 256 x 1000 237 / 222 / 295, Y'Y of 512 columns, 6000 rows 91 / 81 / 86, 20000 rows 213 / 242 / 269;
+// without the DMA kernel's alignment, 12347 x 527 x 1999 - / 574 / 686, 4001 x 301 x 1501 - / 131 /
+// 107.  (128 x 128 tiles staged through registers and LDS, which these replace, took 231 us for
+// 2000 x 80 x 1000, 18 now, 809 for 12347 x 527 x 1999 and 4580 for 20000 x 1024 x 4000, 3311 now.)
+constexpr double kDmaRate = 60.0, kNarrowRate = 50.0, kWave2Rate = 44.0, kWave1Rate = 38.0;
+
+struct WavePlan {
+  int wg = 0;  // 1: 32 x 32 tiles, 2: 64 x 64
+  int64_t splits = 1, kchunk = 0;
+  double cost = 0.0;
+};
+
+// The cheaper form of the wave kernel, and of the split-K factors up to p.splits (where the sums
+// are taken here) the cheapest, a partial written and read at 3 TB/s.
+WavePlan wave_plan(const GemmF64Args& p) {
+  WavePlan best;
+  const int64_t lo = p.splits > 1 && p.partial != nullptr && p.C != nullptr ? 1 : p.splits;
+  for (int64_t s = p.splits; s >= lo; s = s > 1 ? std::max<int64_t>(s * 3 / 4, 1) : 0) {
+    const int64_t chunk = s == p.splits ? p.kchunk : ceil_div(p.K, s);
+    const int64_t kchunk = std::max<int64_t>(ceil_div(chunk, 16) * 16, 16);
+    const int64_t splits = std::max<int64_t>(ceil_div(p.K, kchunk), 1);
+    for (int wg = 1; wg <= 2; ++wg) {
+      const double sums = splits > 1 || p.lower_only
+                              ? 8.0 / 3.0 * static_cast<double>(splits) * static_cast<double>(p.M) *
+                                    static_cast<double>(p.N) * static_cast<double>(p.batch)
+                              : 0.0;
+      const double cost = sums + rounds_cost(wave_blocks(p, wg, splits), 1024 * wg * wg, kchunk,
+                                             wg == 1 ? kWave1Rate : kWave2Rate);
+      if (best.wg == 0 || cost < best.cost) best = {wg, splits, kchunk, cost};
+    }
   }
+  return best;
+}
+
+template <typename TA, typename TB, bool A_MC, bool B_NC>
+void launch_wave(const GemmF64Args& p, int wg, hipStream_t st) {
+  const int64_t nblocks = wave_blocks(p, wg, p.splits);
+  MCNLA_REQUIRE(nblocks < (1LL << 31), MCNLA_ERR_INVALID, "GEMM grid too large");
+  if (wg == 1)
+    hipLaunchKernelGGL((gemm_f64_wave_kernel<TA, TB, A_MC, B_NC, 1, 8>),
+                       dim3(static_cast<unsigned>(nblocks)), dim3(512), 0, st, p);
+  else
+    hipLaunchKernelGGL((gemm_f64_wave_kernel<TA, TB, A_MC, B_NC, 2, 2>),
+                       dim3(static_cast<unsigned>(nblocks)), dim3(512), 0, st, p);
+  MCNLA_LAUNCHED();
 }
 
 template <typename TA, typename TB>
-void launch_types(const GemmF64Args& p, hipStream_t st) {
+void launch_types(const GemmF64Args& p, int wg, hipStream_t st) {
+  if (wg != 0) {
+    if (p.a_mcontig) {
+      if (p.b_ncontig) launch_wave<TA, TB, true, true>(p, wg, st);
+      else launch_wave<TA, TB, true, false>(p, wg, st);
+    } else {
+      if (p.b_ncontig) launch_wave<TA, TB, false, true>(p, wg, st);
+      else launch_wave<TA, TB, false, false>(p, wg, st);
+    }
+    return;
+  }
   if (p.a_mcontig) {
-    if (p.b_ncontig) launch_shape<TA, TB, true, true>(p, st);
-    else launch_shape<TA, TB, true, false>(p, st);
+    if (p.b_ncontig) launch_tall_tiles<TA, TB, true, true>(p, st);
+    else launch_tall_tiles<TA, TB, true, false>(p, st);
   } else {
-    if (p.b_ncontig) launch_shape<TA, TB, false, true>(p, st);
-    else launch_shape<TA, TB, false, false>(p, st);
+    if (p.b_ncontig) launch_tall_tiles<TA, TB, false, true>(p, st);
+    else launch_tall_tiles<TA, TB, false, false>(p, st);
   }
 }
 
@@ -1161,15 +1372,46 @@ void gemm_f64(GemmF64Args p, hipStream_t st) {
   // 256 x 128 DMA tiles from N = 128, 256 x 64 ones for 32 < N <= 64 (an even K: B's k-rows go
   // in pairs; no lower-triangle schedule)
   const bool narrow = p.N > 32 && p.N <= 64 && !p.lower_only && p.K % 2 == 0;
-  const bool dma = p.kernel == 0 && !p.a_f32 && !p.b_f32 && p.a_mcontig && p.b_ncontig &&
-                   p.shape == GemmShape::kSquare && p.M >= 128 && (p.N >= 128 || narrow) &&
-                   even16(p.A, p.lda, p.stride_a) &&
-                   even16(p.B, p.ldb, p.stride_b);
+  bool dma = p.kernel == 0 && !p.a_f32 && !p.b_f32 && p.a_mcontig && p.b_ncontig &&
+             p.shape == GemmShape::kSquare && p.M >= 128 && (p.N >= 128 || narrow) &&
+             even16(p.A, p.lda, p.stride_a) && even16(p.B, p.ldb, p.stride_b);
   const bool tall = !p.a_mcontig && p.b_ncontig && !p.b_f32 && p.N <= 64 && p.batch == 1 &&
                     !p.lower_only && p.M >= 128 &&
                     (p.shape == GemmShape::kTallN32 || p.shape == GemmShape::kTallN64);
   const bool stream = tall && (p.splits == 1 || p.partial != nullptr) && tall_stream_ok(p);
-  // The register-staged kernels need split ranges that are whole K tiles (16); the DMA kernels
+  // The wave kernel takes every product but the tall ones and those large enough for the DMA
+  // tiles; of the tall ones that tall_* cannot take (A along M), it takes those of fewer 128-row
+  // tiles than CUs (2000 x 20 x 2000 in 8 splits: 28 -> 16 us; in 512 tiles, 1999 x 31 x 12347, the
+  // shared B of the larger ones wins, 57 against 71 us).  Partials that the caller sums (C null)
+  // keep their split and, where they had it, the DMA kernel.
+  const bool tall_tiles = p.shape == GemmShape::kTallN32 || p.shape == GemmShape::kTallN64;
+  WavePlan wave;
+  if (!tall && !(dma && p.C == nullptr) &&
+      !(tall_tiles && ceil_div(p.M, 128) * ceil_div(p.N, p.shape == GemmShape::kTallN32 ? 32 : 64) *
+                              p.splits * p.batch >= device_cus())) {
+    wave = wave_plan(p);
+    if (dma) {
+      const int64_t tm = ceil_div(p.M, 256), area = 256 * (p.N <= 64 ? 64 : 128);
+      const int64_t blocks = (p.N <= 64      ? tm
+                              : p.lower_only ? tm * tm + tm
+                                             : tm * ceil_div(p.N, 128)) * p.splits * p.batch;
+      const double sums = p.splits > 1 || p.lower_only
+                              ? 8.0 / 3.0 * static_cast<double>(p.splits) *
+                                    static_cast<double>(p.M) * static_cast<double>(p.N) *
+                                    static_cast<double>(p.batch)
+                              : 0.0;
+      if (sums + rounds_cost(blocks, area, p.kchunk, p.N <= 64 ? kNarrowRate : kDmaRate) <=
+          wave.cost)
+        wave.wg = 0;
+      else
+        dma = false;
+    }
+    if (wave.wg != 0) {
+      p.splits = wave.splits;
+      p.kchunk = wave.kchunk;
+    }
+  }
+  // The register-fed kernels need split ranges that are whole K tiles (16); the DMA kernels
   // mask a partial last tile, so their splits can be equal.
   if (stream) {
     if (p.a_f32)
@@ -1184,8 +1426,8 @@ void gemm_f64(GemmF64Args p, hipStream_t st) {
   MCNLA_REQUIRE(!(p.splits > 1 && p.partial == nullptr), MCNLA_ERR_INVALID,
                 "split-K GEMM needs a partial buffer");
   MCNLA_REQUIRE(!p.lower_only || p.M == p.N, MCNLA_ERR_INVALID, "lower_only needs M == N");
-  MCNLA_REQUIRE(!p.lower_only || p.shape == GemmShape::kSquare || p.shape == GemmShape::kSmall,
-                MCNLA_ERR_INVALID, "lower_only needs square tiles");
+  MCNLA_REQUIRE(!p.lower_only || dma || wave.wg != 0, MCNLA_ERR_INVALID,
+                "lower_only needs square tiles");
   if (p.ev_begin) MCNLA_HIP(hipEventRecord(p.ev_begin, st));
   if (tall) {
     // defaults (the fastest measured at the benchmark shapes): both operands streamed into LDS
@@ -1240,11 +1482,11 @@ void gemm_f64(GemmF64Args p, hipStream_t st) {
     }
     MCNLA_LAUNCHED();
   } else if (p.a_f32) {
-    if (p.b_f32) launch_types<float, float>(p, st);
-    else launch_types<float, double>(p, st);
+    if (p.b_f32) launch_types<float, float>(p, wave.wg, st);
+    else launch_types<float, double>(p, wave.wg, st);
   } else {
-    if (p.b_f32) launch_types<double, float>(p, st);
-    else launch_types<double, double>(p, st);
+    if (p.b_f32) launch_types<double, float>(p, wave.wg, st);
+    else launch_types<double, double>(p, wave.wg, st);
   }
   if (p.ev_end) MCNLA_HIP(hipEventRecord(p.ev_end, st));
   if (p.partial != nullptr && p.C != nullptr && p.lower_only) {
