@@ -806,7 +806,7 @@ size_t integration_workspace(int kind, int64_t N, int l) {
 // the Nl x l coefficients of Qbar.  Returns the iteration count (0 for the combining kinds).
 int64_t run_integration(int kind, const double* Bs, int64_t N, int l, int64_t maxiter, double tol,
                         double* coef, DevBuf& ws, hipStream_t st, bool* conv, bool* ok,
-                        IterationGraphs* graphs = nullptr) {
+                        IterationGraphs* graphs = nullptr, const KnPoll* poll = nullptr) {
   ws.ensure(integration_workspace(kind, N, l));
   if (is_combining(kind)) {
     if (kind == MCNLA_INT_ROW_BLOCK_REDUCTION)
@@ -827,6 +827,7 @@ int64_t run_integration(int kind, const double* Bs, int64_t N, int l, int64_t ma
   gi.ws = ws.as<char>();
   gi.ws_bytes = ws.bytes;
   gi.graphs = graphs;
+  gi.poll = poll;
   return integrate_gram(gi, coef, st, conv, ok);
 }
 
@@ -1180,6 +1181,12 @@ void SolveRes::create() {
     for (auto& e : marks) MCNLA_HIP(hipEventCreate(&e));
     for (hipEvent_t* e : {&sketch_beg, &sketch_end, &gram_beg, &gram_end, &former_beg, &former_end})
       MCNLA_HIP(hipEventCreate(e));
+    for (auto& e : poll.done) MCNLA_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    void* p = nullptr;
+    if (hipHostMalloc(&p, 2 * 2 * kMaxKnGroup * sizeof(int), hipHostMallocDefault) == hipSuccess)
+      poll.flags = static_cast<int*>(p);
+    else
+      (void)hipGetLastError();  // solves read their flags chunk by chunk instead
   } catch (...) {
     destroy();
     throw;
@@ -1192,6 +1199,9 @@ void SolveRes::destroy() {
     if (*e) (void)hipEventDestroy(*e), *e = nullptr;
   for (auto& e : marks)
     if (e) (void)hipEventDestroy(e), e = nullptr;
+  for (auto& e : poll.done)
+    if (e) (void)hipEventDestroy(e), e = nullptr;
+  if (poll.flags) (void)hipHostFree(poll.flags), poll.flags = nullptr;
   if (side) (void)hipStreamDestroy(side), side = nullptr;
 }
 
@@ -1476,6 +1486,7 @@ GramIntegrator solver_kn_integrator(mcnla_solver s) {
   gi.Bs = s->Bs.as<double>();
   gi.ws = s->ws.as<char>();
   gi.ws_bytes = s->ws.bytes;
+  gi.poll = &s->res->poll;
   return gi;
 }
 
@@ -2137,7 +2148,7 @@ mcnla_status mcnla_solver_solve(mcnla_solver s, const void* A, int64_t lda, int 
     if (c.graph && !s->graphs) s->graphs = std::make_unique<IterationGraphs>();
     s->iteration = run_integration(c.integrator, s->Bs.as<double>(), p.num_sketch, l, c.maxiter,
                                    c.tol, s->coef.as<double>(), s->ws, st, &cx.conv, &cx.ok,
-                                   s->graphs.get());
+                                   s->graphs.get(), &s->res->poll);
     s->converged = cx.conv;
     solve_finish(s, A, lda, a_dtype, a_order, st, cx, true);
     int bad = 0;
@@ -2239,7 +2250,7 @@ mcnla_status mcnla_solver_solve_host(mcnla_solver s, const void* A, int64_t lda,
     if (c.graph && !s->graphs) s->graphs = std::make_unique<IterationGraphs>();
     s->iteration = run_integration(c.integrator, s->Bs.as<double>(), p.num_sketch, l, c.maxiter,
                                    c.tol, s->coef.as<double>(), s->ws, st, &cx.conv, &cx.ok,
-                                   s->graphs.get());
+                                   s->graphs.get(), &s->res->poll);
     s->converged = cx.conv;
     solve_finish(s, dA, len, a_dtype, a_order, st, cx, true);
     int bad = 0;

@@ -1947,12 +1947,31 @@ void run_kn(const GramIntegrator* gs, double* const* coefs, int count, hipStream
   std::vector<int> conv_at(count, INT_MAX), nan_seen(count, 0), flags(2 * count);
   int64_t t = 0;
   int64_t chunk = 8;
+  // With `poll` the host reads a chunk's flags while the next chunk runs (the device never waits
+  // for the host: 50 to 60 us a chunk at any size, three or four chunks a solve), in chunks that
+  // stay at 8, so that at most 15 iterations are launched in vain.
+  const KnPoll* poll = graphs == nullptr && gs[0].poll && gs[0].poll->flags ? gs[0].poll : nullptr;
+  int turn = 0;          // the set of the next chunk
+  bool pending = false;  // the other set's chunk has not been read
+  auto read_flags = [&](const int* f) {
+    for (int i = 0; i < count; ++i) {
+      conv_at[i] = f[2 * i];
+      nan_seen[i] = f[2 * i + 1];
+    }
+  };
+  auto read_poll = [&](int set) {
+    MCNLA_HIP(hipEventSynchronize(poll->done[set]));
+    read_flags(poll->flags + set * 2 * kMaxKnGroup);
+  };
   hipStream_t ls = st;  // where the iteration launches go: a capture stream while recording
   for (;;) {
     int64_t tmax = 0;  // the furthest iteration any unconverged member may still run
     for (int i = 0; i < count; ++i)
       if (conv_at[i] == INT_MAX) tmax = std::max(tmax, gs[i].maxiter);
-    if (t >= tmax) break;
+    if (t >= tmax) {
+      if (pending) read_poll(turn ^ 1);
+      break;
+    }
     const int64_t tend = (t + chunk < tmax) ? t + chunk : tmax;
     hipGraphExec_t exec = graphs ? graphs->find(t, tend) : nullptr;
     const bool recording = exec == nullptr && graphs != nullptr;
@@ -1995,15 +2014,23 @@ void run_kn(const GramIntegrator* gs, double* const* coefs, int count, hipStream
       exec = made;
     }
     if (exec != nullptr) MCNLA_HIP(hipGraphLaunch(exec, st));
-    hipLaunchKernelGGL(kn_flags_kernel, dim3(1), dim3(kWave), 0, st, all, Ls[0].flags);
+    hipLaunchKernelGGL(kn_flags_kernel, dim3(1), dim3(kWave), 0, st, all,
+                       poll ? poll->flags + turn * 2 * kMaxKnGroup : Ls[0].flags);
     MCNLA_LAUNCHED();
+    if (poll) {
+      MCNLA_HIP(hipEventRecord(poll->done[turn], st));
+      turn ^= 1;
+      if (pending) read_poll(turn);
+      pending = true;
+      if (std::all_of(conv_at.begin(), conv_at.end(), [](int c) { return c != INT_MAX; })) break;
+      continue;
+    }
     MCNLA_HIP(hipMemcpyAsync(flags.data(), Ls[0].flags, 2 * count * sizeof(int),
                              hipMemcpyDeviceToHost, st));
     MCNLA_HIP(hipStreamSynchronize(st));
+    read_flags(flags.data());
     bool running = false;
     for (int i = 0; i < count; ++i) {
-      conv_at[i] = flags[2 * i];
-      nan_seen[i] = flags[2 * i + 1];
       if (conv_at[i] == INT_MAX && t < gs[i].maxiter) running = true;
     }
     if (!running) break;

@@ -194,6 +194,15 @@ struct IterationGraphs {
   }
 };
 
+// Where the host reads a KN group's convergence flags one chunk of iterations behind the launches:
+// two sets of 2 kMaxKnGroup ints of pinned memory that the device writes, and an event for each.
+// Owned by what outlives the run; runs that share one must not overlap.
+constexpr int kMaxKnGroup = 16;
+struct KnPoll {
+  int* flags = nullptr;  // null: none, the host reads them chunk by chunk
+  hipEvent_t done[2] = {};
+};
+
 struct GramIntegrator {
   int64_t N = 0;
   int l = 0;
@@ -205,11 +214,14 @@ struct GramIntegrator {
   char* ws = nullptr;
   size_t ws_bytes = 0;
   IterationGraphs* graphs = nullptr;  // record/replay the iteration chunks as HIP graphs
+  const KnPoll* poll = nullptr;       // KN without graphs: chunks enqueued ahead of their flags
 };
 size_t integrator_workspace_bytes(int64_t N, int l);
 // Runs the whole iteration on the device.  On return (stream-ordered) the Nl x l coefficient
 // matrix M with Qbar = Qs * M is in `coef` (Qs = the orthonormal collection whose Gram is Bs).
-// Returns the iteration count (this call synchronizes the stream once per chunk of iterations).
+// Returns the iteration count (this call synchronizes the stream once per chunk of iterations; with
+// `poll` it waits for the chunk before the one just enqueued, and may return with launches in
+// flight that change nothing but poll's flags).
 int64_t integrate_gram(const GramIntegrator& g, double* coef, hipStream_t st, bool* converged,
                        bool* numeric_ok);
 
@@ -218,7 +230,6 @@ int64_t integrate_gram(const GramIntegrator& g, double* coef, hipStream_t st, bo
 // Bs product: one per tile-width class, l <= 32 and l > 32), and the host reads the group's
 // convergence flags once per chunk of iterations.  Member i's coefficients, iteration count and
 // flags are bit-identical to integrate_gram(gs[i]) alone.  `graphs` of the members are not used.
-constexpr int kMaxKnGroup = 16;
 void integrate_gram_group(const GramIntegrator* gs, double* const* coefs, int count,
                           hipStream_t st, int64_t* iterations, bool* converged, bool* numeric_ok);
 

@@ -53,6 +53,7 @@ struct SolveRes {
   hipEvent_t marks[kMarks] = {};
   hipEvent_t sketch_beg = nullptr, sketch_end = nullptr, gram_beg = nullptr, gram_end = nullptr;
   hipEvent_t former_beg = nullptr, former_end = nullptr;
+  KnPoll poll;
   bool ready() const { return side != nullptr; }
   void create();   // on the current device; throws Error (and holds nothing) on failure
   void destroy();  // idempotent, never throws
