@@ -27,6 +27,7 @@
 // scale kernels raise a device flag, and the caller's FP64 product, launched behind it and gated
 // on the flag, replaces the result.
 #include <algorithm>
+#include <cmath>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -721,16 +722,16 @@ size_t residue_bytes(const ResidueArgs& a, size_t limit, double* cost) {
   return p.bytes;
 }
 
-// Both sides measured on MI355X.  The FP64 kernels: 256 x 128 DMA tiles (M-contiguous FP64 A of
-// even sizes) at 0.237 us per k and round of the CUs, the rows past whole rounds with K split in up
-// to 4; else 128 x 128 register-staged tiles, one per CU at 0.20 us per k, two at 0.42.  The
+// Both sides measured on MI355X.  The FP64 kernels: the register-fed tiles in whole rounds of the
+// CUs, 64 x 64 at 44 TFLOP/s or 32 x 32 at 38, or 256 x 128 DMA tiles (M-contiguous FP64 A of even
+// sizes) at 0.237 us per k and round, the rows past whole rounds with K split in up to 4.  The
 // residue product: its INT8 grid, the norm, pack and reconstruction passes at 5 TB/s and 30 us of
 // launches.  Examples (FP64 / residue): 100000 x 2048 x 10000 57.3 / 33.1 ms,
-// 30011 x 840 x 2503 3.39 / 1.95 ms, 10000 x 800 x 4000 1.89 / 1.03 ms, but 40000 x 800 x 1000
-// 1.26 / 1.58 ms and 10000 x 400 x 1000 0.25 / 0.28 ms (start-up, padding and epilogue of 20-step
-// workgroups).  Symmetric, where the FP64 side also writes and sums its split-K partials (`limit`
-// is their size): 2048^2 x 100000 6.62 / 4.37 ms, 1000^2 x 10000 306 / 205 us, 640^2 x 10000
-// 183 / 130 us; 512^2 x 10000 and 1000^2 x 3000 are even.
+// 30011 x 840 x 2503 2.9 / 1.95 ms, 10000 x 800 x 4000 1.1 / 1.03 ms, but 40000 x 800 x 1000
+// 1.26 / 1.58 ms and 10000 x 400 x 1000 0.2 / 0.28 ms (start-up, padding and epilogue of 20-step
+// workgroups).  Symmetric, where the DMA side also writes and sums its split-K partials (`limit`
+// is their size): 2048^2 x 100000 6.62 / 4.37 ms, 1000^2 x 10000 265 / 205 us; 640^2 x 10000
+// (125 / 130 us), 512^2 x 10000 and 1000^2 x 3000 are even.
 bool residue_pays(const ResidueArgs& a, size_t limit) {
   const double M = static_cast<double>(a.M), N = static_cast<double>(a.N),
                K = static_cast<double>(a.K);
@@ -738,21 +739,28 @@ bool residue_pays(const ResidueArgs& a, size_t limit) {
   const int64_t cus = compute_units();
   double fp64;
   if (a.sym) {
-    const int64_t tm = ceil_div(a.M, 256);
-    fp64 = static_cast<double>(tm * (tm + 1)) * K * 0.237 / static_cast<double>(cus) +
-           2 * static_cast<double>(limit) / 4.5e6;
-  } else if (a.a_mcontig && !a.a_f32 && a.b_ncontig && a.N >= 128 && a.M % 2 == 0 &&
-             a.N % 2 == 0) {
+    const int64_t tm = ceil_div(a.M, 256), t64 = ceil_div(a.M, 64);
+    fp64 = std::min(static_cast<double>(tm * (tm + 1)) * K * 0.237 / static_cast<double>(cus) +
+                        2 * static_cast<double>(limit) / 4.5e6,
+                    static_cast<double>(t64 * (t64 + 1)) * 4096 * K / 44e6 + 15.0);
+  } else {
+    fp64 = HUGE_VAL;
+    for (int wg = 1; wg <= 2; ++wg) {
+      const int64_t t = ceil_div(a.M, 32 * wg) * ceil_div(a.N, 32 * wg);
+      fp64 = std::min(fp64, static_cast<double>(ceil_div(t, cus)) *
+                                (static_cast<double>(cus * 2048 * wg * wg) * K /
+                                     (wg == 1 ? 38e6 : 44e6) + 4.0));
+    }
+  }
+  if (!a.sym && a.a_mcontig && !a.a_f32 && a.b_ncontig && a.N >= 128 && a.M % 2 == 0 &&
+      a.N % 2 == 0) {
     // the DMA tiles; by the shape alone, so that a problem takes one path wherever its operands lie
     const int64_t tiles = ceil_div(a.M, 256) * ceil_div(a.N, 128), full = tiles / cus;
     const int64_t rest = tiles - full * cus;
     double last = rest ? 1.0 : 0.0;
     if (full > 0 && rest > 0 && 2 * rest <= cus)
       last = 1.0 / static_cast<double>(std::min<int64_t>(cus / rest, 4));
-    fp64 = (static_cast<double>(full) + last) * K * 0.237;
-  } else {
-    const int64_t t = ceil_div(a.M, 128) * ceil_div(a.N, 128);
-    fp64 = t <= cus ? K * 0.20 : K * 0.42 * static_cast<double>(t) / (2.0 * cus);
+    fp64 = std::min(fp64, (static_cast<double>(full) + last) * K * 0.237);
   }
   if (fp64 < 60.0) return false;
   const Plan p = plan_for(a, limit);
