@@ -114,20 +114,28 @@ __global__ void gram_diag_blocks_kernel(const double* __restrict__ G, int64_t ld
 }
 
 // Bs = blockdiag(T)' G blockdiag(T), block (I, J) = T_I' G_IJ T_J for I >= J: one workgroup per
-// block pair, G_IJ, T_I, T_J and H = G_IJ T_J in LDS (dynamic, 4 np (np + 1) doubles, np =
-// pad16(l), zero-padded) and both products on f64 MFMA tiles.  Bs is symmetric in exact
-// arithmetic; the entries with global row >= column are computed and written to both halves, so
-// that it is exactly symmetric (its rows can then stand in for its columns).
-__global__ __launch_bounds__(256) void congruence_kernel(const double* __restrict__ G,
-                                                        const double* __restrict__ T,
-                                                        double* __restrict__ Bs, int64_t N,
-                                                        int l) {
+// block pair, G_IJ, T_I, T_J and H = G_IJ T_J in LDS (dynamic, 4 NP (NP + 1) doubles, l <= NP,
+// zero-padded) and both products on f64 MFMA tiles.  Bs is symmetric in exact arithmetic; the
+// entries with global row >= column are computed and written to both halves, so that it is exactly
+// symmetric (its rows can then stand in for its columns).  Bound by one workgroup's chain of loads,
+// products and stores per CU at l = 64 (33 KB a matrix): all loads are in flight together, and the
+// block goes through LDS so that it and its mirror image are written in whole rows (the mirror entry
+// by entry, 64 KB apart, and the loads one round after another took 1015 us at l = 64, N = 128, 396
+// now, and 92 at l = 60, N = 32, 33 now).
+constexpr int kCongThreads = 512;
+
+template <int NP>
+__global__ __launch_bounds__(kCongThreads) void congruence_kernel(const double* __restrict__ G,
+                                                                 const double* __restrict__ T,
+                                                                 double* __restrict__ Bs, int64_t N,
+                                                                 int l) {
   extern __shared__ double smem[];
-  const int np = pad16(l), ld = np + 1, nb = np * ld;
-  double* sG = smem;
-  double* sTi = sG + nb;
-  double* sTj = sTi + nb;
-  double* sH = sTj + nb;
+  constexpr int LD = NP + 1, NB = NP * LD, NT = NP / 16, NW = kCongThreads / kWave;
+  constexpr int E = (NP * NP + kCongThreads - 1) / kCongThreads;
+  double* sG = smem;  // then the result
+  double* sTi = sG + NB;
+  double* sTj = sTi + NB;
+  double* sH = sTj + NB;
   const int64_t nl = N * l;
   // block pair p -> (I, J), I >= J, p = I (I + 1) / 2 + J
   const int64_t p = blockIdx.x;
@@ -135,34 +143,49 @@ __global__ __launch_bounds__(256) void congruence_kernel(const double* __restric
   while (I * (I + 1) / 2 > p) --I;
   while ((I + 1) * (I + 2) / 2 <= p) ++I;
   const int64_t J = p - I * (I + 1) / 2;
-  const int ll = l * l;
-  for (int e = threadIdx.x; e < np * np; e += blockDim.x) {
-    const int a = e / np, b = e % np;
+  const int tid = threadIdx.x;
+  const double* g = G + I * l * nl + J * l;
+  const double* ti = T + I * l * l;
+  const double* tj = T + J * l * l;
+  double v[3][E];
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const int e = tid + u * kCongThreads, a = e / NP, b = e % NP;
     const bool in = a < l && b < l;
-    sG[a * ld + b] = in ? G[(I * l + a) * nl + J * l + b] : 0.0;
-    sTi[a * ld + b] = in ? T[I * ll + a * l + b] : 0.0;
-    sTj[a * ld + b] = in ? T[J * ll + a * l + b] : 0.0;
+    v[0][u] = in ? g[a * nl + b] : 0.0;
+    v[1][u] = in ? ti[a * l + b] : 0.0;
+    v[2][u] = in ? tj[a * l + b] : 0.0;
+  }
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const int e = tid + u * kCongThreads, a = e / NP, b = e % NP;
+    if (a >= NP) break;
+    sG[a * LD + b] = v[0][u];
+    sTi[a * LD + b] = v[1][u];
+    sTj[a * LD + b] = v[2][u];
   }
   __syncthreads();
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int nt1 = np / 16, tiles = nt1 * nt1, nw = blockDim.x / kWave;
-  for (int t = wave; t < tiles; t += nw) {  // H = G_IJ T_J
-    const int i0 = (t / nt1) * 16, j0 = (t % nt1) * 16;
-    const d4 acc = lds_mfma_tile<false, false>(np, ld, sG, sTj, i0, j0);
+  const int wave = tid / kWave, lane = tid % kWave;
+  for (int t = wave; t < NT * NT; t += NW) {  // H = G_IJ T_J
+    const int i0 = (t / NT) * 16, j0 = (t % NT) * 16;
+    const d4 acc = lds_mfma_tile<false, false>(NP, LD, sG, sTj, i0, j0);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sH[(i0 + lane / 16 + 4 * r) * ld + j0 + lane % 16] = acc[r];
+    for (int r = 0; r < 4; ++r) sH[(i0 + lane / 16 + 4 * r) * LD + j0 + lane % 16] = acc[r];
   }
   __syncthreads();
-  for (int t = wave; t < tiles; t += nw) {  // T_I' H
-    const int i0 = (t / nt1) * 16, j0 = (t % nt1) * 16;
-    const d4 acc = lds_mfma_tile<true, false>(np, ld, sTi, sH, i0, j0);
+  for (int t = wave; t < NT * NT; t += NW) {  // T_I' H
+    const int i0 = (t / NT) * 16, j0 = (t % NT) * 16;
+    const d4 acc = lds_mfma_tile<true, false>(NP, LD, sTi, sH, i0, j0);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int r = i0 + lane / 16 + 4 * q, c = j0 + lane % 16;
-      if (r >= l || c >= l || (I == J && r < c)) continue;
-      Bs[(I * l + r) * nl + J * l + c] = acc[q];
-      Bs[(J * l + c) * nl + I * l + r] = acc[q];
-    }
+    for (int r = 0; r < 4; ++r) sG[(i0 + lane / 16 + 4 * r) * LD + j0 + lane % 16] = acc[r];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const int e = tid + u * kCongThreads, a = e / NP, b = e % NP;
+    if (a >= l || b >= l) continue;
+    Bs[(I * l + a) * nl + J * l + b] = sG[I == J && a < b ? b * LD + a : a * LD + b];
+    if (I != J) Bs[(J * l + a) * nl + I * l + b] = sG[b * LD + a];
   }
 }
 
@@ -397,9 +420,16 @@ void congruence_blockdiag(const double* G, const double* Tst, double* Bs, int64_
   MCNLA_REQUIRE(l >= 1 && l <= kMaxL, MCNLA_ERR_INVALID, "l > 64");
   const int64_t pairs = N * (N + 1) / 2;
   if (pairs == 0) return;
-  const size_t lds = static_cast<size_t>(4) * pad16(l) * (pad16(l) + 1) * sizeof(double);
-  hipLaunchKernelGGL(congruence_kernel, dim3(static_cast<unsigned>(pairs)), dim3(256), lds, st, G,
-                     Tst, Bs, N, l);
+  const int np = pad16(l);
+  const size_t lds = static_cast<size_t>(4) * np * (np + 1) * sizeof(double);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(pairs)), dim3(kCongThreads), lds, st, G,
+                       Tst, Bs, N, l);
+  };
+  if (np == 16) go(congruence_kernel<16>);
+  else if (np == 32) go(congruence_kernel<32>);
+  else if (np == 48) go(congruence_kernel<48>);
+  else go(congruence_kernel<64>);
   MCNLA_LAUNCHED();
 }
 
