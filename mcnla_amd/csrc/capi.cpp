@@ -1178,6 +1178,8 @@ void SolveRes::create() {
     MCNLA_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
     MCNLA_HIP(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
     MCNLA_HIP(hipEventCreateWithFlags(&join, hipEventDisableTiming));
+    MCNLA_HIP(hipEventCreateWithFlags(&enter, hipEventDisableTiming));
+    MCNLA_HIP(hipEventCreateWithFlags(&leave, hipEventDisableTiming));
     for (auto& e : marks) MCNLA_HIP(hipEventCreate(&e));
     for (hipEvent_t* e : {&sketch_beg, &sketch_end, &gram_beg, &gram_end, &former_beg, &former_end})
       MCNLA_HIP(hipEventCreate(e));
@@ -1195,7 +1197,7 @@ void SolveRes::create() {
 
 void SolveRes::destroy() {
   for (hipEvent_t* e :
-       {&fork, &join, &sketch_beg, &sketch_end, &gram_beg, &gram_end, &former_beg, &former_end})
+       {&fork, &join, &enter, &leave, &sketch_beg, &sketch_end, &gram_beg, &gram_end, &former_beg, &former_end})
     if (*e) (void)hipEventDestroy(*e), *e = nullptr;
   for (auto& e : marks)
     if (e) (void)hipEventDestroy(e), e = nullptr;
@@ -1515,9 +1517,35 @@ void solve_batch(int count, const mcnla_solver* solvers, const void* const* A, c
                     "a solver appears twice in the batch");
     check_a(solvers[i]->prm, A[i], lda[i], a_dtype[i], a_order[i]);
   }
+  // The members' sketches and orthogonalizers, and later their formers, each on its own side stream:
+  // they are chains of kernels of which many fill a few CUs only, the eigenproblems one (a batch of
+  // twelve 14.2 ms with all of them one after another on `st`, 12.1 with the formers on their own
+  // streams, 10.6 so).
   std::vector<SolveCtx> cx(count);
   for (int i = 0; i < count; ++i)
-    solve_begin(solvers[i], A[i], lda[i], a_dtype[i], a_order[i], st, cx[i], false);
+    if (!solvers[i]->res->ready()) solvers[i]->res->create();
+  auto fork = [&] { MCNLA_HIP(hipEventRecord(solvers[0]->res->enter, st)); };
+  auto enter = [&](int i) {
+    MCNLA_HIP(hipStreamWaitEvent(solvers[i]->res->side, solvers[0]->res->enter, 0));
+    return solvers[i]->res->side;
+  };
+  auto leave = [&](int i) {
+    MCNLA_HIP(hipEventRecord(solvers[i]->res->leave, solvers[i]->res->side));
+    MCNLA_HIP(hipStreamWaitEvent(st, solvers[i]->res->leave, 0));
+  };
+  struct Settle {  // after an error nothing may still run where `st` does not wait for it
+    int count;
+    const mcnla_solver* solvers;
+    bool done = false;
+    ~Settle() {
+      for (int i = 0; !done && i < count; ++i) (void)hipStreamSynchronize(solvers[i]->res->side);
+    }
+  } settle{count, solvers};
+  fork();
+  for (int i = 0; i < count; ++i) {
+    solve_begin(solvers[i], A[i], lda[i], a_dtype[i], a_order[i], enter(i), cx[i], false);
+    leave(i);
+  }
   // KN members in one group; the others one after another
   std::vector<GramIntegrator> group;
   std::vector<double*> coefs;
@@ -1551,21 +1579,15 @@ void solve_batch(int count, const mcnla_solver* solvers, const void* const* A, c
       cx[who[k]].ok = ok[k];
     }
   }
-  // Each member's former on its own side stream: its l x l eigenproblem is one workgroup for 60 to
-  // 200 us, and one after another on `st` a batch of twelve spent 1.4 of 13.7 ms in them alone.
   std::vector<int> bad(count, 0);
-  hipEvent_t fork = solvers[0]->res->fork;
-  MCNLA_HIP(hipEventRecord(fork, st));
-  for (int i = 0; i < count; ++i) {
-    hipStream_t side = solvers[i]->res->side;
-    MCNLA_HIP(hipStreamWaitEvent(side, fork, 0));
-    solve_finish(solvers[i], A[i], lda[i], a_dtype[i], a_order[i], side, cx[i], false);
-  }
+  fork();
+  for (int i = 0; i < count; ++i)
+    solve_finish(solvers[i], A[i], lda[i], a_dtype[i], a_order[i], enter(i), cx[i], false);
   for (int i = 0; i < count; ++i) {
     read_bad(solvers[i], &bad[i], solvers[i]->res->side);
-    MCNLA_HIP(hipEventRecord(solvers[i]->res->join, solvers[i]->res->side));
-    MCNLA_HIP(hipStreamWaitEvent(st, solvers[i]->res->join, 0));
+    leave(i);
   }
+  settle.done = true;
   MCNLA_HIP(hipStreamSynchronize(st));
   if (errors) errors->assign(count, std::string());
   std::string first_error;

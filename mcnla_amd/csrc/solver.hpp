@@ -50,6 +50,7 @@ struct SolveRes {
   static constexpr int kMarks = 5;  // start + one per stage
   hipStream_t side = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
+  hipEvent_t enter = nullptr, leave = nullptr;  // a batch member's work on `side`
   hipEvent_t marks[kMarks] = {};
   hipEvent_t sketch_beg = nullptr, sketch_end = nullptr, gram_beg = nullptr, gram_end = nullptr;
   hipEvent_t former_beg = nullptr, former_end = nullptr;
