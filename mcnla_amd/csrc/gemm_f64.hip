@@ -128,7 +128,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_f64_kernel(
   if (p.gate != nullptr && *p.gate < p.gate_t) return;
   // ---- tile schedule: logical id = (batch, split, tile), tile fastest -------------------------
   const int64_t tiles_m = ceil_div(p.M, BM), tiles_n = ceil_div(p.N, BN);
-  const int64_t ntiles = p.lower_only ? tiles_m * (tiles_m + 1) / 2 : tiles_m * tiles_n;
+  const int64_t ntiles = tiles_m * tiles_n;
   const int64_t nblocks = ntiles * p.splits * p.batch;
   const int64_t logical = xcd_swizzle(blockIdx.x, nblocks);
   const int64_t bat = logical / (ntiles * p.splits);
@@ -137,16 +137,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_f64_kernel(
 
   const TA* __restrict__ A = static_cast<const TA*>(p.A) + bat * p.stride_a;
   const TB* __restrict__ B = static_cast<const TB*>(p.B) + bat * p.stride_b;
-  int64_t tm, tn;
-  if (p.lower_only) {
-    tm = static_cast<int64_t>((sqrt(8.0 * static_cast<double>(t) + 1.0) - 1.0) * 0.5);
-    while (tm * (tm + 1) / 2 > t) --tm;
-    while ((tm + 1) * (tm + 2) / 2 <= t) ++tm;
-    tn = t - tm * (tm + 1) / 2;
-  } else {
-    tm = t / tiles_n;
-    tn = t % tiles_n;
-  }
+  const int64_t tm = t / tiles_n, tn = t % tiles_n;
   const int64_t m0 = tm * BM, n0 = tn * BN;
   const int64_t kbeg = split * p.kchunk;
   const int64_t kend = (kbeg + p.kchunk < p.K) ? kbeg + p.kchunk : p.K;
@@ -264,7 +255,10 @@ __global__ __launch_bounds__(WG* WG* WK * 64) void gemm_f64_wave_kernel(GemmF64A
   if (p.gate != nullptr && *p.gate < p.gate_t) return;
   const int64_t tiles_m = ceil_div(p.M, T), tiles_n = ceil_div(p.N, T);
   const int64_t ntiles = p.lower_only ? tiles_m * (tiles_m + 1) / 2 : tiles_m * tiles_n;
-  const int64_t logical = xcd_swizzle(blockIdx.x, ntiles * p.splits * p.batch);
+  const int64_t nblocks = ntiles * p.splits * p.batch;
+  const int64_t linear = blockIdx.y * static_cast<int64_t>(gridDim.x) + blockIdx.x;
+  if (linear >= nblocks) return;
+  const int64_t logical = xcd_swizzle(linear, nblocks);
   const int64_t bat = logical / (ntiles * p.splits);
   const int64_t split = (logical / ntiles) % p.splits, t = logical % ntiles;
   int64_t tm, tn;
@@ -1247,8 +1241,7 @@ template <typename TA, typename TB, bool A_MC, bool B_NC, int BM, int BN, int BK
 void launch_cfg(const GemmF64Args& p, hipStream_t st) {
   using Cfg = TileCfg<BM, BN, BK, WM, WN>;
   const int64_t tiles_m = ceil_div(p.M, BM), tiles_n = ceil_div(p.N, BN);
-  const int64_t ntiles = p.lower_only ? tiles_m * (tiles_m + 1) / 2 : tiles_m * tiles_n;
-  const int64_t nblocks = ntiles * p.splits * p.batch;
+  const int64_t nblocks = tiles_m * tiles_n * p.splits * p.batch;
   MCNLA_REQUIRE(nblocks < (1LL << 31), MCNLA_ERR_INVALID, "GEMM grid too large");
   // 16-byte loads need 16-byte aligned operands whose leading dimensions and batch strides are
   // multiples of the vector length.
@@ -1328,12 +1321,14 @@ template <typename TA, typename TB, bool A_MC, bool B_NC>
 void launch_wave(const GemmF64Args& p, int wg, hipStream_t st) {
   const int64_t nblocks = wave_blocks(p, wg, p.splits);
   MCNLA_REQUIRE(nblocks < (1LL << 31), MCNLA_ERR_INVALID, "GEMM grid too large");
+  const int64_t gx = std::min<int64_t>(nblocks, 1 << 22);  // a dimension holds < 2^32 threads
+  const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(ceil_div(nblocks, gx)));
   if (wg == 1)
-    hipLaunchKernelGGL((gemm_f64_wave_kernel<TA, TB, A_MC, B_NC, 1, 8>),
-                       dim3(static_cast<unsigned>(nblocks)), dim3(512), 0, st, p);
+    hipLaunchKernelGGL((gemm_f64_wave_kernel<TA, TB, A_MC, B_NC, 1, 8>), grid, dim3(512), 0, st,
+                       p);
   else
-    hipLaunchKernelGGL((gemm_f64_wave_kernel<TA, TB, A_MC, B_NC, 2, 2>),
-                       dim3(static_cast<unsigned>(nblocks)), dim3(512), 0, st, p);
+    hipLaunchKernelGGL((gemm_f64_wave_kernel<TA, TB, A_MC, B_NC, 2, 2>), grid, dim3(512), 0, st,
+                       p);
   MCNLA_LAUNCHED();
 }
 

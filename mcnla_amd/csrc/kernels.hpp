@@ -226,9 +226,9 @@ int64_t integrate_gram(const GramIntegrator& g, double* coef, hipStream_t st, bo
                        bool* numeric_ok);
 
 // KN integrations of up to kMaxKnGroup solves (wen_yin false; any N, l, tol, maxiter each) run in
-// lockstep on one stream: each iteration is one launch per kernel for the whole group (the
-// Bs product: one per tile-width class, l <= 32 and l > 32), and the host reads the group's
-// convergence flags once per chunk of iterations.  Member i's coefficients, iteration count and
+// lockstep on one stream: each iteration is one launch per kernel for the whole group (product and
+// update: one per class of l, up to 32, 48 and 64, and of rows per workgroup), and the host reads the
+// group's convergence flags once per chunk of iterations.  Member i's coefficients, iteration count and
 // flags are bit-identical to integrate_gram(gs[i]) alone.  `graphs` of the members are not used.
 void integrate_gram_group(const GramIntegrator* gs, double* const* coefs, int count,
                           hipStream_t st, int64_t* iterations, bool* converged, bool* numeric_ok);

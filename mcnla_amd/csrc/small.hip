@@ -1,4 +1,5 @@
 // Batched small-matrix kernels of the orthogonalizer and the formers (FP64).
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -138,7 +139,8 @@ __global__ __launch_bounds__(kCongThreads) void congruence_kernel(const double* 
   double* sH = sTj + NB;
   const int64_t nl = N * l;
   // block pair p -> (I, J), I >= J, p = I (I + 1) / 2 + J
-  const int64_t p = blockIdx.x;
+  const int64_t p = blockIdx.y * static_cast<int64_t>(gridDim.x) + blockIdx.x;
+  if (p >= N * (N + 1) / 2) return;
   int64_t I = static_cast<int64_t>((sqrt(8.0 * static_cast<double>(p) + 1.0) - 1.0) / 2.0);
   while (I * (I + 1) / 2 > p) --I;
   while ((I + 1) * (I + 2) / 2 <= p) ++I;
@@ -288,7 +290,9 @@ __global__ __launch_bounds__(256) void apply_blockdiag_kernel(T* __restrict__ Y,
   constexpr int LA = NP + 2, LB = NP + 16, NT = NP / 16;  // fragments on distinct banks
   __shared__ double sy[64 * LA];
   __shared__ double st[NP * LB];
-  const int64_t b = blockIdx.x % N, nl = N * l, first = blockIdx.x / N * kBdRows;
+  const int64_t blk = blockIdx.y * static_cast<int64_t>(gridDim.x) + blockIdx.x;
+  const int64_t b = blk % N, nl = N * l, first = blk / N * kBdRows;
+  if (first >= m) return;
   const int64_t r1 = first + kBdRows < m ? first + kBdRows : m;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, c = lane & 15,
             kq = lane >> 4;
@@ -422,9 +426,10 @@ void congruence_blockdiag(const double* G, const double* Tst, double* Bs, int64_
   if (pairs == 0) return;
   const int np = pad16(l);
   const size_t lds = static_cast<size_t>(4) * np * (np + 1) * sizeof(double);
+  const int64_t gx = std::min<int64_t>(pairs, 1 << 22);  // a dimension holds fewer than 2^32 threads
+  const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(ceil_div(pairs, gx)));
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(pairs)), dim3(kCongThreads), lds, st, G,
-                       Tst, Bs, N, l);
+    hipLaunchKernelGGL(kernel, grid, dim3(kCongThreads), lds, st, G, Tst, Bs, N, l);
   };
   if (np == 16) go(congruence_kernel<16>);
   else if (np == 32) go(congruence_kernel<32>);
@@ -469,7 +474,8 @@ void apply_blockdiag(void* Y, bool y_f32, int64_t m, int64_t N, int l, const dou
                      hipStream_t st) {
   MCNLA_REQUIRE(l <= kMaxL, MCNLA_ERR_INVALID, "l > 64");
   if (m <= 0 || N <= 0) return;
-  const dim3 grid(static_cast<unsigned>(ceil_div(m, kBdRows) * N));
+  const int64_t blocks = ceil_div(m, kBdRows) * N, gx = std::min<int64_t>(blocks, 1 << 22);
+  const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(ceil_div(blocks, gx)));
   auto launch = [&](auto* y) {
     using T = std::remove_pointer_t<decltype(y)>;
     auto go = [&](auto kernel) {

@@ -86,3 +86,21 @@ def test_solve_edges(k, p, N):
     assert abs(s.iteration() - iters) <= 1
     assert np.max(np.abs(s.vectorS() - S) / S) < 1e-9
     assert np.abs(U @ U.T - s.matrixU() @ s.matrixU().T).max() < 1e-8
+
+
+def test_solve_many_sketches():
+    """N = 4200 sketches of one column: 8.8 million block pairs in the congruence B_s = T'GT, more
+    workgroups of 512 than one grid dimension holds."""
+    m, n, N = 60, 40, 4200
+    rng = np.random.default_rng(8)
+    A = (basis(rng, m, n) * 0.7 ** np.arange(n)) @ basis(rng, n, n).T
+    om = oracle.omega_ref(3, n, N, col_block=True)
+    Q, _ = oracle.gramian_orthogonalize(oracle.sketch(A, om), 1, N)
+    Qb, iters = oracle.kn_rowblock(Q, 1, N, 256, 1e-4)
+    S, U, _ = oracle.svd_former(A, Qb, 1)
+    P = mc.Parameters().setSize(m, n).setRank(1).setOverRank(0).setNumSketch(N)
+    s = mc.Solver(P, seed=3, omega_mode=mc.OMEGA_REFERENCE, route=mc._lib.ROUTE_SKETCH)
+    s.solve(mc.DeviceArray.from_numpy(np.asfortranarray(A)))
+    assert abs(s.iteration() - iters) <= 1
+    assert np.max(np.abs(s.vectorS() - S) / S) < 1e-9
+    assert np.abs(U @ U.T - s.matrixU() @ s.matrixU().T).max() < 1e-8
