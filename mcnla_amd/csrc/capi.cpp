@@ -425,7 +425,8 @@ struct GramCore {
   int kern = 0;
   // Arguments of G = Y'Y except the pointers.
   GemmF64Args plan(bool y_f32, int64_t m, int64_t nl) const {
-    // Lower-triangle tiles: 256 x 128 on the FP64 fast path (tm (tm+1) tiles), else 128 x 128.
+    // Lower-triangle tiles: 256 x 128 on the FP64 fast path (tm (tm+1) tiles), else counted as 128
+    // x 128 (the register-fed tiles take fewer splits where that is cheaper).
     // Split K so that the grid fills whole rounds of about `target` workgroups.
     const int64_t tm = ceil_div(nl, 256), t = ceil_div(nl, 128);
     const int64_t tiles = (!y_f32 && nl >= 128 && kern == 0) ? tm * (tm + 1) : t * (t + 1) / 2;
