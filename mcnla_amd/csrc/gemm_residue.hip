@@ -63,9 +63,9 @@ constexpr u128 crt_weight(int i) {
   while ((m * w) % kP[i] != 1) ++w;
   return M * static_cast<u128>(w);
 }
-// The weights and P in two parts: multiples of 2^82, and the rest rounded to FP64.  With at most
-// kMaxRanges ranges, |sum r_i| <= 2^12 per modulus and the sum of the high parts is an integer
-// multiple of 2^82 below 2^134: exact in FP64.
+// The weights and P in two parts: multiples of 2^82, and the rest rounded to FP64.  |r_i| <= 2^7, so
+// the sum of the high parts is an integer multiple of 2^82 below 2^129: exact in FP64.  (The
+// residues of at most kMaxRanges ranges are added first, as integers below 2^12.)
 constexpr int kGrid = 82;
 constexpr int kMaxRanges = 32;
 constexpr double hi_part(u128 v) {
@@ -440,28 +440,52 @@ __global__ __launch_bounds__(256) void residue_gemm_kernel(
 }
 
 // ---- reconstruction ---------------------------------------------------------------------------
-// The sums of 4 consecutive columns from their residues: R points at modulus 0 of range 0.
+// The sums of 4 consecutive columns from their residues: R points at modulus 0 of range 0.  The
+// ranges' residues are added and reduced before the weights are applied, so that what the FP64
+// arithmetic sees is the residue of the whole sum in [-p/2, p/2], however K was cut (the GEMM
+// leaves that residue for one range; the two-part sums below are rounded, and would differ in
+// their last bits for other representatives).
 __device__ __forceinline__ void reconstruct4(const int8_t* __restrict__ R, int64_t plane,
                                              int ranges, double* out) {
-  double c1[4] = {0.0, 0.0, 0.0, 0.0}, c2[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int g = 0; g < ranges; ++g) {
-    const int8_t* Rg = R + g * kMods * plane;
-    uint32_t w[kMods];
+  int r[kMods][4];
 #pragma unroll
-    for (int m = 0; m < kMods; ++m) w[m] = *reinterpret_cast<const uint32_t*>(Rg + m * plane);
+  for (int m = 0; m < kMods; ++m) {
+    const uint32_t w = *reinterpret_cast<const uint32_t*>(R + m * plane);
 #pragma unroll
-    for (int m = 0; m < kMods; ++m)
+    for (int i = 0; i < 4; ++i) r[m][i] = static_cast<int8_t>(w >> (8 * i));
+  }
+  if (ranges > 1) {
+    for (int g = 1; g < ranges; ++g) {
+      const int8_t* Rg = R + g * kMods * plane;
+      uint32_t w[kMods];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const double r = static_cast<double>(static_cast<int8_t>(w[m] >> (8 * i)));
-        c1[i] = fma(r, kCrt.hi[m], c1[i]);
-        c2[i] = fma(r, kCrt.lo[m], c2[i]);
+      for (int m = 0; m < kMods; ++m) w[m] = *reinterpret_cast<const uint32_t*>(Rg + m * plane);
+#pragma unroll
+      for (int m = 0; m < kMods; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[m][i] += static_cast<int8_t>(w[m] >> (8 * i));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      r[0][i] = static_cast<int8_t>(r[0][i]);  // p = 256: -128, never 128, as the GEMM stores it
+#pragma unroll
+      for (int m = 1; m < kMods; ++m) {  // odd p: no ties, and |sum| / p < 2^5 is far from one
+        const float s = static_cast<float>(r[m][i]);
+        r[m][i] -= kP[m] * static_cast<int>(rintf(s * (1.0f / static_cast<float>(kP[m]))));
       }
+    }
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const double q = rint(c1[i] * kCrt.P_inv);
-    out[i] = fma(-q, kCrt.P_hi, c1[i]) + fma(-q, kCrt.P_lo, c2[i]);
+    double c1 = 0.0, c2 = 0.0;
+#pragma unroll
+    for (int m = 0; m < kMods; ++m) {
+      const double x = static_cast<double>(r[m][i]);
+      c1 = fma(x, kCrt.hi[m], c1);
+      c2 = fma(x, kCrt.lo[m], c2);
+    }
+    const double q = rint(c1 * kCrt.P_inv);
+    out[i] = fma(-q, kCrt.P_hi, c1) + fma(-q, kCrt.P_lo, c2);
   }
 }
 

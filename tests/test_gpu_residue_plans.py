@@ -1,0 +1,61 @@
+"""An FP64 product by residues gives the same bits however its rows and K are cut (gemm_residue.hip):
+workspaces of different sizes take other panels and other K ranges.  The operands are orthogonal to
+2^-20 of their norms, so that the sums are small beside the moduli's product: there the FP64
+arithmetic of the reconstruction would show which residues it was given."""
+import numpy as np
+import pytest
+
+import mcnla_amd as mc
+import residue
+
+pytestmark = pytest.mark.gpu
+
+
+def plans(a):
+    """Workspace sizes from the largest that is of use down, each of another plan."""
+    limit, out = 2 << 30, []
+    while len(out) < 8:
+        size = residue.workspace(a, limit)
+        if size == 0:
+            break
+        out.append(size)
+        limit = min(size - 1, int(0.85 * size))
+    return out
+
+
+@pytest.mark.parametrize("m,n,k,dtype,order", [
+    (700, 300, 6000, np.float64, "F"),
+    (700, 300, 6000, np.float32, "C"),
+    (1500, 333, 9001, np.float64, "C"),
+])
+def test_product_of_any_plan(m, n, k, dtype, order):
+    rng = np.random.default_rng(m + k)
+    A = rng.standard_normal((m, k)).astype(dtype)
+    q = np.linalg.qr(A.astype(np.float64).T)[0]
+    B = rng.standard_normal((k, n))
+    B = B - q @ (q.T @ B) + 2.0 ** -20 * rng.standard_normal((k, n))
+    dA = mc.DeviceArray.from_numpy(A, order=order)
+    dB = mc.DeviceArray.from_numpy(B, order="C")
+    sizes = plans(residue.args(dA, dB))
+    assert len(sizes) >= 3
+    results = [residue.product(dA, dB, size) for size in sizes]
+    assert all(flag == 0 for _, flag in results)
+    for c, _ in results[1:]:
+        np.testing.assert_array_equal(c, results[0][0])
+
+
+@pytest.mark.parametrize("m,k,dtype,order", [
+    (300, 60000, np.float64, "F"), (600, 20001, np.float32, "F"), (260, 9000, np.float64, "C"),
+])
+def test_symmetric_product_of_any_plan(m, k, dtype, order):
+    rng = np.random.default_rng(m + k)
+    q = np.linalg.qr(rng.standard_normal((k, m)))[0].T
+    A = (q + 2.0 ** -20 / np.sqrt(k) * rng.standard_normal((m, k))).astype(dtype)
+    dA = mc.DeviceArray.from_numpy(A, order=order)
+    sizes = plans(residue.args(dA))
+    assert len(sizes) >= 3
+    results = [residue.product(dA, limit=size) for size in sizes]
+    assert all(flag == 0 for _, flag in results)
+    for c, _ in results[1:]:
+        np.testing.assert_array_equal(c, results[0][0])
+    np.testing.assert_array_equal(results[0][0], results[0][0].T)
