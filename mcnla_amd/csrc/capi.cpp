@@ -11,6 +11,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "pending.hpp"
 #include "solver.hpp"
 
 namespace mcnla {
@@ -1534,14 +1535,10 @@ void solve_batch(int count, const mcnla_solver* solvers, const void* const* A, c
     MCNLA_HIP(hipEventRecord(solvers[i]->res->leave, solvers[i]->res->side));
     MCNLA_HIP(hipStreamWaitEvent(st, solvers[i]->res->leave, 0));
   };
-  struct Settle {  // after an error nothing may still run where `st` does not wait for it
-    int count;
-    const mcnla_solver* solvers;
-    bool done = false;
-    ~Settle() {
-      for (int i = 0; !done && i < count; ++i) (void)hipStreamSynchronize(solvers[i]->res->side);
-    }
-  } settle{count, solvers};
+  // the members' hazard flags; after an error nothing may still run where `st` does not wait for it
+  PendingInts bad(count, [&] {
+    for (int i = 0; i < count; ++i) (void)hipStreamSynchronize(solvers[i]->res->side);
+  });
   fork();
   for (int i = 0; i < count; ++i) {
     solve_begin(solvers[i], A[i], lda[i], a_dtype[i], a_order[i], enter(i), cx[i], false);
@@ -1580,16 +1577,15 @@ void solve_batch(int count, const mcnla_solver* solvers, const void* const* A, c
       cx[who[k]].ok = ok[k];
     }
   }
-  std::vector<int> bad(count, 0);
   fork();
   for (int i = 0; i < count; ++i)
     solve_finish(solvers[i], A[i], lda[i], a_dtype[i], a_order[i], enter(i), cx[i], false);
   for (int i = 0; i < count; ++i) {
-    read_bad(solvers[i], &bad[i], solvers[i]->res->side);
+    read_bad(solvers[i], bad.at(i), solvers[i]->res->side);
     leave(i);
   }
-  settle.done = true;
   MCNLA_HIP(hipStreamSynchronize(st));
+  bad.landed();
   if (errors) errors->assign(count, std::string());
   std::string first_error;
   for (int i = 0; i < count; ++i) {
