@@ -133,6 +133,13 @@ struct DevBuf {
     }
     bytes = n;
   }
+  // Makes this n bytes of another buffer, which outlives it; 0: empty.
+  void view(void* at, size_t n) {
+    if (p && !borrowed) (void)hipFree(p);
+    p = at;
+    bytes = n;
+    borrowed = n > 0;
+  }
   template <class T>
   T* as() const {
     return static_cast<T*>(p);
@@ -245,7 +252,7 @@ struct ResidueScratch {
   size_t bytes = 0, limit = 0;
   int* flag = nullptr;
 };
-// The most workspace taken for the sake of speed alone: the larger plans measured 2 % faster.
+// The most workspace a sketcher stage takes.
 constexpr size_t kResidueBytes = size_t{2} << 30;
 
 // Y = A * Omega with Omega generated into `omega` (n x Nl FP64).
@@ -285,10 +292,27 @@ struct SketchCore {
     r.ldc = r.N;
     return r;
   }
-  // Allocates Omega and, for a mixed precision, the BF16 panels of A and Omega.
-  void prepare(const mcnla_params& p, int precision) {
+  // The rows past the whole rounds of the DMA-tiled FP64 sketch's grid, their split of K, and its
+  // partials (gemm_f64_dma_tail); no rows: none.
+  struct Tail {
+    int64_t rows = 0, splits = 1, kchunk = 0;
+    size_t bytes = 0;
+  };
+  static Tail f64_tail(const mcnla_params& p) {
+    const int64_t nl = (p.rank + p.over_rank) * p.num_sketch;
+    Tail t;
+    int64_t ts = 1;
+    const int64_t main = gemm_f64_dma_tail(p.nrow, nl, p.ncol, &ts);
+    if (ts <= 1) return t;
+    t.rows = p.nrow - main;
+    t.kchunk = ceil_div(ceil_div(p.ncol, ts), 16) * 16;
+    t.splits = ceil_div(p.ncol, t.kchunk);
+    t.bytes = gemm_f64_partial_elems(t.rows, nl, t.splits) * sizeof(double);
+    return t;
+  }
+  // Allocates Omega.
+  void prepare(const mcnla_params& p) {
     omega.ensure(p.ncol * (p.rank + p.over_rank) * p.num_sketch * sizeof(double));
-    if (precision != MCNLA_PREC_F64) ws.ensure(sketch_bf16_workspace(bf16_args(p, precision)));
   }
   void generate(const mcnla_params& p, uint64_t seed, int mode, int threads, bool col_block,
                 hipStream_t st) {
@@ -346,21 +370,19 @@ struct SketchCore {
       // run a few full-length workgroups on a mostly idle device: 6256 tiles at 100000 x 10000,
       // Nl = 2048, are 24 rounds and 112 tiles).  Not for a solver carved from a reserved
       // region, which may not allocate the partials.
-      int64_t ts = 1;
-      const int64_t main = (g.a_mcontig && !g.a_f32 && !omega.borrowed)
-                               ? gemm_f64_dma_tail(g.M, g.N, g.K, &ts)
-                               : g.M;
+      Tail tl;
+      if (g.a_mcontig && !g.a_f32 && !omega.borrowed) tl = f64_tail(p);
       MCNLA_HIP(hipEventRecord(gemm_beg, st));
-      if (ts > 1) {
+      if (tl.rows > 0) {
         GemmF64Args t = g;
-        t.M = p.nrow - main;
-        t.A = static_cast<const double*>(A) + main;
-        t.C = static_cast<double*>(Y) + main * nl;
-        t.kchunk = ceil_div(ceil_div(g.K, ts), 16) * 16;
-        t.splits = ceil_div(g.K, t.kchunk);
-        tail.ensure(gemm_f64_partial_elems(t.M, t.N, t.splits) * sizeof(double));
+        g.M = p.nrow - tl.rows;
+        t.M = tl.rows;
+        t.A = static_cast<const double*>(A) + g.M;
+        t.C = static_cast<double*>(Y) + g.M * nl;
+        t.kchunk = tl.kchunk;
+        t.splits = tl.splits;
+        tail.ensure(tl.bytes);
         t.partial = tail.as<double>();
-        g.M = main;
         gemm_f64(g, st);
         gemm_f64(t, st);
       } else {
@@ -467,17 +489,15 @@ struct GramCore {
   size_t partial_bytes(bool y_f32, int64_t m, int64_t nl) const {
     return gemm_f64_partial_elems(nl, nl, plan(y_f32, m, nl).splits) * sizeof(double);
   }
-  // Allocates the partials; with more memory than a reserved region holds, at least `more` bytes.
-  void prepare(int64_t m, int64_t nl, size_t more) {
-    const size_t need = partial_bytes(false, m, nl);
-    if (more > need && more > partial.bytes) {
-      try {
-        partial.ensure(more);
-      } catch (const Error& e) {
-        if (e.code != MCNLA_ERR_NOMEM) throw;
-      }
+  // Grows the partials' buffer by `more` bytes where the memory is there.
+  void grow(size_t more) {
+    const size_t had = partial.bytes;
+    try {
+      partial.ensure(had + more);
+    } catch (const Error& e) {
+      if (e.code != MCNLA_ERR_NOMEM) throw;
+      partial.ensure(had);
     }
-    partial.ensure(need);
   }
   bool by_residues(int64_t m, int64_t nl) const {
     return kern == 0 && residue_pays(residue_args(nullptr, false, m, nl, nullptr),
@@ -1074,23 +1094,19 @@ void apply_tuning(mcnla_solver_s* s, const mcnla_tuning& t) {
                            gemm_f64_partial_elems(n, l, n_by_l_splits(n, nl, t.n_by_l)),
                            gemm_f64_partial_elems(n, l, n_by_l_splits(n, n, t.n_by_l))}) *
                  sizeof(double));
-  // the products by residues (Gram, and an FP64 sketch before it) work in the partials' buffer:
-  // give them the workspace of their best plans where memory is not reserved by the byte
-  size_t more = 0;
-  const int64_t gn = via_a ? n : nl;
-  if (current_carve() == nullptr && !s->gram.partial.borrowed) {
-    if (s->gram.by_residues(m, gn))
-      more = residue_bytes(GramCore::residue_args(nullptr, false, m, gn, nullptr), kResidueBytes);
-    const ResidueArgs r = SketchCore::residue_args(s->prm, nullptr, m, MCNLA_F64, MCNLA_COL_MAJOR,
-                                                   nullptr, nullptr);
-    if (!via_a && s->cfg.precision == MCNLA_PREC_F64 &&
-        residue_pays(r, s->gram.partial_bytes(false, m, nl)))
-      more = std::max(more, residue_bytes(r, kResidueBytes));
+  size_t part = s->gram.partial_bytes(false, m, via_a ? n : nl), packed = 0;
+  if (!via_a) {  // the Qbar product's split-K partials reuse the Gram's (free by then)
+    part = std::max(part, gemm_f64_partial_elems(m, l, qbar_splits(m, nl, t.qbar)) *
+                              sizeof(double));
+    if (is_mixed(s->cfg.precision))
+      packed = sketch_bf16_workspace(SketchCore::bf16_args(s->prm, s->cfg.precision));
   }
-  s->gram.prepare(m, gn, more);
-  if (!via_a)  // the Qbar product's split-K partials reuse the Gram's (free by then)
-    s->gram.partial.ensure(gemm_f64_partial_elems(m, l, qbar_splits(m, nl, t.qbar)) *
-                           sizeof(double));
+  // A 16-bit sketch's packed operands follow the partials in one buffer: they are done with when
+  // the Gram starts, and a Gram by residues works in all of it.
+  part = align_up(part, kCarveAlign);
+  s->sketch.ws.view(nullptr, 0);  // should the buffer not be had
+  s->gram.partial.ensure(part + packed);
+  if (packed) s->sketch.ws.view(s->gram.partial.as<char>() + part, packed);
   s->form.prepare(s->prm);
 }
 
@@ -1147,7 +1163,17 @@ std::unique_ptr<mcnla_solver_s> new_solver(const mcnla_params* params,
   s->L0.ensure(l * l * sizeof(double));
   s->T0.ensure(l * l * sizeof(double));
   s->W0.ensure(l * l * sizeof(double));
-  s->sketch.prepare(*params, via_a ? static_cast<int>(MCNLA_PREC_F64) : cfg->precision);
+  s->sketch.prepare(*params);
+  if (current_carve() == nullptr && !via_a && cfg->precision == MCNLA_PREC_F64) {
+    // An FP64 sketch by residues works in the Gram's partials.  A solver with its own memory adds
+    // what the sketch on the FP64 tiles would take for its tail, and now leaves alone: 100000 x
+    // 10000, Nl = 2048 runs in panels of 4352 rows instead of 2048 so (45.0 -> 43.5 ms a solve).
+    const SketchCore::Tail t = SketchCore::f64_tail(*params);
+    if (t.rows > 0 && residue_pays(SketchCore::residue_args(*params, nullptr, m, MCNLA_F64,
+                                                            MCNLA_COL_MAJOR, nullptr, nullptr),
+                                   s->gram.partial_bytes(false, m, nl)))
+      s->gram.grow(t.bytes);
+  }
   return s;
 }
 }  // namespace
@@ -1266,11 +1292,9 @@ void solve_sketch(mcnla_solver_s* s, const void* A, int64_t lda, int a_dtype, in
 // Stage 2: G = Y'Y (or Omega'(H Omega)), the per-block transforms T and Bs = T'GT.
 void solve_orthogonalize(mcnla_solver_s* s, hipStream_t st, SolveCtx& cx) {
   const auto& p = s->prm;
-  const auto& c = s->cfg;
   const int l = static_cast<int>(p.rank + p.over_rank);
   const int64_t N = p.num_sketch, nl = l * N, m = p.nrow, n = p.ncol;
   const bool via_a = s->route == MCNLA_ROUTE_GRAM_OF_A;
-  (void)c;
   // 2. orthogonalize through the Gram matrix: G = Y'Y, T_i from G_ii, Bs = T' G T.  The
   // reference's T_i = V_i S_i^{-1/2} (eig of G_ii) needs a Jacobi eigen-solve per block; for
   // the KN and WY integrators, which are equivariant in the basis of the first sketch (Qbar
@@ -2145,11 +2169,12 @@ mcnla_status mcnla_solver_workspace_bytes(mcnla_solver s, size_t* bytes) {
     size_t b = 0;
     for (const DevBuf* d : {&s->Y, &s->A64, &s->H, &s->P, &s->X, &s->gp, &s->L0, &s->T0, &s->W0,
                             &s->G, &s->W, &s->w, &s->V, &s->T, &s->Bs, &s->tmp, &s->ws,
-                            &s->coef, &s->M2, &s->Qbar, &s->bad, &s->sketch.omega, &s->sketch.ws, &s->sketch.tail,
+                            &s->coef, &s->M2, &s->Qbar, &s->bad, &s->sketch.omega, &s->sketch.tail,
                             &s->gram.partial, &s->form.Z, &s->form.partial, &s->form.Wg,
                             &s->form.eigw, &s->form.eigv, &s->form.Wk, &s->form.S, &s->form.U,
                             &s->form.V})
       b += d->bytes;
+    if (!s->sketch.ws.borrowed) b += s->sketch.ws.bytes;  // else part of gram.partial
     *bytes = b;
     return MCNLA_OK;
   });

@@ -628,7 +628,8 @@ constexpr int64_t kMaxK = 1 << 17;  // |sum| <= 2^14 K < 2^31 (2^31 = 0 mod 256)
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
 // How a product is cut into panels: M panels of `rows` with the whole K (general), or K panels
-// (symmetric), each multiplied in `ranges` K ranges of kper steps.
+// (symmetric), each multiplied in `ranges` K ranges of kper steps.  The norms' partials lie where the
+// first product's residues go: the exponents are made before it.
 struct Plan {
   int64_t rows = 0, kpanel = 0, panels = 0, steps = 0, ranges = 0, kper = 0;
   size_t off_part = 0, off_ea = 0, off_eb = 0, off_b = 0, off_a = 0, off_r = 0, bytes = 0;
@@ -670,8 +671,6 @@ Plan plan_general(const ResidueArgs& a, int64_t cus, int64_t tm, int64_t ranges)
   p.cost = (p.panels - 1) * p.cost + kPanel * p.panels +
            grid_cost(cus, last * tn * kMods * p.ranges, p.kper);
   size_t o = 0;
-  p.off_part = o;
-  o += align256(16 * std::max(norm_pairs(A, a.M, a.K), norm_pairs(B, a.N, a.K)));
   p.off_ea = o;
   o += align256(4 * a.M);
   p.off_eb = o;
@@ -680,8 +679,9 @@ Plan plan_general(const ResidueArgs& a, int64_t cus, int64_t tm, int64_t ranges)
   o += static_cast<size_t>(kMods) * tn * p.steps * kBlk;
   p.off_a = o;
   o += static_cast<size_t>(kMods) * tm * p.steps * kBlk;
-  p.off_r = o;
-  o += static_cast<size_t>(p.ranges) * kMods * p.rows * tn * kBR;
+  p.off_r = p.off_part = o;
+  o += std::max(align256(16 * std::max(norm_pairs(A, a.M, a.K), norm_pairs(B, a.N, a.K))),
+                static_cast<size_t>(p.ranges) * kMods * p.rows * tn * kBR);
   p.bytes = o;
   return p;
 }
@@ -697,14 +697,13 @@ Plan plan_sym(const ResidueArgs& a, int64_t cus, int64_t panels, int64_t ranges)
   if (!set_ranges(p, cus, tm * (tm + 1) / 2, ranges)) return Plan{};
   p.cost = p.panels * (p.cost + kPanel);
   size_t o = 0;
-  p.off_part = o;
-  o += align256(16 * norm_pairs(A, a.M, a.K));
   p.off_ea = o;
   o += align256(4 * a.M);
   p.off_a = o;
   o += static_cast<size_t>(kMods) * tm * p.steps * kBlk;
-  p.off_r = o;
-  o += static_cast<size_t>(p.ranges) * kMods * p.rows * p.rows;
+  p.off_r = p.off_part = o;
+  o += std::max(align256(16 * norm_pairs(A, a.M, a.K)),
+                static_cast<size_t>(p.ranges) * kMods * p.rows * p.rows);
   p.bytes = o;
   return p;
 }

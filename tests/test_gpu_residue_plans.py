@@ -2,6 +2,8 @@
 workspaces of different sizes take other panels and other K ranges.  The operands are orthogonal to
 2^-20 of their norms, so that the sums are small beside the moduli's product: there the FP64
 arithmetic of the reconstruction would show which residues it was given."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -59,3 +61,24 @@ def test_symmetric_product_of_any_plan(m, k, dtype, order):
     for c, _ in results[1:]:
         np.testing.assert_array_equal(c, results[0][0])
     np.testing.assert_array_equal(results[0][0], results[0][0].T)
+
+
+@pytest.mark.parametrize("precision,route", [
+    (mc.PREC_F64, mc.ROUTE_SKETCH), (mc.PREC_MIXED_BF16, mc.ROUTE_SKETCH),
+    (mc.PREC_F64, mc.ROUTE_GRAM_OF_A),
+])
+def test_solver_holds_what_it_reports(precision, route):
+    """A solver's products by residues work in memory it has anyway: it holds what required_bytes
+    says, and on the FP64 sketch route at most the partials that a sketch on the FP64 tiles would
+    take for its last rows."""
+    m, n, k, p, N = 60000, 3000, 20, 12, 48
+    P = mc.Parameters().setSize(m, n).setRank(k).setOverRank(p).setNumSketch(N)
+    s = mc.Solver(P, precision=precision, route=route)
+    tail = 0
+    if precision == mc.PREC_F64 and route == mc.ROUTE_SKETCH:
+        splits = ctypes.c_int64()
+        main = residue.function("gemm_f64_dma_tail", ctypes.c_int64, *[ctypes.c_int64] * 3,
+                                ctypes.c_void_p)(m, (k + p) * N, n, ctypes.byref(splits))
+        tail = 8 * (m - main) * (k + p) * N * splits.value
+    required = mc.required_bytes(m, n, k, p, N, precision=precision, route=route)
+    assert s.workspace_bytes() <= required + tail
