@@ -358,9 +358,9 @@ mcnla_status mcnla_solve_static(const mcnla_params* params, const mcnla_solver_c
  * count or tile shape changes only the order of the sums, so a tuned plan gives the same results
  * to rounding, and the same plan always gives the same bits.
  *
- * Large FP64 sketches and Gram matrices run by residues on the INT8 cores instead (the `gram`
- * target then only sizes their workspace; kernels bit 1 keeps the Gram on the FP64 tiles); their
- * results do not depend on the plan.
+ * Large FP64 sketches and Gram matrices run by residues on the INT8 cores instead, by the shape of
+ * the problem alone; the targets change neither that nor their results (a `gram` target above the
+ * default enlarges their workspace).  kernels bit 1 keeps the Gram on the FP64 tiles.
  *
  * Tuned plans are kept in a process-wide table keyed by (route, precision, m, n, l, N); a solver
  * created after an entry exists for its key uses it (servers too, per request shape). */

@@ -244,9 +244,9 @@ GemmShape tall_shape(int64_t ncols) {
 // Shared pipeline pieces.
 
 // Workspace lent to an FP64 product that may run by residues (gemm_residue.hip).  Whether it does
-// is decided on `limit` bytes, the part every solver of the shape has, so that it does not depend
-// on where the solver lives; `bytes` (>= limit) is what is there.  flag: the product's device
-// flag, outside ws.  A null flag: no workspace.
+// is decided on `limit` bytes, a function of the problem's shape alone, so that it depends neither
+// on where a solver lives nor on its tuned plan; `bytes` (>= limit) is what is there, and changes
+// the time only.  flag: the product's device flag, outside ws.  A null flag: no workspace.
 struct ResidueScratch {
   void* ws = nullptr;
   size_t bytes = 0, limit = 0;
@@ -259,6 +259,7 @@ constexpr size_t kResidueBytes = size_t{2} << 30;
 struct SketchCore {
   DevBuf omega, ws;
   DevBuf tail;  // split-K partials of the sketch's last rows (allocated on first use)
+  bool ran_by_residues = false;  // the last projection
   std::vector<double> host;
   hipEvent_t gemm_beg = nullptr, gemm_end = nullptr;
   bool own_ev = true;     // false: the events belong to a SolveRes
@@ -354,8 +355,8 @@ struct SketchCore {
       g.ldc = nl;
       g.shape = GemmShape::kSquare;
       const ResidueArgs ra = residue_args(p, A, lda, dtype, order, omega.as<double>(), Y);
-      const bool by_residues = scratch.flag != nullptr && residue_pays(ra, scratch.limit);
-      if (by_residues) {
+      ran_by_residues = scratch.flag != nullptr && residue_pays(ra, scratch.limit);
+      if (ran_by_residues) {
         MCNLA_HIP(hipEventRecord(gemm_beg, st));
         gemm_residue(ra, scratch.ws, scratch.bytes, scratch.flag, st);
         g.gate = scratch.flag;  // rows without a scale: the FP64 product after all
@@ -446,6 +447,7 @@ struct GramCore {
   // workgroups the split-K grid aims at (about 9 per CU by default), and the kernel (tile shape)
   int64_t target = kDefaultTuning.gram;
   int kern = 0;
+  bool ran_by_residues = false;  // the last product
   // Arguments of G = Y'Y except the pointers.
   GemmF64Args plan(bool y_f32, int64_t m, int64_t nl) const {
     // Lower-triangle tiles: 256 x 128 on the FP64 fast path (tm (tm+1) tiles), else counted as 128
@@ -485,6 +487,11 @@ struct GramCore {
     r.ldc = nl;
     return r;
   }
+  // The workspace that decides whether this product, and an FP64 sketch before it, run by residues:
+  // the partials of the default plan, which every solver of the shape has, whatever its own.
+  static size_t residue_limit(int64_t m, int64_t nl) {
+    return GramCore().partial_bytes(false, m, nl);
+  }
   // Bytes of the FP64 product's split-K partials.
   size_t partial_bytes(bool y_f32, int64_t m, int64_t nl) const {
     return gemm_f64_partial_elems(nl, nl, plan(y_f32, m, nl).splits) * sizeof(double);
@@ -501,7 +508,7 @@ struct GramCore {
   }
   bool by_residues(int64_t m, int64_t nl) const {
     return kern == 0 && residue_pays(residue_args(nullptr, false, m, nl, nullptr),
-                                     partial_bytes(false, m, nl));
+                                     residue_limit(m, nl));
   }
   // Y has leading dimension ld.  A product by residues works in `ws` if that is the larger buffer,
   // or in that of the partials (flag: its device flag).
@@ -513,7 +520,9 @@ struct GramCore {
     }
     const bool residues = by_residues(m, nl);
     GemmF64Args g = plan(y_f32 && !residues, m, nl);
-    partial.ensure(gemm_f64_partial_elems(nl, nl, g.splits) * sizeof(double));
+    partial.ensure(std::max(gemm_f64_partial_elems(nl, nl, g.splits) * sizeof(double),
+                            residues ? residue_limit(m, nl) : 0));
+    ran_by_residues = residues;
     g.a_f32 = y_f32;
     g.b_f32 = y_f32;
     g.lda = ld;
@@ -1094,7 +1103,9 @@ void apply_tuning(mcnla_solver_s* s, const mcnla_tuning& t) {
                            gemm_f64_partial_elems(n, l, n_by_l_splits(n, nl, t.n_by_l)),
                            gemm_f64_partial_elems(n, l, n_by_l_splits(n, n, t.n_by_l))}) *
                  sizeof(double));
-  size_t part = s->gram.partial_bytes(false, m, via_a ? n : nl), packed = 0;
+  const int64_t gn = via_a ? n : nl;
+  size_t part = std::max(s->gram.partial_bytes(false, m, gn), GramCore::residue_limit(m, gn));
+  size_t packed = 0;
   if (!via_a) {  // the Qbar product's split-K partials reuse the Gram's (free by then)
     part = std::max(part, gemm_f64_partial_elems(m, l, qbar_splits(m, nl, t.qbar)) *
                               sizeof(double));
@@ -1171,7 +1182,7 @@ std::unique_ptr<mcnla_solver_s> new_solver(const mcnla_params* params,
     const SketchCore::Tail t = SketchCore::f64_tail(*params);
     if (t.rows > 0 && residue_pays(SketchCore::residue_args(*params, nullptr, m, MCNLA_F64,
                                                             MCNLA_COL_MAJOR, nullptr, nullptr),
-                                   s->gram.partial_bytes(false, m, nl)))
+                                   GramCore::residue_limit(m, nl)))
       s->gram.grow(t.bytes);
   }
   return s;
@@ -1266,7 +1277,7 @@ void solve_sketch(mcnla_solver_s* s, const void* A, int64_t lda, int a_dtype, in
     if (c.precision == MCNLA_PREC_F64) {
       scratch.ws = s->gram.partial.p;
       scratch.bytes = s->gram.partial.bytes;
-      scratch.limit = s->gram.partial_bytes(false, m, nl);
+      scratch.limit = GramCore::residue_limit(m, nl);
       scratch.flag = s->bad.as<int>() + mcnla_solver_s::kSketchFlag;
     }
     s->sketch.project(p, c.precision, A, lda, a_dtype, a_order, s->Y.p, st, true, scratch);
@@ -1519,6 +1530,15 @@ GramIntegrator solver_kn_integrator(mcnla_solver s) {
 }
 
 double* solver_coef(mcnla_solver s) { return s->coef.as<double>(); }
+
+void solver_products_by_residues(mcnla_solver s, bool* sketch, bool* gram) {
+  *sketch = s->sketch.ran_by_residues;
+  *gram = s->gram.ran_by_residues;
+}
+
+bool sketcher_by_residues(mcnla_stage s) {
+  return s->type == mcnla_stage_s::kSketcher && static_cast<Sketcher*>(s)->core.ran_by_residues;
+}
 
 void solver_set_integration(mcnla_solver s, int64_t iterations, bool converged) {
   s->iteration = iterations;
@@ -2418,10 +2438,7 @@ mcnla_status mcnla_solver_autotune(mcnla_solver s, const void* A, int64_t lda, i
                {&mcnla_tuning::omega_p, {256, 512, 1024, 2048}, 2u, kKernOmegaP},
                {&mcnla_tuning::n_by_l, {128, 256, 512, 1024, 2048}, 12u, kKernNbyL}};
     } else {
-      // the Gram's partials are also where an FP64 sketch by residues works: their size decides
-      // whether it does (at 100000 x 10000 the sketch takes 57 instead of 34 ms with 576)
-      const unsigned gram_stages = s->cfg.precision == MCNLA_PREC_F64 ? 3u : 2u;
-      knobs = {{&mcnla_tuning::gram, {576, 1152, 2304, 4608, 9216}, gram_stages, kKernGram},
+      knobs = {{&mcnla_tuning::gram, {576, 1152, 2304, 4608, 9216}, 2u, kKernGram},
                {&mcnla_tuning::former, {1024, 2048, 4096, 8192}, 8u, kKernFormer},
                {&mcnla_tuning::qbar, {512, 1024, 2048, 3072, 4096}, 4u, kKernQbar}};
     }

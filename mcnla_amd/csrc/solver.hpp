@@ -101,6 +101,11 @@ GramIntegrator solver_kn_integrator(mcnla_solver s);
 double* solver_coef(mcnla_solver s);
 void solver_set_integration(mcnla_solver s, int64_t iterations, bool converged);
 
+// Whether the last solve's sketch and Gram matrix, or the last run of a sketcher stage, were FP64
+// products by residues (gemm_residue.hip).
+void solver_products_by_residues(mcnla_solver s, bool* sketch, bool* gram);
+bool sketcher_by_residues(mcnla_stage s);
+
 // The batch solve of mcnla_solver_solve_batch on stream `st` (synchronized on return); with
 // `errors`, member i's error text (empty when status[i] is OK).  Throws Error for invalid
 // arguments (before anything is enqueued) or a HIP failure.

@@ -70,3 +70,16 @@ def product(A, B=None, limit=2 << 30):
              ctypes.c_void_p, ctypes.c_void_p)(ctypes.byref(a), ws.ptr, size, flag.ptr, None)
     mc.synchronize()
     return C.numpy(), int(flag.numpy().view(np.int32)[0])
+
+
+def solver_paths(solver):
+    """(sketch, Gram): whether the last solve's products ran by residues."""
+    s, g = ctypes.c_bool(), ctypes.c_bool()
+    function("solver_products_by_residues", None, ctypes.c_void_p, ctypes.c_void_p,
+             ctypes.c_void_p)(solver._h, ctypes.byref(s), ctypes.byref(g))
+    return s.value, g.value
+
+
+def sketcher_path(stage):
+    """Whether the last run of this sketcher was by residues."""
+    return function("sketcher_by_residues", ctypes.c_bool, ctypes.c_void_p)(stage._h)

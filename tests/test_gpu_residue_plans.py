@@ -82,3 +82,31 @@ def test_solver_holds_what_it_reports(precision, route):
         tail = 8 * (m - main) * (k + p) * N * splits.value
     required = mc.required_bytes(m, n, k, p, N, precision=precision, route=route)
     assert s.workspace_bytes() <= required + tail
+
+
+@pytest.fixture
+def untuned():
+    mc.tune_clear()
+    yield
+    mc.tune_clear()
+
+
+def test_tuned_plan_keeps_the_route(untuned):
+    """The Gram's split target changes neither the route of an FP64 sketch and its Gram nor a bit
+    of the results: with 576 its partials alone could not hold the sketch's packed Omega."""
+    m, n, k, p, N = 6000, 9000, 20, 12, 50
+    rng = np.random.default_rng(8)
+    a = (rng.standard_normal((m, 60)) * 0.95 ** np.arange(60)) @ rng.standard_normal((60, n))
+    a += 1e-3 * rng.standard_normal((m, n))
+    A = mc.DeviceArray.from_numpy(a, order="F")
+    P = mc.Parameters().setSize(m, n).setRank(k).setOverRank(p).setNumSketch(N)
+    out = []
+    for gram in (2304, 576, 9216):
+        mc.tune_set(P, dict(mc.tuning_default(), gram=gram))
+        s = mc.Solver(P, seed=9)
+        s.solve(A)
+        assert residue.solver_paths(s) == (True, True)
+        out.append((s.vectorS(), s.matrixU(), s.matrixV(), s.matrixQbar()))
+    for other in out[1:]:
+        for x, y in zip(out[0], other):
+            np.testing.assert_array_equal(x, y)
