@@ -141,7 +141,10 @@ mcnla_status mcnla_sketcher_create(const mcnla_params* params, int kind, int pre
  * of the reference run whose stream should be reproduced (REFERENCE mode only). */
 mcnla_status mcnla_sketcher_set_seed(mcnla_stage s, uint64_t seed, int omega_mode, int threads);
 /* Y = A * Omega.  A: m x n (a_dtype, a_order, lda).  Y: row-major m x (N*l), FP64 for
- * MCNLA_PREC_F64, FP32 for the mixed precisions. */
+ * MCNLA_PREC_F64, FP32 for the mixed precisions.  A large FP64 sketch runs by residues on the INT8
+ * cores: the first such run takes a workspace of at most 2 GiB and an eighth of the free memory,
+ * which the sketcher keeps.  Its size does not change Y; without memory for any, this sketcher
+ * stays on the FP64 kernels, whose Y differs by rounding. */
 mcnla_status mcnla_sketcher_run(mcnla_stage s, const void* A, int64_t lda, int a_dtype,
                                 int a_order, void* Y, void* stream);
 /* setExponent (gaussian_projection_sketcher.hh:87): q power iterations after Y = A Omega,

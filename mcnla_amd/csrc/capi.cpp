@@ -245,14 +245,15 @@ GemmShape tall_shape(int64_t ncols) {
 
 // Workspace lent to an FP64 product that may run by residues (gemm_residue.hip).  Whether it does
 // is decided on `limit` bytes, a function of the problem's shape alone, so that it depends neither
-// on where a solver lives nor on its tuned plan; `bytes` (>= limit) is what is there, and changes
-// the time only.  flag: the product's device flag, outside ws.  A null flag: no workspace.
+// on where a solver lives nor on its tuned plan; `bytes` is what is there (enough for one of the
+// product's plans), and changes the time only.  flag: the product's device flag, outside ws.  A null flag: no workspace.
 struct ResidueScratch {
   void* ws = nullptr;
   size_t bytes = 0, limit = 0;
   int* flag = nullptr;
 };
-// The most workspace a sketcher stage takes.
+// The most workspace a sketcher stage takes, and what its route is decided on: it holds no Gram
+// partials that it could work in.
 constexpr size_t kResidueBytes = size_t{2} << 30;
 
 // Y = A * Omega with Omega generated into `omega` (n x Nl FP64).
@@ -733,22 +734,32 @@ struct Sketcher : mcnla_stage_s {
   int64_t exponent = 0;
   SketchCore core;
   DevBuf residue;                  // flag and workspace of the FP64 sketch by residues
+  bool no_residue = false;         // there was no memory for it
   DevBuf idx, partial;             // column-sampling indices; split-K partials of A'Y
   std::vector<int64_t> host_idx;
   Sketcher() : mcnla_stage_s(kSketcher) {}
-  // The workspace of an FP64 sketch of this A by residues, taken on the first run; none when the
-  // FP64 kernels are faster or the memory is not there.
+  // The workspace of an FP64 sketch of this A by residues, taken on the first run: at most an eighth
+  // of the memory that is free then (a smaller one changes the time, not the result).  None when
+  // the FP64 kernels are faster, or once there was no memory for any.
   ResidueScratch scratch(const void* A, int64_t lda, int dtype, int order, void* Y) {
-    if (precision != MCNLA_PREC_F64) return {};
+    if (precision != MCNLA_PREC_F64 || no_residue) return {};
     const ResidueArgs r =
         SketchCore::residue_args(prm, A, lda, dtype, order, core.omega.as<double>(), Y);
     if (!residue_pays(r, kResidueBytes)) return {};
-    const size_t need = residue_bytes(r, kResidueBytes);
-    try {
-      residue.ensure(kCarveAlign + need);
-    } catch (const Error& e) {
-      if (e.code != MCNLA_ERR_NOMEM) throw;
-      return {};
+    if (residue.bytes <= kCarveAlign || residue_bytes(r, residue.bytes - kCarveAlign) == 0) {
+      size_t avail = 0, total = 0;
+      MCNLA_HIP(hipMemGetInfo(&avail, &total));
+      size_t need = residue_bytes(r, std::min(kResidueBytes, avail / 8));
+      for (; need != 0; need = residue_bytes(r, need / 2)) {
+        try {
+          residue.ensure(kCarveAlign + need);
+          break;
+        } catch (const Error& e) {
+          if (e.code != MCNLA_ERR_NOMEM) throw;
+        }
+      }
+      no_residue = need == 0;
+      if (no_residue) return {};
     }
     ResidueScratch s;
     s.flag = residue.as<int>();

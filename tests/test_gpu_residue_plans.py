@@ -110,3 +110,32 @@ def test_tuned_plan_keeps_the_route(untuned):
     for other in out[1:]:
         for x, y in zip(out[0], other):
             np.testing.assert_array_equal(x, y)
+
+
+def test_sketcher_with_little_memory():
+    """A sketcher stage takes at most an eighth of the free memory for its residue workspace, and
+    gives the same bits in a smaller one."""
+    m, n, l, N = 4001, 4099, 41, 25
+    A = mc.DeviceArray.from_numpy(np.random.default_rng(4).standard_normal((m, n)), order="F")
+    P = mc.Parameters().setSize(m, n).setRank(l).setOverRank(0).setNumSketch(N)
+
+    def sketch():
+        s = mc.ColBlockGaussianProjectionSketcher(P, seed=3).initialize()
+        before = mc.mem_info()[0]
+        s(A, Q)
+        mc.synchronize()
+        assert residue.sketcher_path(s)
+        return Q.numpy(), before, before - mc.mem_info()[0]
+    Q = P.createCollectionQ()
+    y, _, taken = sketch()
+    assert taken > 400 << 20
+    held, left = [], 5 << 29
+    try:
+        while (free := mc.mem_info()[0]) > left + (64 << 20):
+            held.append(mc.DeviceArray((min(free - left, 16 << 30) // 8,)))
+        z, before, taken = sketch()
+    finally:
+        for x in held:
+            x.free()
+    assert taken <= before // 8 + (4 << 20)
+    np.testing.assert_array_equal(y, z)
