@@ -212,3 +212,35 @@ def test_gram_of_a_with_a_column_without_a_scale(scale, order):
         assert np.max(np.abs(out[0][1] - out[1][1]) / out[1][1]) < 1e-10
     else:
         assert out[0][0] != 0
+
+
+@pytest.mark.parametrize("kind", ["lognormal", "cauchy", "outliers"])
+def test_gram_of_a_with_spread_columns(kind):
+    """Columns whose entries spread over many orders of magnitude: the residue product holds the
+    small ones to fewer bits than FP64 does, and bounds the error of an entry of A'A by the two
+    columns' norms alone.  Sigma takes no harm: either product's error is below m 2^-53 of the
+    columns' norms, so sigma_j differs by at most m 2^-53 (||A||_F / sigma_j)^2 of itself."""
+    m, n, k, N = 40000, 1200, 20, 40
+    rng = np.random.default_rng(7)
+    if kind == "lognormal":
+        a = np.exp(3 * rng.standard_normal((m, n))) * rng.choice([-1.0, 1.0], (m, n))
+    elif kind == "cauchy":
+        a = rng.standard_normal((m, n)) / rng.standard_normal((m, n))
+    else:
+        a = rng.standard_normal((m, n))
+        a[rng.permutation(m)[:n], np.arange(n)] = 1e8 * 0.9 ** np.arange(n) + 1e3
+    A = mc.DeviceArray.from_numpy(a, order="C")
+    P = mc.Parameters().setSize(m, n).setRank(k).setOverRank(10).setNumSketch(N)
+    out = []
+    try:
+        for kernels in (0, 1):
+            mc.tune_clear()
+            mc.tune_set(P, dict(mc.tuning_default(), kernels=kernels), route=mc.ROUTE_GRAM_OF_A)
+            s = mc.Solver(P, seed=9, route=mc.ROUTE_GRAM_OF_A)
+            s.solve(A)
+            assert residue.solver_paths(s)[1] == (kernels == 0)
+            out.append(s.vectorS())
+    finally:
+        mc.tune_clear()
+    bound = m * 2.0 ** -53 * (np.linalg.norm(a) / out[1]) ** 2
+    assert np.all(np.abs(out[0] - out[1]) <= bound * out[1])
