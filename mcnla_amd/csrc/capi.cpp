@@ -638,7 +638,6 @@ struct FormCore {
     w.ldb = l;
     w.C = Wg.as<double>();
     w.ldc = l;
-    w.shape = GemmShape::kSmall;
     w.kchunk = w_kchunk(n);
     w.splits = ceil_div(n, w.kchunk);
     z.partial = partial.as<double>();
@@ -687,7 +686,6 @@ struct FormCore {
       u.b_ncontig = false;
       u.C = U.as<double>();
       u.ldc = m;
-      u.shape = (k <= 32) ? GemmShape::kWideM32 : GemmShape::kSquare;
     } else {
       u.M = m;
       u.N = k;
@@ -899,7 +897,6 @@ int orthogonalize_inplace(Orthogonalizer& o, void* Qs, hipStream_t st) {
   g.b_f32 = f32;
   g.C = o.W.as<double>();
   g.ldc = l;
-  g.shape = (l <= 32) ? GemmShape::kSmall : GemmShape::kSquare;
   g.batch = N;
   g.stride_a = l;
   g.stride_b = l;
@@ -1394,7 +1391,6 @@ void solve_finish(mcnla_solver_s* s, const void* A, int64_t lda, int a_dtype, in
     wr.ldb = l;
     wr.C = s->W0.as<double>();
     wr.ldc = l;
-    wr.shape = GemmShape::kSmall;
     gemm_f64(wr, st);
     GemmF64Args cr;  // coef W_0 (Nl x l) into the scratch
     cr.M = nl;
@@ -1422,7 +1418,6 @@ void solve_finish(mcnla_solver_s* s, const void* A, int64_t lda, int a_dtype, in
   tm.ldb = l;
   tm.C = s->M2.as<double>();
   tm.ldc = l;
-  tm.shape = GemmShape::kSmall;
   tm.batch = N;
   tm.stride_a = static_cast<int64_t>(l) * l;
   tm.stride_b = static_cast<int64_t>(l) * l;

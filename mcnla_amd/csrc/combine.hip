@@ -197,7 +197,6 @@ int64_t small_splits(int64_t batch, int64_t K) { return gemm_f64_splits_for(batc
 // Batched l x l products P_b = op(A_b) B_b with K = Nl rows, split over K.
 void small_products(GemmF64Args g, int64_t batch, double* partial, hipStream_t st) {
   g.batch = batch;
-  g.shape = g.M <= 32 ? GemmShape::kSmall : GemmShape::kSquare;
   g.splits = small_splits(batch, g.K);
   g.kchunk = ceil_div(ceil_div(g.K, g.splits), 16) * 16;
   g.splits = ceil_div(g.K, g.kchunk);

@@ -8,9 +8,15 @@
 //   Gram          G  = Y' * Y           both operands are rows of Y: M- and N-contiguous
 //   basis         Qb = Y * M            Y row-major (K-contiguous), M row-major
 //   former        Z  = A' * Qbar        A col-major (K-contiguous) / row-major (M-contiguous)
-// Tiles are staged through LDS as [k][mn] (mn contiguous) so that every MFMA operand fragment is
-// one LDS row segment; v_mfma_f64_16x16x4f64 does the arithmetic.  Source elements may be FP32
-// (mixed precision collections); they are widened to FP64 on the way into LDS.
+// Four kinds of kernel, chosen in gemm_f64 by shape, types and alignment, all on
+// v_mfma_f64_16x16x4f64 (or FP32 MFMA where a mixed precision asks for it); FP32 operands are
+// widened on their way:
+//   DMA tiles      256 x 128 and 256 x 64, aligned FP64 operands along M and N, LDS filled by
+//                  global_load_lds: large sketches, Gram matrices, the integrators' Bs products
+//   tall kernels   N <= 64 with A along K (tall_direct.hpp, tall_stream_kernel, tall_kernel) and
+//                  the LDS-staged 128 x 32 / 64 tiles ([k][mn], mn contiguous) for A along M
+//   wave tiles     32 x 32 or 64 x 64 from cache straight into MFMA registers: everything else
+// (gemm_residue.hip takes the largest FP64 sketches and Gram matrices away from these.)
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -1295,11 +1301,11 @@ struct WavePlan {
   double cost = 0.0;
 };
 
-// The cheaper form of the wave kernel, and of the split-K factors up to p.splits (where the sums
-// are taken here) the cheapest, a partial written and read at 3 TB/s.
+// The cheaper form of the wave kernel, and the cheapest of the split-K factors up to p.splits, a
+// partial written and read at 3 TB/s.
 WavePlan wave_plan(const GemmF64Args& p) {
   WavePlan best;
-  const int64_t lo = p.splits > 1 && p.partial != nullptr && p.C != nullptr ? 1 : p.splits;
+  const int64_t lo = p.splits > 1 && p.partial != nullptr ? 1 : p.splits;
   for (int64_t s = p.splits; s >= lo; s = s > 1 ? std::max<int64_t>(s * 3 / 4, 1) : 0) {
     const int64_t chunk = s == p.splits ? p.kchunk : ceil_div(p.K, s);
     const int64_t kchunk = std::max<int64_t>(ceil_div(chunk, 16) * 16, 16);
@@ -1377,11 +1383,10 @@ void gemm_f64(GemmF64Args p, hipStream_t st) {
   // The wave kernel takes every product but the tall ones and those large enough for the DMA
   // tiles; of the tall ones that tall_* cannot take (A along M), it takes those of fewer 128-row
   // tiles than CUs (2000 x 20 x 2000 in 8 splits: 28 -> 16 us; in 512 tiles, 1999 x 31 x 12347, the
-  // shared B of the larger ones wins, 57 against 71 us).  Partials that the caller sums (C null)
-  // keep their split and, where they had it, the DMA kernel.
+  // shared B of the larger ones wins, 57 against 71 us).
   const bool tall_tiles = p.shape == GemmShape::kTallN32 || p.shape == GemmShape::kTallN64;
   WavePlan wave;
-  if (!tall && !(dma && p.C == nullptr) &&
+  if (!tall &&
       !(tall_tiles && ceil_div(p.M, 128) * ceil_div(p.N, p.shape == GemmShape::kTallN32 ? 32 : 64) *
                               p.splits * p.batch >= device_cus())) {
     wave = wave_plan(p);
@@ -1417,7 +1422,7 @@ void gemm_f64(GemmF64Args p, hipStream_t st) {
   else if (!dma)
     p.kchunk = ceil_div(p.kchunk, 16) * 16;
   if (p.K > 0) p.splits = ceil_div(p.K, p.kchunk);
-  if (p.splits == 1 && !p.lower_only && p.C != nullptr) p.partial = nullptr;
+  if (p.splits == 1 && !p.lower_only) p.partial = nullptr;
   MCNLA_REQUIRE(!(p.splits > 1 && p.partial == nullptr), MCNLA_ERR_INVALID,
                 "split-K GEMM needs a partial buffer");
   MCNLA_REQUIRE(!p.lower_only || p.M == p.N, MCNLA_ERR_INVALID, "lower_only needs M == N");
@@ -1484,7 +1489,7 @@ void gemm_f64(GemmF64Args p, hipStream_t st) {
     else launch_types<double, double>(p, wave.wg, st);
   }
   if (p.ev_end) MCNLA_HIP(hipEventRecord(p.ev_end, st));
-  if (p.partial != nullptr && p.C != nullptr && p.lower_only) {
+  if (p.partial != nullptr && p.lower_only) {
     const int64_t T = ceil_div(p.N, 64);
     MCNLA_REQUIRE(T * (T + 1) / 2 < (1LL << 31) && p.batch < 65536, MCNLA_ERR_INVALID,
                   "GEMM grid too large");
@@ -1493,7 +1498,7 @@ void gemm_f64(GemmF64Args p, hipStream_t st) {
                        dim3(1024), 0, st, p.partial, p.splits, p.N, p.alpha, p.beta, p.C, p.ldc,
                        p.stride_c, p.gate, p.gate_t);
     MCNLA_LAUNCHED();
-  } else if (p.partial != nullptr && p.C != nullptr) {
+  } else if (p.partial != nullptr) {
     const int64_t total = p.M * p.N * p.batch;
     const int threads = 256;
     int64_t blocks = ceil_div(total, threads);

@@ -1785,8 +1785,8 @@ IterationGraphs::~IterationGraphs() {
 
 namespace {
 
-// Bout = Bs * Bin / N (Bout null: only the split-K partials into L.Pbg), gated on t, through the
-// GEMM dispatch (the Wen-Yin iterations and the final polish).
+// Bout = Bs * Bin / N, gated on t, through the GEMM dispatch (the Wen-Yin iterations and the final
+// polish).
 void bs_product(const GramIntegrator& g, const Layout& L, const double* Bin, double* Bout, int t,
                 hipStream_t st) {
   const int64_t nl = L.nl;

@@ -10,7 +10,8 @@ namespace mcnla {
 
 // ------------------------------------------------------------------------------------------------
 // FP64 MFMA GEMM (gemm_f64.hip).
-enum class GemmShape { kSquare, kTallN32, kTallN64, kWideM32, kSmall };
+// kTallN32 / kTallN64: N <= 32 / 64 and many rows; kSquare: any other product.
+enum class GemmShape { kSquare, kTallN32, kTallN64 };
 
 struct GemmF64Args {
   int64_t M = 0, N = 0, K = 0;
@@ -25,7 +26,7 @@ struct GemmF64Args {
   // Tall FP32-A products only: FP32 MFMA (B rounded to FP32, FP32 sums within a split, FP64
   // across splits) instead of FP64 arithmetic.  Other shapes ignore it.
   bool f32_mfma = false;
-  double* C = nullptr;      // row-major, ldc; may be null when only partials are wanted
+  double* C = nullptr;      // row-major, ldc
   int64_t ldc = 0;
   double alpha = 1.0, beta = 0.0;
   int64_t splits = 1;       // split-K factor (requires `partial`)
