@@ -24,8 +24,8 @@
 // 30011 x 840 x 2503 3.39 -> 2.0 ms, 2048^2 x 100000 (symmetric) 6.7 -> 4.4 ms.
 //
 // Rows with a non-finite entry, or whose norm leaves [2^-400, 2^400], have no such scale: the
-// scale kernels raise a device flag, and the caller's FP64 product, launched behind it and gated
-// on the flag, replaces the result.
+// scale kernels raise a device flag, at which everything after them ends at once, and the caller's
+// FP64 product, launched behind it and gated on the flag, makes the result.
 #include <algorithm>
 #include <cmath>
 
@@ -220,7 +220,8 @@ __global__ __launch_bounds__(256) void exponent_kernel(const double2* __restrict
 template <typename TS, bool R_CONTIG>
 __global__ __launch_bounds__(256) void pack_residues_kernel(
     const TS* __restrict__ src, int64_t ld, int64_t rows, int64_t K, int64_t steps, int64_t tiles,
-    const int* __restrict__ exps, uint8_t* __restrict__ dst) {
+    const int* __restrict__ exps, const int* __restrict__ flag, uint8_t* __restrict__ dst) {
+  if (*flag != 0) return;
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int64_t kt = R_CONTIG ? blockIdx.y : blockIdx.x;
   const int64_t strip = (R_CONTIG ? blockIdx.x : blockIdx.y) * 4ll + wave;  // 16 rows
@@ -303,8 +304,9 @@ __device__ __forceinline__ void mfma_i8(i32x4& acc, const u32x4& a, const u32x4&
 __global__ __launch_bounds__(256) void residue_gemm_kernel(
     const uint8_t* __restrict__ Ab, const uint8_t* __restrict__ Bb, int64_t tiles_m,
     int64_t tiles_n, int64_t steps, int64_t kper, bool accumulate, bool sym, int64_t ldr,
-    int64_t plane, int8_t* __restrict__ R) {
+    int64_t plane, const int* __restrict__ flag, int8_t* __restrict__ R) {
   constexpr int L = 8;  // DMA instructions per wave and stage (4 per operand)
+  const int no_scale = *flag;  // looked at once the first stages are on their way
   __shared__ __attribute__((aligned(16))) uint8_t S0[2 * kBlk], S1[2 * kBlk], S2[2 * kBlk],
       S3[2 * kBlk], S4[2 * kBlk];
   const int64_t ntiles = sym ? tiles_m * (tiles_m + 1) / 2 : tiles_m * tiles_n;
@@ -392,6 +394,10 @@ __global__ __launch_bounds__(256) void residue_gemm_kernel(
   issue(kbeg + 2, S2);
   issue(kbeg + 3, S3);
   asm volatile("" ::: "memory");
+  if (no_scale != 0) {
+    wait_vmcnt<0>();
+    return;
+  }
   wait_vmcnt<3 * L>();  // stage 0 landed in every wave
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
@@ -495,7 +501,9 @@ __global__ __launch_bounds__(256) void reconstruct_kernel(const int8_t* __restri
                                                           int64_t plane, int ranges, int64_t rows,
                                                           int64_t N, const int* __restrict__ ea,
                                                           const int* __restrict__ eb,
+                                                          const int* __restrict__ flag,
                                                           double* __restrict__ C, int64_t ldc) {
+  if (*flag != 0) return;
   const int64_t quads = ceil_div(N, 4), total = rows * quads;
   for (int64_t t = blockIdx.x * 256ll + threadIdx.x; t < total; t += gridDim.x * 256ll) {
     const int64_t i = t / quads, j = (t % quads) * 4;
@@ -514,9 +522,11 @@ __global__ __launch_bounds__(256) void reconstruct_sym_kernel(const int8_t* __re
                                                               int64_t ldr, int64_t plane,
                                                               int ranges, int64_t N,
                                                               const int* __restrict__ e,
+                                                              const int* __restrict__ flag,
                                                               double* __restrict__ C,
                                                               int64_t ldc) {
   __shared__ double t[64][65];
+  if (*flag != 0) return;
   const int64_t x = blockIdx.x;
   int64_t ti = static_cast<int64_t>((sqrt(8.0 * static_cast<double>(x) + 1.0) - 1.0) / 2.0);
   while (ti * (ti + 1) / 2 > x) --ti;
@@ -600,27 +610,27 @@ void scales(const Operand& o, int64_t r0, int64_t rows, int64_t K, double2* part
 
 template <typename TS>
 void launch_pack(const Operand& o, const void* src, int64_t rows, int64_t K, int64_t steps,
-                 int64_t tiles, const int* e, uint8_t* dst, hipStream_t st) {
+                 int64_t tiles, const int* e, const int* flag, uint8_t* dst, hipStream_t st) {
   const unsigned strips = static_cast<unsigned>(tiles * (kBR / 64));
   const TS* s = static_cast<const TS*>(src);
   if (o.rcontig)
     hipLaunchKernelGGL((pack_residues_kernel<TS, true>),
                        dim3(strips, static_cast<unsigned>(steps)), dim3(256), 0, st, s, o.ld, rows,
-                       K, steps, tiles, e, dst);
+                       K, steps, tiles, e, flag, dst);
   else
     hipLaunchKernelGGL((pack_residues_kernel<TS, false>),
                        dim3(static_cast<unsigned>(steps), strips), dim3(256), 0, st, s, o.ld, rows,
-                       K, steps, tiles, e, dst);
+                       K, steps, tiles, e, flag, dst);
   MCNLA_LAUNCHED();
 }
 
 void pack(const Operand& o, int64_t r0, int64_t rows, int64_t k0, int64_t K, int64_t steps,
-          int64_t tiles, const int* e, uint8_t* dst, hipStream_t st) {
+          int64_t tiles, const int* e, const int* flag, uint8_t* dst, hipStream_t st) {
   const void* src = o.at(r0, k0);
   if (o.f32)
-    launch_pack<float>(o, src, rows, K, steps, tiles, e, dst, st);
+    launch_pack<float>(o, src, rows, K, steps, tiles, e, flag, dst, st);
   else
-    launch_pack<double>(o, src, rows, K, steps, tiles, e, dst, st);
+    launch_pack<double>(o, src, rows, K, steps, tiles, e, flag, dst, st);
 }
 
 constexpr int64_t kMaxK = 1 << 17;  // |sum| <= 2^14 K < 2^31 (2^31 = 0 mod 256)
@@ -815,7 +825,7 @@ void gemm_residue(const ResidueArgs& a, void* ws, size_t ws_bytes, int* flag, hi
     const int64_t blocks = tiles * kMods * p.ranges;
     MCNLA_REQUIRE(blocks < (1LL << 31), MCNLA_ERR_INVALID, "GEMM grid too large");
     hipLaunchKernelGGL(residue_gemm_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st,
-                       pa, pb, tm, tn, p.steps, p.kper, accumulate, a.sym, ldr, plane, R);
+                       pa, pb, tm, tn, p.steps, p.kper, accumulate, a.sym, ldr, plane, flag, R);
     MCNLA_LAUNCHED();
   };
   if (a.sym) {
@@ -824,13 +834,13 @@ void gemm_residue(const ResidueArgs& a, void* ws, size_t ws_bytes, int* flag, hi
     const int64_t plane = p.rows * p.rows;
     for (int64_t q = 0; q < p.panels; ++q) {
       const int64_t k0 = q * p.kpanel, kn = std::min(p.kpanel, a.K - k0);
-      pack(A, 0, a.M, k0, kn, p.steps, tm, ea, pa, st);
+      pack(A, 0, a.M, k0, kn, p.steps, tm, ea, flag, pa, st);
       gemm(pa, tm, tm, q > 0, p.rows, plane);
     }
     const int64_t T = ceil_div(a.M, 64);
     hipLaunchKernelGGL(reconstruct_sym_kernel, dim3(static_cast<unsigned>(T * (T + 1) / 2)),
                        dim3(256), 0, st, R, p.rows, plane, static_cast<int>(p.ranges),
-                       a.M, ea, a.C, a.ldc);
+                       a.M, ea, flag, a.C, a.ldc);
     MCNLA_LAUNCHED();
     return;
   }
@@ -839,17 +849,17 @@ void gemm_residue(const ResidueArgs& a, void* ws, size_t ws_bytes, int* flag, hi
   uint8_t* pb = reinterpret_cast<uint8_t*>(w + p.off_b);
   const int64_t tn = ceil_div(a.N, kBR);
   scales(B, 0, a.N, a.K, part, eb, flag, st);
-  pack(B, 0, a.N, 0, a.K, p.steps, tn, eb, pb, st);
   scales(A, 0, a.M, a.K, part, ea, flag, st);
+  pack(B, 0, a.N, 0, a.K, p.steps, tn, eb, flag, pb, st);
   for (int64_t r0 = 0; r0 < a.M; r0 += p.rows) {
     const int64_t rows = std::min(p.rows, a.M - r0), tm = ceil_div(rows, kBR);
-    pack(A, r0, rows, 0, a.K, p.steps, tm, ea + r0, pa, st);
+    pack(A, r0, rows, 0, a.K, p.steps, tm, ea + r0, flag, pa, st);
     const int64_t ldr = tn * kBR, plane = tm * kBR * ldr;
     gemm(pb, tm, tn, false, ldr, plane);
     const int64_t quads = rows * ceil_div(a.N, 4);
     const int64_t blocks = std::min<int64_t>(ceil_div(quads, 256), 16384);
     hipLaunchKernelGGL(reconstruct_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st,
-                       R, ldr, plane, static_cast<int>(p.ranges), rows, a.N, ea + r0, eb,
+                       R, ldr, plane, static_cast<int>(p.ranges), rows, a.N, ea + r0, eb, flag,
                        a.C + r0 * a.ldc, a.ldc);
     MCNLA_LAUNCHED();
   }

@@ -82,8 +82,8 @@ size_t residue_bytes(const ResidueArgs& a, size_t limit, double* cost = nullptr)
 // of `limit` bytes.
 bool residue_pays(const ResidueArgs& a, size_t limit);
 // Enqueues the product.  *flag (device) ends nonzero when an operand has a row without a scale (a
-// non-finite entry, or a norm out of range): C is undefined then, and the caller replaces it by
-// an FP64 product gated on the flag (gate_t = 1).  `ws` is 256-byte aligned.
+// non-finite entry, or a norm out of range): C is not written then, and the caller makes it by an
+// FP64 product gated on the flag (gate_t = 1).  `ws` is 256-byte aligned.
 void gemm_residue(const ResidueArgs& a, void* ws, size_t ws_bytes, int* flag, hipStream_t st);
 // Compute units of the current device (cached per device).
 int compute_units();

@@ -106,11 +106,13 @@ def test_flag(value, scaled, order):
             line *= value
         else:
             line[k - 1] = value
-        _, flag = residue.product(device(a, order), device(b, "C"))
+        c, flag = residue.product(device(a, order), device(b, "C"))
         assert (flag == 0) == scaled, (which, at)
+        assert np.all(np.isnan(c)) != scaled  # nothing is written behind a raised flag
         if which == 0:
-            _, flag = residue.product(device(a, order))
+            c, flag = residue.product(device(a, order))
             assert (flag == 0) == scaled, at
+            assert np.all(np.isnan(c)) != scaled
 
 
 def sketch(A, order, N, l, pad=0):
