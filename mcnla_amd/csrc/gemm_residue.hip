@@ -20,6 +20,17 @@
 // 2.7e-16 against 1.5e-15 (K = 2503), 1.5e-16 against 7e-16 (K = 700); symmetric (squares on the
 // diagonal) 6.9e-15 against 8.6e-14 (K = 100000).
 //
+// The error is bounded by the two rows' norms -- at most 1.7 units of 2^-53 ||a_i|| ||b_j||
+// measured on any data, where sums in FP64 had 54 to 2200 -- and not entry by entry by |A||B|: an
+// entry 2^-j below its row's largest keeps about 53 - j bits.  Where the large entries of two rows
+// lie at different places that is less than FP64 sums give.  In units of 2^-53 |A||B|, residues
+// against FP64 sums: Gaussian rows 0.8 / 54, Y = A Omega of the matrices in perf/cases.py 0.8-2 /
+// 130-500, but A'A for columns with lognormal(3) entries 3.8e3 / 104, Cauchy 1.5e4 / 170, a lone
+// 1e8 in each column 4e8 / 2e3.  What a solve computes from such an A'A multiplies it by dense
+// matrices, which rounds by norms in any arithmetic: sigma of these three matrices (40000 x 1200,
+// Gram-of-A route) are 8e-15, 9e-15 and 1.6e-14 from 64 bits, on the FP64 tiles 1.2e-14, 1.1e-14 and
+// 2.6e-14.
+//
 // Time (FP64 kernels -> this): 100000 x 2048 x 10000 57.3 -> 33.2 ms (123 TFLOP/s of FP64 work),
 // 30011 x 840 x 2503 3.39 -> 2.0 ms, 2048^2 x 100000 (symmetric) 6.7 -> 4.4 ms.
 //
@@ -300,7 +311,11 @@ __device__ __forceinline__ void mfma_i8(i32x4& acc, const u32x4& a, const u32x4&
 // stage four ahead issued between the MFMA rows of step k) on twice the k per byte.  The rows of
 // the MFMA result are output columns, so a lane holds 4 consecutive columns and stores them as
 // one word.  Grid: ((range * kMods + modulus) * tiles + tile); sym: lower-triangle tiles only.
-// Bound by the INT8 matrix cores and the L2-to-LDS path together.
+// Bound by the INT8 matrix cores and the L2-to-LDS path together: matrix pipe 60 % busy in the sketch
+// and 51 % in the Gram at 100000 x 10000, Nl = 2048 (one wave per SIMD and a barrier per 64 k leave
+// the rest), waves waiting 20 and 28 % of their cycles, 0.2 % on LDS, 39 and 18 % of the L2 requests
+// missing (3.8 TB/s).  With all operands zero the same launches take 19 % less: that much is the
+// clock under load.
 __global__ __launch_bounds__(256) void residue_gemm_kernel(
     const uint8_t* __restrict__ Ab, const uint8_t* __restrict__ Bb, int64_t tiles_m,
     int64_t tiles_n, int64_t steps, int64_t kper, bool accumulate, bool sym, int64_t ldr,
