@@ -84,6 +84,33 @@ def test_solver_holds_what_it_reports(precision, route):
     assert s.workspace_bytes() <= required + tail
 
 
+def decaying(m, n):
+    rng = np.random.default_rng(8)
+    a = (rng.standard_normal((m, 60)) * 0.95 ** np.arange(60)) @ rng.standard_normal((60, n))
+    return a + 1e-3 * rng.standard_normal((m, n))
+
+
+@pytest.mark.parametrize("m,n,k,p,N", [(6000, 9000, 20, 12, 50), (30000, 2500, 50, 10, 32)])
+def test_solve_in_a_server(m, n, k, p, N):
+    """An FP64 solve whose Gram (and sketch, in the first case) run by residues gives the same bits
+    in a server's region and in a solver's own memory, whatever workspace either has."""
+    A = mc.DeviceArray.from_numpy(decaying(m, n), order="F")
+    P = mc.Parameters().setSize(m, n).setRank(k).setOverRank(p).setNumSketch(N)
+    s = mc.Solver(P, seed=12)
+    s.solve(A)
+    assert residue.solver_paths(s)[1]
+    need = mc.required_bytes(m, n, k, p, N)
+    results = 8 * (k + m * k + n * k + m * (k + p)) + (1 << 20)
+    with mc.Server(hbm_budget=need + results, slots=1) as srv:
+        rid = srv.submit(A, m, n, k, p, N, seed=12)
+        assert srv.wait(rid, 60.0)
+        r = srv.result(rid)
+        assert r.ok, r.error
+        for x, y in ((r.S, s.vectorS()), (r.U, s.matrixU()), (r.V, s.matrixV()),
+                     (r.Qbar, s.matrixQbar())):
+            np.testing.assert_array_equal(x.numpy(), y)
+
+
 @pytest.fixture
 def untuned():
     mc.tune_clear()
@@ -91,21 +118,21 @@ def untuned():
     mc.tune_clear()
 
 
-def test_tuned_plan_keeps_the_route(untuned):
+@pytest.mark.parametrize("m,n,k,p,N,sketch", [
+    (6000, 9000, 20, 12, 50, True),    # with 576 the partials could not hold the packed Omega
+    (40000, 1000, 50, 10, 32, False),  # with 9216 the Gram takes other panels and ranges
+])
+def test_tuned_plan_keeps_the_route(untuned, m, n, k, p, N, sketch):
     """The Gram's split target changes neither the route of an FP64 sketch and its Gram nor a bit
-    of the results: with 576 its partials alone could not hold the sketch's packed Omega."""
-    m, n, k, p, N = 6000, 9000, 20, 12, 50
-    rng = np.random.default_rng(8)
-    a = (rng.standard_normal((m, 60)) * 0.95 ** np.arange(60)) @ rng.standard_normal((60, n))
-    a += 1e-3 * rng.standard_normal((m, n))
-    A = mc.DeviceArray.from_numpy(a, order="F")
+    of the results."""
+    A = mc.DeviceArray.from_numpy(decaying(m, n), order="F")
     P = mc.Parameters().setSize(m, n).setRank(k).setOverRank(p).setNumSketch(N)
     out = []
     for gram in (2304, 576, 9216):
-        mc.tune_set(P, dict(mc.tuning_default(), gram=gram))
-        s = mc.Solver(P, seed=9)
+        mc.tune_set(P, dict(mc.tuning_default(), gram=gram), route=mc.ROUTE_SKETCH)
+        s = mc.Solver(P, seed=9, route=mc.ROUTE_SKETCH)
         s.solve(A)
-        assert residue.solver_paths(s) == (True, True)
+        assert residue.solver_paths(s) == (sketch, True)
         out.append((s.vectorS(), s.matrixU(), s.matrixV(), s.matrixQbar()))
     for other in out[1:]:
         for x, y in zip(out[0], other):
