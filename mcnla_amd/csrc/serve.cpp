@@ -147,8 +147,6 @@ struct mcnla_server_s {
   int* flags = nullptr;  // per worker: 2 kMaxKnGroup ints of device memory for its KN group
   std::mutex mu;
   std::condition_variable cv_work, cv_done;
-  int ready = 0;  // workers whose streams and events exist (or could not be created)
-  std::condition_variable cv_ready;
   Arena arena{0};
   std::deque<Req*> pending;
   std::unordered_map<uint64_t, std::unique_ptr<Req>> reqs;
@@ -202,7 +200,6 @@ struct mcnla_server_s {
   void run(Req* q, hipStream_t st, SolveRes* res);
   void finish_locked(Req* q);
   void worker(int index);
-  void worker_ready();
   void worker_kn(hipStream_t st, SolveRes* res, int* flags, int cap);
 };
 
@@ -335,7 +332,6 @@ void mcnla_server_s::worker_kn(hipStream_t st, SolveRes* res, int* flags, int ca
     if (aux) (void)hipStreamDestroy(aux);
     aux = nullptr;
   }
-  worker_ready();
   KnBatch kb(flags);
   uint64_t my_chunks = 0, my_members = 0;  // flushed into the server's totals under its lock
   double my_seconds = 0.0;
@@ -523,17 +519,6 @@ void mcnla_server_s::worker_kn(hipStream_t st, SolveRes* res, int* flags, int ca
   if (chunk_done) (void)hipEventDestroy(chunk_done);
 }
 
-// The server's creation waits for every worker's streams, events and pinned flags: they take longer
-// than several small solves, and the worker that had its own first would run all requests of the
-// first milliseconds.
-void mcnla_server_s::worker_ready() {
-  {
-    std::lock_guard<std::mutex> lk(mu);
-    ++ready;
-  }
-  cv_ready.notify_one();
-}
-
 // A worker owns its stream and the HIP objects its solves record into (SolveRes) for its whole
 // life, so that admitting, running and finishing a request creates and destroys no HIP stream or
 // event.
@@ -558,7 +543,6 @@ void mcnla_server_s::worker(int index) {
   if (st && kn && cfg.batch_max > 1) {
     worker_kn(st, &res, flags + index * (kFlagBytes / sizeof(int)), cfg.batch_max);
   } else {
-    worker_ready();
     for (;;) {
       Req* q = nullptr;
       {
@@ -658,10 +642,6 @@ mcnla_status mcnla_server_create(const mcnla_server_config* cfg, mcnla_server* o
     s->flags = reinterpret_cast<int*>(s->base + foff);
     for (int i = 0; i < s->cfg.slots; ++i)
       s->workers.emplace_back([srv = s.get(), i] { srv->worker(i); });
-    {
-      std::unique_lock<std::mutex> lk(s->mu);
-      s->cv_ready.wait(lk, [&] { return s->ready == s->cfg.slots; });
-    }
     *out = s.release();
     return MCNLA_OK;
   });
