@@ -3,6 +3,12 @@ import sys
 
 import pytest
 
+# Numpy's BLAS threads spin for about 30 ms after each product before they sleep, on as many CPUs as
+# the process has: a server created meanwhile cannot get its workers scheduled, and one worker serves
+# the first ten small requests (test_gpu_serve.py asks for two at once).  2^4 cycles instead of 2^26;
+# read when numpy loads.
+os.environ.setdefault("OPENBLAS_THREAD_TIMEOUT", "4")
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 for p in (ROOT, os.path.join(ROOT, "tests")):
     if p not in sys.path:
