@@ -1004,6 +1004,8 @@ struct mcnla_solver_s {
   }
   // Creates the solver's own set if it has none, and points the timer and cores at it.
   void bind_res() {
+    // a change of plan may have found no memory, not even for the plan before it
+    MCNLA_REQUIRE(gram.partial.p != nullptr, MCNLA_ERR_STATE, "the solver has lost its workspace");
     if (!res->ready()) res->create();
     timer.borrow(res->marks, mcnla::SolveRes::kMarks);
     sketch.gemm_beg = res->sketch_beg;
@@ -1095,7 +1097,7 @@ GemmF64Args plan_omega_p(int64_t n, int64_t nl, int64_t target, int kern) {
   return g;
 }
 
-// Sets the solver's GEMM plan and sizes the split-K scratch it needs (grows only).
+// Sets the solver's GEMM plan and sizes the scratch it needs (grows only).
 void apply_tuning(mcnla_solver_s* s, const mcnla_tuning& t) {
   s->tune = t;
   s->gram.target = t.gram;
@@ -1105,27 +1107,37 @@ void apply_tuning(mcnla_solver_s* s, const mcnla_tuning& t) {
   const int64_t l = s->prm.rank + s->prm.over_rank, nl = l * s->prm.num_sketch;
   const int64_t m = s->prm.nrow, n = s->prm.ncol;
   const bool via_a = s->route == MCNLA_ROUTE_GRAM_OF_A;
-  if (via_a)
-    s->gp.ensure(std::max({gemm_f64_partial_elems(n, nl, plan_h_omega(n, nl, t.h_omega, kern_bit(t, kKernHOmega)).splits),
-                           gemm_f64_partial_elems(nl, nl, plan_omega_p(n, nl, t.omega_p, kern_bit(t, kKernOmegaP)).splits),
-                           gemm_f64_partial_elems(n, l, n_by_l_splits(n, nl, t.n_by_l)),
-                           gemm_f64_partial_elems(n, l, n_by_l_splits(n, n, t.n_by_l))}) *
-                 sizeof(double));
   const int64_t gn = via_a ? n : nl;
   size_t part = std::max(s->gram.partial_bytes(false, m, gn), GramCore::residue_limit(m, gn));
-  size_t packed = 0;
-  if (!via_a) {  // the Qbar product's split-K partials reuse the Gram's (free by then)
+  // What lies behind the Gram's partials in one buffer: on the sketch route a 16-bit sketch's packed
+  // operands, done with when the Gram starts; on the Gram-of-A route P and the later products'
+  // partials, not begun.  A Gram by residues works in all of it.
+  size_t packed = 0, gp = 0, P = 0;
+  if (via_a) {
+    gp = std::max({gemm_f64_partial_elems(n, nl, plan_h_omega(n, nl, t.h_omega, kern_bit(t, kKernHOmega)).splits),
+                   gemm_f64_partial_elems(nl, nl, plan_omega_p(n, nl, t.omega_p, kern_bit(t, kKernOmegaP)).splits),
+                   gemm_f64_partial_elems(n, l, n_by_l_splits(n, nl, t.n_by_l)),
+                   gemm_f64_partial_elems(n, l, n_by_l_splits(n, n, t.n_by_l))}) *
+         sizeof(double);
+    P = n * nl * sizeof(double);
+  } else {  // the Qbar product's split-K partials reuse the Gram's (free by then)
     part = std::max(part, gemm_f64_partial_elems(m, l, qbar_splits(m, nl, t.qbar)) *
                               sizeof(double));
     if (is_mixed(s->cfg.precision))
       packed = sketch_bf16_workspace(SketchCore::bf16_args(s->prm, s->cfg.precision));
   }
-  // A 16-bit sketch's packed operands follow the partials in one buffer: they are done with when
-  // the Gram starts, and a Gram by residues works in all of it.
-  part = align_up(part, kCarveAlign);
-  s->sketch.ws.view(nullptr, 0);  // should the buffer not be had
-  s->gram.partial.ensure(part + packed);
-  if (packed) s->sketch.ws.view(s->gram.partial.as<char>() + part, packed);
+  const std::pair<DevBuf*, size_t> behind[] = {{&s->sketch.ws, packed}, {&s->gp, gp}, {&s->P, P}};
+  size_t total = align_up(part, kCarveAlign);
+  for (const auto& b : behind) {
+    b.first->view(nullptr, 0);  // should the buffer not be had
+    total += align_up(b.second, kCarveAlign);
+  }
+  s->gram.partial.ensure(total);
+  size_t at = align_up(part, kCarveAlign);
+  for (const auto& b : behind) {
+    if (b.second) b.first->view(s->gram.partial.as<char>() + at, b.second);
+    at += align_up(b.second, kCarveAlign);
+  }
   s->form.prepare(s->prm);
 }
 
@@ -1163,7 +1175,6 @@ std::unique_ptr<mcnla_solver_s> new_solver(const mcnla_params* params,
   } else {
     s->A64.ensure(m * n * sizeof(double));
     s->H.ensure(n * n * sizeof(double));
-    s->P.ensure(n * nl * sizeof(double));
     s->X.ensure(n * l * sizeof(double));
   }
   apply_tuning(s.get(), lookup_tuning(tune_key(*params, s->route, cfg->precision), nullptr));
@@ -1362,6 +1373,7 @@ void solve_orthogonalize(mcnla_solver_s* s, hipStream_t st, SolveCtx& cx) {
 void solve_begin(mcnla_solver_s* s, const void* A, int64_t lda, int a_dtype, int a_order,
                  hipStream_t st, SolveCtx& cx, bool timed) {
   s->bind_res();
+  MCNLA_REQUIRE(s->gram.partial.p != nullptr, MCNLA_ERR_STATE, "the solver lost its workspace");
   if (timed) s->timer.start(st);
   solve_sketch(s, A, lda, a_dtype, a_order, st, cx);
   if (timed) s->timer.mark(st);
@@ -2193,7 +2205,7 @@ mcnla_status mcnla_solver_workspace_bytes(mcnla_solver s, size_t* bytes) {
   return guard([&] {
     MCNLA_REQUIRE(s && bytes, MCNLA_ERR_INVALID, "null argument");
     size_t b = 0;
-    for (const DevBuf* d : {&s->Y, &s->A64, &s->H, &s->P, &s->X, &s->gp, &s->L0, &s->T0, &s->W0,
+    for (const DevBuf* d : {&s->Y, &s->A64, &s->H, &s->X, &s->L0, &s->T0, &s->W0,
                             &s->G, &s->W, &s->w, &s->V, &s->T, &s->Bs, &s->tmp, &s->ws,
                             &s->coef, &s->M2, &s->Qbar, &s->bad, &s->sketch.omega, &s->sketch.tail,
                             &s->gram.partial, &s->form.Z, &s->form.partial, &s->form.Wg,
@@ -2466,29 +2478,35 @@ mcnla_status mcnla_solver_autotune(mcnla_solver s, const void* A, int64_t lda, i
       }
       return best;
     };
-    mcnla_tuning t = s->tune;
-    for (const Knob& k : knobs) {
-      int64_t best_v = t.*k.field;
-      double best_t = measure(k.stages);
-      for (int64_t v : k.candidates) {
-        if (v == best_v) continue;
-        mcnla_tuning c = t;
-        c.*k.field = v;
-        apply_tuning(s, c);
-        const double ct = measure(k.stages);
-        if (ct < 0.99 * best_t) {
-          best_t = ct;
-          best_v = v;
+    const mcnla_tuning before = s->tune;
+    mcnla_tuning t = before;
+    try {
+      for (const Knob& k : knobs) {
+        int64_t best_v = t.*k.field;
+        double best_t = measure(k.stages);
+        for (int64_t v : k.candidates) {
+          if (v == best_v) continue;
+          mcnla_tuning c = t;
+          c.*k.field = v;
+          apply_tuning(s, c);
+          const double ct = measure(k.stages);
+          if (ct < 0.99 * best_t) {
+            best_t = ct;
+            best_v = v;
+          }
         }
+        t.*k.field = best_v;
+        apply_tuning(s, t);
+        // then the GEMM's other kernel (tile shape) at the chosen target
+        mcnla_tuning c = t;
+        c.kernels ^= k.kernel_bit;
+        apply_tuning(s, c);
+        if (measure(k.stages) < 0.99 * best_t) t = c;
+        apply_tuning(s, t);
       }
-      t.*k.field = best_v;
-      apply_tuning(s, t);
-      // then the GEMM's other kernel (tile shape) at the chosen target
-      mcnla_tuning c = t;
-      c.kernels ^= k.kernel_bit;
-      apply_tuning(s, c);
-      if (measure(k.stages) < 0.99 * best_t) t = c;
-      apply_tuning(s, t);
+    } catch (const Error&) {  // no memory for a candidate, most likely
+      apply_tuning(s, before);
+      throw;
     }
     solve();  // leave the results of the tuned plan
     store_tuning(tune_key(s->prm, s->route, s->cfg.precision), t);

@@ -2,12 +2,14 @@
 workspaces of different sizes take other panels and other K ranges.  The operands are orthogonal to
 2^-20 of their norms, so that the sums are small beside the moduli's product: there the FP64
 arithmetic of the reconstruction would show which residues it was given."""
+import contextlib
 import ctypes
 
 import numpy as np
 import pytest
 
 import mcnla_amd as mc
+from mcnla_amd import _lib
 import residue
 
 pytestmark = pytest.mark.gpu
@@ -139,6 +141,19 @@ def test_tuned_plan_keeps_the_route(untuned, m, n, k, p, N, sketch):
             np.testing.assert_array_equal(x, y)
 
 
+@contextlib.contextmanager
+def little_memory(left):
+    """All but about `left` bytes of the device's memory taken."""
+    held = []
+    try:
+        while (free := mc.mem_info()[0]) > left + (64 << 20):
+            held.append(mc.DeviceArray((min(free - left, 16 << 30) // 8,)))
+        yield
+    finally:
+        for x in held:
+            x.free()
+
+
 def test_sketcher_with_little_memory():
     """A sketcher stage takes at most an eighth of the free memory for its residue workspace, and
     gives the same bits in a smaller one."""
@@ -156,13 +171,26 @@ def test_sketcher_with_little_memory():
     Q = P.createCollectionQ()
     y, _, taken = sketch()
     assert taken > 400 << 20
-    held, left = [], 5 << 29
-    try:
-        while (free := mc.mem_info()[0]) > left + (64 << 20):
-            held.append(mc.DeviceArray((min(free - left, 16 << 30) // 8,)))
+    with little_memory(5 << 29):
         z, before, taken = sketch()
-    finally:
-        for x in held:
-            x.free()
     assert taken <= before // 8 + (4 << 20)
     np.testing.assert_array_equal(y, z)
+
+
+def test_autotune_without_memory(untuned):
+    """Candidate plans that there is no memory for: the tuner reports it, and the solver goes on
+    with the plan it had."""
+    m, n, k, p, N = 30000, 2500, 50, 10, 32
+    A = mc.DeviceArray.from_numpy(decaying(m, n), order="F")
+    P = mc.Parameters().setSize(m, n).setRank(k).setOverRank(p).setNumSketch(N)
+    s = mc.Solver(P, seed=12)
+    s.solve(A)
+    before, plan = (s.vectorS(), s.matrixU(), s.matrixV(), s.matrixQbar()), s.tuning()
+    with little_memory(1 << 29):
+        with pytest.raises(mc.McnlaError) as e:
+            s.autotune(A, reps=1)
+        assert e.value.status == _lib.ERR_NOMEM
+        assert s.tuning() == plan
+        s.solve(A)
+        for x, y in zip(before, (s.vectorS(), s.matrixU(), s.matrixV(), s.matrixQbar())):
+            np.testing.assert_array_equal(x, y)
